@@ -216,90 +216,141 @@ __global__ __launch_bounds__(kRows) void k_dense_resid_dd(const int2 *__restrict
 // (bx, by) takes rows bx * kRows .. and columns by * cspan ..; with several
 // column ranges each writes its partial sums to part[by][r][row], which
 // k_rect_reduce adds to y in range order (deterministic).
+//
+// Bound by the FP64 (FP32) vector instructions of the profile.  A thread
+// holds one row and walks the columns, staged 128 at a time in LDS as one
+// record (coordinates, then the NR right-hand sides) that every lane reads
+// by broadcast.  The profile and the right-hand sides per pass are template
+// arguments, so the column loop has no branches and four columns' dependent
+// chains overlap: with the profile chosen inside the loop a column cost a
+// wave 1,500 cycles.  60,000 x 60,000, before and now: multiquadric with
+// eight right-hand sides 9.7 -> 4.0 ms, 1/(r + p) in FP32 5.7 -> 2.3 ms,
+// Gaussian with sixteen 15.3 -> 6.1 ms (FP64 issue bound).
 constexpr int kRectRhs = 16;
+constexpr int kRectCols = 128;  // columns staged per step
+constexpr int kRectUnroll = 4;
 
-template <int D, bool FP32>
+template <int D, bool FP32, int NR, int TYPE>
+__device__ __forceinline__ void rect_body(int64_t nrows, const double *__restrict__ rp,
+                                          int64_t ncols, const double *__restrict__ cp,
+                                          const KernelDesc &k, int nrhs,
+                                          const double *__restrict__ x, int64_t ldx,
+                                          double *__restrict__ y, int64_t ldy, int64_t cspan,
+                                          double *__restrict__ part, double *__restrict__ rec) {
+  constexpr int W = (D + NR + 1) & ~1;  // doubles per record, 16-byte aligned
+  const int64_t i = int64_t(blockIdx.x) * kRows + threadIdx.x;
+  const bool act = i < nrows;
+  double xi[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) xi[d] = act ? rp[i * D + d] : 0.0;
+  double acc[NR];
+  float a32[NR], c32[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    acc[r] = 0.0;
+    a32[r] = 0.0f;
+    c32[r] = 0.0f;
+  }
+  auto pair = [&](const double *e) {
+    if (FP32) {
+      float s = 0.0f;
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const float dx = float(e[d] - xi[d]);
+        s = s + dx * dx;
+      }
+      const float f = abh::phi32t<TYPE>(k, s);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) abh::kb_add(a32[r], c32[r], f * float(e[D + r]));
+    } else {
+      double s = 0.0;
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const double dx = e[d] - xi[d];
+        s = fma(dx, dx, s);
+      }
+      const double f = abh::phi64t<TYPE>(k, s);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) acc[r] = fma(f, e[D + r], acc[r]);
+    }
+  };
+  const int64_t cb = int64_t(blockIdx.y) * cspan;
+  const int64_t ce = cb + cspan < ncols ? cb + cspan : ncols;
+  for (int64_t c0 = cb; c0 < ce; c0 += kRectCols) {
+    const int m = int(ce - c0 < kRectCols ? ce - c0 : kRectCols);
+    __syncthreads();
+    for (int e = threadIdx.x; e < m * D; e += kRows) rec[(e / D) * W + e % D] = cp[c0 * D + e];
+    for (int e = threadIdx.x; e < kRectCols * NR; e += kRows) {
+      const int j = e % kRectCols, r = e / kRectCols;
+      if (j < m) rec[j * W + D + r] = r < nrhs ? x[int64_t(r) * ldx + c0 + j] : 0.0;
+    }
+    __syncthreads();
+    int j = 0;
+#pragma unroll 1
+    for (; j + kRectUnroll <= m; j += kRectUnroll)
+#pragma unroll
+      for (int u = 0; u < kRectUnroll; ++u) pair(rec + (j + u) * W);
+#pragma unroll 1
+    for (; j < m; ++j) pair(rec + j * W);
+  }
+  if (!act) return;
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+    if (r < nrhs) {
+      const double v = FP32 ? double(a32[r]) + double(c32[r]) : acc[r];
+      if (part) part[(int64_t(blockIdx.y) * nrhs + r) * nrows + i] = v;
+      else y[int64_t(r) * ldy + i] += v;
+    }
+}
+
+template <int D, bool FP32, int NR>
 __global__ __launch_bounds__(kRows) void k_dense_rect(int64_t nrows, const double *__restrict__ rp,
                                                       int64_t ncols, const double *__restrict__ cp,
                                                       KernelDesc k, int nrhs,
                                                       const double *__restrict__ x, int64_t ldx,
                                                       double *__restrict__ y, int64_t ldy,
                                                       int64_t cspan, double *__restrict__ part) {
-  __shared__ double sp[kRows][D];
-  __shared__ double sx[kRectRhs][kRows];
-  const int64_t i = int64_t(blockIdx.x) * kRows + threadIdx.x;
-  const bool act = i < nrows;
-  double xi[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) xi[d] = act ? rp[i * D + d] : 0.0;
-  double acc[kRectRhs];
-  float a32[kRectRhs], c32[kRectRhs];
-#pragma unroll
-  for (int r = 0; r < kRectRhs; ++r) {
-    acc[r] = 0.0;
-    a32[r] = 0.0f;
-    c32[r] = 0.0f;
+  __shared__ __align__(16) double rec[kRectCols * ((D + NR + 1) & ~1)];
+#define ABH_RECT_BODY(T)                                                                        \
+  case T:                                                                                       \
+    rect_body<D, FP32, NR, T>(nrows, rp, ncols, cp, k, nrhs, x, ldx, y, ldy, cspan, part, rec); \
+    break;
+  switch (k.type) {
+    ABH_RECT_BODY(ABH_KERNEL_CONSTANT)
+    ABH_RECT_BODY(ABH_KERNEL_GAUSSIAN)
+    ABH_RECT_BODY(ABH_KERNEL_WENDLAND_C2)
+    ABH_RECT_BODY(ABH_KERNEL_MULTIQUADRIC)
+    ABH_RECT_BODY(ABH_KERNEL_SMOOTH_INV_R)
   }
-  const int64_t cb = int64_t(blockIdx.y) * cspan;
-  const int64_t ce = cb + cspan < ncols ? cb + cspan : ncols;
-  for (int64_t c0 = cb; c0 < ce; c0 += kRows) {
-    const int m = int(ce - c0 < kRows ? ce - c0 : kRows);
-    __syncthreads();
-    if (int(threadIdx.x) < m) {
-      const int64_t j = c0 + threadIdx.x;
-#pragma unroll
-      for (int d = 0; d < D; ++d) sp[threadIdx.x][d] = cp[j * D + d];
-      for (int r = 0; r < nrhs; ++r) sx[r][threadIdx.x] = x[int64_t(r) * ldx + j];
-    }
-    __syncthreads();
-    if (!act) continue;
-    for (int j = 0; j < m; ++j) {
-      if (FP32) {
-        float s = 0.0f;
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-          const float dx = float(sp[j][d] - xi[d]);
-          s = s + dx * dx;
-        }
-        const float f = abh::phi32(k, s);
-#pragma unroll
-        for (int r = 0; r < kRectRhs; ++r)
-          if (r < nrhs) abh::kb_add(a32[r], c32[r], f * float(sx[r][j]));
-      } else {
-        double s = 0.0;
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-          const double dx = sp[j][d] - xi[d];
-          s = s + dx * dx;
-        }
-        const double f = abh::phi64(k, s);
-#pragma unroll
-        for (int r = 0; r < kRectRhs; ++r)
-          if (r < nrhs) acc[r] += f * sx[r][j];
-      }
-    }
-  }
-  if (act)
-#pragma unroll
-    for (int r = 0; r < kRectRhs; ++r)
-      if (r < nrhs) {
-        const double v = FP32 ? double(a32[r]) + double(c32[r]) : acc[r];
-        if (part) part[(int64_t(blockIdx.y) * nrhs + r) * nrows + i] = v;
-        else y[int64_t(r) * ldy + i] += v;
-      }
+#undef ABH_RECT_BODY
 }
 
-// y[r][i] += sum over the column ranges s (in order) of part[s][r][i]
+// y[r][i] += sum over the column ranges s (in order) of part[s][r][i]: the
+// ranges are cut into 8 consecutive groups summed by 8 threads of a block,
+// their sums added in group order, so that a few thousand outputs still
+// spread over the chip (32 outputs per block, 256-byte reads).
+constexpr int kRedOut = 32, kRedGroups = 8;
 __global__ __launch_bounds__(256) void k_rect_reduce(int64_t nrows, int nrhs, int ns,
                                                      const double *__restrict__ part,
                                                      double *__restrict__ y, int64_t ldy) {
-  const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (t >= nrows * nrhs) return;
-  const int r = int(t / nrows);
-  const int64_t i = t % nrows;
+  __shared__ double sum[kRedGroups][kRedOut];
+  const int o = threadIdx.x % kRedOut, g = threadIdx.x / kRedOut;
+  const int64_t t = int64_t(blockIdx.x) * kRedOut + o;
+  const int64_t total = nrows * nrhs;
+  const int per = (ns + kRedGroups - 1) / kRedGroups;
+  const int s0 = g * per, s1 = min(ns, s0 + per);
   double v = 0.0;
-  for (int s = 0; s < ns; ++s) v += part[(int64_t(s) * nrhs + r) * nrows + i];
-  y[int64_t(r) * ldy + i] += v;
+  if (t < total) {
+#pragma unroll 4
+    for (int s = s0; s < s1; ++s) v += part[int64_t(s) * total + t];
+  }
+  sum[g][o] = v;
+  __syncthreads();
+  if (g != 0 || t >= total) return;
+#pragma unroll
+  for (int q = 1; q < kRedGroups; ++q) v += sum[q][o];
+  const int r = int(t / nrows);
+  y[int64_t(r) * ldy + (t - int64_t(r) * nrows)] += v;
 }
 
 }  // namespace
@@ -426,6 +477,15 @@ struct abh_dense_batch {
 
 namespace {
 
+bool stream_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
 // y += K x for the rectangular operator.  part_ext == nullptr: the column
 // split's partial sums live in the context's grow-only buffer; otherwise in
 // part_ext (part_cap doubles), and a split that needs more is refused.
@@ -452,15 +512,33 @@ void dense_apply_impl(abh_context *ctx, int dim, int64_t nrows, const double *ro
   const bool f32 = precision == ABH_FP32_COMPENSATED;
   hipStream_t s = ctx->stream;
   const int64_t grows = abh::ceil_div(nrows, kRows);
-  // few row blocks (a tall operator has plenty): split the columns into
-  // ranges of at least 2,048 so that about 8 blocks per CU run
+  // Few row blocks (a tall operator has plenty): split the columns so that
+  // about 8 blocks (32 waves) per CU run.  The coarse split has ranges of at
+  // least 2,048 columns; its partial sums decide what the allocation-free
+  // entry point refuses.  Where they fit the static scratch, both entry
+  // points take the fine split, ranges down to 32 columns as long as their
+  // partial sums fit it too: a wave's time is its range's length, and a
+  // 5,000 x 4,001 Gaussian took 1,313 us in one range (20 blocks), 26 us in
+  // 126 ranges; 300 x 50,000 760 us in 24, 52 us in 1,563.  A captured
+  // abh_dense_apply keeps the coarse split, which needs no buffer of the
+  // context for the shapes that never needed one (the context may replace
+  // its buffer before the graph is replayed).
   int64_t ns = 1;
   const int64_t want = int64_t(ctx->n_cu) * 8;
   if (grows < want && ncols > 0)
     ns = std::max<int64_t>(1, std::min(abh::ceil_div(want, grows), ncols / 2048));
-  const int64_t cspan =
+  int64_t cspan =
       ncols > 0 ? abh::ceil_div(abh::ceil_div(ncols, ns), int64_t(kRows)) * kRows : 1;
   ns = ncols > 0 ? abh::ceil_div(ncols, cspan) : 1;
+  const int64_t fit =
+      int64_t(kNoAllocScratchDoubles) / (int64_t(std::min(nrhs, kRectRhs)) * nrows);
+  if (grows < want && ns <= fit && (part_ext || !stream_capturing(s))) {
+    const int64_t fine = std::min({abh::ceil_div(want, grows), fit, ncols / 32});
+    if (fine > ns) {
+      cspan = abh::ceil_div(abh::ceil_div(ncols, fine), int64_t(32)) * 32;
+      ns = abh::ceil_div(ncols, cspan);
+    }
+  }
   double *part = nullptr;
   if (ns > 1) {
     // part[s][r][i] for the ranges s, the right-hand sides r of one pass and
@@ -484,20 +562,26 @@ void dense_apply_impl(abh_context *ctx, int dim, int64_t nrows, const double *ro
     const int nr = std::min(kRectRhs, nrhs - r0);
     const double *xr = x + int64_t(r0) * ldx;
     double *yr = y + int64_t(r0) * ldy;
-#define ABH_RECT(DD)                                                                            \
-  if (f32)                                                                                      \
-    k_dense_rect<DD, true><<<grid, kRows, 0, s>>>(nrows, row_pos, ncols, col_pos, k, nr, xr, ldx, \
-                                                  yr, ldy, cspan, part);                        \
-  else                                                                                          \
-    k_dense_rect<DD, false><<<grid, kRows, 0, s>>>(nrows, row_pos, ncols, col_pos, k, nr, xr,   \
-                                                   ldx, yr, ldy, cspan, part);
+#define ABH_RECT2(DD, F32, NR)                                                                 \
+  k_dense_rect<DD, F32, NR><<<grid, kRows, 0, s>>>(nrows, row_pos, ncols, col_pos, k, nr, xr, ldx, \
+                                                   yr, ldy, cspan, part);
+#define ABH_RECT1(DD, F32)               \
+  if (nr == 1) { ABH_RECT2(DD, F32, 1) } \
+  else if (nr <= 4) { ABH_RECT2(DD, F32, 4) } \
+  else if (nr <= 8) { ABH_RECT2(DD, F32, 8) } \
+  else { ABH_RECT2(DD, F32, 16) }
+#define ABH_RECT(DD)                \
+  if (f32) { ABH_RECT1(DD, true) }  \
+  else { ABH_RECT1(DD, false) }
     if (dim == 1) { ABH_RECT(1) }
     else if (dim == 2) { ABH_RECT(2) }
     else { ABH_RECT(3) }
 #undef ABH_RECT
+#undef ABH_RECT1
+#undef ABH_RECT2
     abh::check_launch();
     if (part) {
-      k_rect_reduce<<<unsigned(abh::ceil_div(nrows * nr, int64_t(256))), 256, 0, s>>>(
+      k_rect_reduce<<<unsigned(abh::ceil_div(nrows * nr, int64_t(kRedOut))), 256, 0, s>>>(
           nrows, nr, int(ns), part, yr, ldy);
       abh::check_launch();
     }

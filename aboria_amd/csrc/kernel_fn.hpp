@@ -51,8 +51,12 @@ __device__ __forceinline__ double rcp_fast(double x) {
 // The radial profiles in FP64 (operators, local matrices, FMM transfer
 // operators): within a few ulp of the libm forms, which is inside every
 // tolerance they are held to (the radius tests never use them).
-__device__ __forceinline__ double phi64(const KernelDesc &k, double s) {
-  switch (k.type) {
+//
+// phi64t / phi32t take the profile as a template argument: a loop over pairs
+// that is compiled per profile has no branch in its body, so the compiler
+// overlaps several pairs' dependent chains.
+template <int TYPE> __device__ __forceinline__ double phi64t(const KernelDesc &k, double s) {
+  switch (TYPE) {
     case ABH_KERNEL_CONSTANT: return 1.0;
     case ABH_KERNEL_GAUSSIAN: return exp(-(s * k.inv2));
     case ABH_KERNEL_WENDLAND_C2: {
@@ -68,10 +72,21 @@ __device__ __forceinline__ double phi64(const KernelDesc &k, double s) {
   return 0.0;
 }
 
-// FP32 profiles with the hardware square root and reciprocal (1 ulp)
-__device__ __forceinline__ float phi32(const KernelDesc &k, float s) {
-  const float p = float(k.param);
+__device__ __forceinline__ double phi64(const KernelDesc &k, double s) {
   switch (k.type) {
+    case ABH_KERNEL_CONSTANT: return phi64t<ABH_KERNEL_CONSTANT>(k, s);
+    case ABH_KERNEL_GAUSSIAN: return phi64t<ABH_KERNEL_GAUSSIAN>(k, s);
+    case ABH_KERNEL_WENDLAND_C2: return phi64t<ABH_KERNEL_WENDLAND_C2>(k, s);
+    case ABH_KERNEL_MULTIQUADRIC: return phi64t<ABH_KERNEL_MULTIQUADRIC>(k, s);
+    case ABH_KERNEL_SMOOTH_INV_R: return phi64t<ABH_KERNEL_SMOOTH_INV_R>(k, s);
+  }
+  return 0.0;
+}
+
+// FP32 profiles with the hardware square root and reciprocal (1 ulp)
+template <int TYPE> __device__ __forceinline__ float phi32t(const KernelDesc &k, float s) {
+  const float p = float(k.param);
+  switch (TYPE) {
     case ABH_KERNEL_CONSTANT: return 1.0f;
     case ABH_KERNEL_GAUSSIAN: return expf(-(s * float(k.inv2)));
     case ABH_KERNEL_WENDLAND_C2: {
@@ -83,6 +98,17 @@ __device__ __forceinline__ float phi32(const KernelDesc &k, float s) {
     }
     case ABH_KERNEL_MULTIQUADRIC: return __builtin_amdgcn_sqrtf(s + float(k.param2));
     case ABH_KERNEL_SMOOTH_INV_R: return __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(s) + p);
+  }
+  return 0.0f;
+}
+
+__device__ __forceinline__ float phi32(const KernelDesc &k, float s) {
+  switch (k.type) {
+    case ABH_KERNEL_CONSTANT: return phi32t<ABH_KERNEL_CONSTANT>(k, s);
+    case ABH_KERNEL_GAUSSIAN: return phi32t<ABH_KERNEL_GAUSSIAN>(k, s);
+    case ABH_KERNEL_WENDLAND_C2: return phi32t<ABH_KERNEL_WENDLAND_C2>(k, s);
+    case ABH_KERNEL_MULTIQUADRIC: return phi32t<ABH_KERNEL_MULTIQUADRIC>(k, s);
+    case ABH_KERNEL_SMOOTH_INV_R: return phi32t<ABH_KERNEL_SMOOTH_INV_R>(k, s);
   }
   return 0.0f;
 }
