@@ -13,6 +13,7 @@
 //   7. gather of the positions into sorted order (Particles::reorder)
 // All FP64 arithmetic is compiled without contraction so bucket indices are
 // the reference's bit for bit.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -140,11 +141,28 @@ __global__ __launch_bounds__(kThreads) void k_bucket_counts(const uint32_t *__re
   }
 }
 
-// end[b] = begin[b] + count[b], the counts held in end
+// end[b] = begin[b] + count[b], the counts held in end; and the sum of the
+// squared counts, one atomic per block (at most kEndBlocks of them: one
+// address takes about 85 million atomics per second)
+constexpr int kEndBlocks = 256;
 __global__ __launch_bounds__(kThreads) void k_bucket_ends(const uint32_t *__restrict__ begin,
-                                                          int64_t nb, uint32_t *__restrict__ end) {
-  const int64_t t = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (t < nb) end[t] = begin[t] + end[t];
+                                                          int64_t nb, uint32_t *__restrict__ end,
+                                                          BuildCounters *__restrict__ ctr) {
+  __shared__ unsigned long long ws[kThreads / 64];
+  unsigned long long sq = 0;
+  for (int64_t t = int64_t(blockIdx.x) * kThreads + threadIdx.x; t < nb;
+       t += int64_t(gridDim.x) * kThreads) {
+    const uint32_t c = end[t];
+    end[t] = begin[t] + c;
+    sq += (unsigned long long)c * c;
+  }
+  sq = abh::wave_sum(sq);
+  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = sq;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kThreads / 64; ++w) sq += ws[w];
+    if (sq) atomicAdd(&ctr->sq_sum, sq);
+  }
 }
 
 template <int D> void launch_enforce(abh_context *ctx, const GridParams &g, int64_t n,
@@ -365,6 +383,7 @@ abh_status abh_cells_update(abh_cells *c, int64_t n, double *pos, uint8_t *alive
     ABH_HIP(hipStreamSynchronize(s));
     const int64_t na = int64_t(h.n_alive);
     c->n_alive = na;
+    c->sq_known = false;
     size_grid(c, size_t(na));
     const int64_t nb = c->nb;
     c->order.ensure(size_t(na + 1) * 4);
@@ -392,8 +411,8 @@ abh_status abh_cells_update(abh_cells *c, int64_t n, double *pos, uint8_t *alive
         abh::check_launch();
       }
       abh::scan_exclusive(ctx, cnt, c->begin.as<uint32_t>(), nb, nullptr);
-      k_bucket_ends<<<unsigned(abh::ceil_div(nb, kThreads)), kThreads, 0, s>>>(
-          c->begin.as<uint32_t>(), nb, cnt);
+      k_bucket_ends<<<unsigned(std::min<int64_t>(kEndBlocks, abh::ceil_div(nb, kThreads))),
+                      kThreads, 0, s>>>(c->begin.as<uint32_t>(), nb, cnt, ctr);
       abh::check_launch();
     }
     if (na > 0)

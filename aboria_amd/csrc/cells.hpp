@@ -20,6 +20,7 @@ struct GridParams {
 struct BuildCounters {
   uint32_t n_alive;
   uint32_t n_wrap_fail;
+  unsigned long long sq_sum;  // squared particle counts summed over the buckets
 };
 
 // enforce_domain_lambda (src/NeighbourSearchBase.h:185-238) over n
@@ -45,6 +46,9 @@ struct abh_cells {
   int64_t nb = 1;
   abh::DevBuf order, keys, begin, end, pos;
   abh::DevBuf flags, offs, counters;  // build temporaries
+  // BuildCounters' sq_sum of the last build, read back when first asked for
+  mutable bool sq_known = false;
+  mutable unsigned long long sq_sum = 0;
   // bucket-pair sequence (pairs.hip): per-source run lengths, total, pairs
   abh::DevBuf pair_src, pair_total, pair_i, pair_j, pair_img;
   int64_t npairs = 0;

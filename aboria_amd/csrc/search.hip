@@ -19,6 +19,7 @@
 // the host widens the stencil and repeats.  The neighbour multiset of every
 // query therefore equals the reference's.
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "cells.hpp"
@@ -26,6 +27,7 @@
 #include "solvers.hpp"
 
 using abh::DevBuf;
+using abh::BuildCounters;
 using abh::GridParams;
 using abh::KernelDesc;
 using abh::kb_add;
@@ -37,6 +39,21 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kMaxSlots = 343;
 constexpr int kGroup = 64;  // queries per work item = lanes per wave
+// Which queries get a wavefront per home cell (k_search, k_matvec) and which
+// eight lanes each (k_search_group).  Measured with a radius of 0.95 cells,
+// search (build, count and fill) and one application of the operator:
+//  - where all cells hold few particles every query is served by
+//    k_search_group, without sorting: at 32 a cell 1,000,000 points in 3D take
+//    2.50 ms (2.52 with work items), at 64 4.04 (2.77); 100,000 0.51 (0.65)
+//    and 0.67 (0.91).  A wave per cell applies the operator faster from about
+//    12 on: at 8 a cell 1.23 ms (1.32), at 16 2.12 (1.70).
+//  - otherwise the cells with kHeavyMin queries and more have work items: the
+//    4M-particle mixture takes 16.6 ms (search) and 24.6 (operator, eight
+//    right-hand sides) with 8, 16.4 and 25.1 with 12, 16.6 and 25.7 with 16.
+constexpr int kHeavyMin = 12;
+constexpr double kLightSearch = 40.0;  // mean occupancy a particle sees, list passes
+constexpr double kLightOp = 13.0;      // the same for an operator's plan
+constexpr int64_t kSmall = 16384;      // particle sets that k_search_group always serves
 
 struct WorkItem {
   int32_t home[3];
@@ -110,62 +127,67 @@ __global__ __launch_bounds__(kThreads) void k_home_keys(const double *__restrict
   if (vals) vals[i] = int32_t(i);
 }
 
-// runs of equal home cell (the key without its sub-cell bits)
-__global__ __launch_bounds__(kThreads) void k_run_flags(const uint32_t *__restrict__ keys,
-                                                        int64_t n, int shift,
-                                                        uint32_t *__restrict__ flags) {
-  const int64_t k = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (k >= n) return;
-  flags[k] = (k == 0 || (keys[k] >> shift) != (keys[k - 1] >> shift)) ? 1u : 0u;
-}
-
-__global__ __launch_bounds__(kThreads) void k_run_starts(const uint32_t *__restrict__ flags,
-                                                         const uint32_t *__restrict__ ridx,
-                                                         int64_t n,
-                                                         uint32_t *__restrict__ run_start) {
-  const int64_t k = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (k >= n || !flags[k]) return;
-  run_start[ridx[k]] = uint32_t(k);
-}
-
-__global__ __launch_bounds__(kThreads) void k_run_chunks(const uint32_t *__restrict__ run_start,
-                                                         const uint32_t *__restrict__ nruns_dev,
-                                                         int64_t n, uint32_t *__restrict__ chunks) {
-  const int64_t r = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (r >= n) return;
-  const int64_t nruns = int64_t(*nruns_dev);
-  if (r >= nruns) {
-    chunks[r] = 0;
-    return;
-  }
-  const int64_t s = run_start[r];
-  const int64_t e = (r + 1 < nruns) ? int64_t(run_start[r + 1]) : n;
-  chunks[r] = uint32_t((e - s + kGroup - 1) / kGroup);
-}
-
+// Runs of equal home cell (the key without its sub-cell bits) cut into work.
+// A run's whole groups of 64, and a remainder of at least heavy_min queries,
+// become work items of k_search; the queries of a smaller remainder go to the
+// list that k_search_group serves.  One thread per run (its first query),
+// which finds the run's end by doubling steps and a binary search; a
+// wavefront takes its places in both lists with one atomic each, so the
+// lists stay close to the sorted order.  ctr[0] = listed queries, ctr[1] =
+// work items, zero at launch.  A row's result does not depend on where its
+// query stands in the lists.
 template <int D>
-__global__ __launch_bounds__(kThreads) void k_fill_work(
-    const uint32_t *__restrict__ run_start, const uint32_t *__restrict__ nruns_dev, int64_t n,
-    const uint32_t *__restrict__ choff, const uint32_t *__restrict__ chunks,
-    const double *__restrict__ q_sorted, GridParams g, WorkItem *__restrict__ work) {
-  const int64_t r = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  const int64_t nruns = int64_t(*nruns_dev);
-  if (r >= nruns) return;
-  const int64_t s = run_start[r];
-  const int64_t e = (r + 1 < nruns) ? int64_t(run_start[r + 1]) : n;
-  double p[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) p[d] = q_sorted[s * D + d];
-  WorkItem w{};
-#pragma unroll
-  for (int d = 0; d < 3; ++d) w.home[d] = d < D ? home_of<D>(g, p, d) : 0;
-  const uint32_t nc = chunks[r];
-  for (uint32_t c = 0; c < nc; ++c) {
-    w.start = int32_t(s + int64_t(c) * kGroup);
-    const int64_t left = e - int64_t(w.start);
-    w.count = int32_t(left < kGroup ? left : kGroup);
-    work[choff[r] + c] = w;
+__global__ __launch_bounds__(kThreads) void k_plan_items(const uint32_t *__restrict__ keys,
+                                                         int64_t n, int shift, int heavy_min,
+                                                         const double *__restrict__ q_sorted,
+                                                         GridParams g, WorkItem *__restrict__ work,
+                                                         int32_t *__restrict__ light,
+                                                         uint32_t *__restrict__ ctr) {
+  const int64_t k = int64_t(blockIdx.x) * kThreads + threadIdx.x;
+  const uint32_t key = k < n ? keys[k] >> shift : 0u;
+  const bool head = k < n && (k == 0 || (keys[k - 1] >> shift) != key);
+  uint32_t nw = 0, nl = 0;
+  int64_t e = k;
+  if (head) {
+    int64_t step = 1;
+    while (e + step < n && (keys[e + step] >> shift) == key) {
+      e += step;
+      step <<= 1;
+    }
+    // keys[e] is in the run, e + step is not (or lies past the end)
+    for (; step > 0; step >>= 1)
+      if (e + step < n && (keys[e + step] >> shift) == key) e += step;
+    ++e;
+    const int64_t c = e - k;
+    const int rem = int(c % kGroup);
+    nw = uint32_t(c / kGroup) + (rem >= heavy_min ? 1u : 0u);
+    nl = rem < heavy_min ? uint32_t(rem) : 0u;
   }
+  const uint32_t iw = abh::wave_incl_scan(nw), il = abh::wave_incl_scan(nl);
+  uint32_t bw = 0, bl = 0;
+  if (abh::lane_id() == 63) {
+    if (il) bl = atomicAdd(&ctr[0], il);
+    if (iw) bw = atomicAdd(&ctr[1], iw);
+  }
+  bw = __shfl(bw, 63, 64) + iw - nw;
+  bl = __shfl(bl, 63, 64) + il - nl;
+  if (!head) return;
+  int64_t at = k;
+  if (nw) {
+    double p[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) p[d] = q_sorted[k * D + d];
+    WorkItem w{};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) w.home[d] = d < D ? home_of<D>(g, p, d) : 0;
+    for (uint32_t c = 0; c < nw; ++c) {
+      w.start = int32_t(at);
+      w.count = int32_t(e - at < kGroup ? e - at : kGroup);
+      work[bw + c] = w;
+      at += w.count;
+    }
+  }
+  for (uint32_t c = 0; c < nl; ++c) light[bl + c] = int32_t(at + c);
 }
 
 // ---------------------------------------------------------------------------
@@ -333,7 +355,6 @@ struct SearchArgs {
   double *val;   // assemble: kernel value of every stored pair
   float *val32;  // assemble (optional): the same value as the FP32 matvec forms it
   uint32_t *escape_flag;
-  uint32_t *next;  // dynamic work counter, zero at launch
   int ring;        // fill: stage each row's entries in LDS and store whole
                    // 64-byte segments (col is 64-byte aligned)
   // matvec
@@ -446,10 +467,131 @@ __device__ __forceinline__ void staged_hit(const SearchArgs &a, bool single, boo
   }
 }
 
+// The stencil of a work item: its buckets (slots), their ascending order
+// (sorder) and every lane's visit multiplicities (mult), all in LDS.  Returns
+// whether this lane's visited buckets leave the stencil (CHECK).
+template <int D, bool CHECK>
+__device__ __forceinline__ bool stencil_setup(const SearchArgs &a, const GridParams &g,
+                                              const WorkItem &it, const double *q, bool active,
+                                              Slot *slots, int32_t *sorder, uint8_t *mult) {
+  const int S = a.nslots, lane = threadIdx.x;
+  int wd[3] = {a.w[0], a.w[1], a.w[2]};
+  int span[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) span[d] = 2 * wd[d] + 1;
+  // image points q + I*L for I = -1, 0, +1 (search_iterator,
+  // src/Search.h:188-190), formed where needed by image_of
+
+  // stencil slots: virtual cell v = home + o -> bucket b under image I
+  for (int s = lane; s < S; s += kGroup) {
+    int o[3] = {0, 0, 0};
+    int rem = s;
+#pragma unroll
+    for (int d = D - 1; d >= 0; --d) {
+      o[d] = rem % span[d] - wd[d];
+      rem /= span[d];
+    }
+    bool ok = true;
+    int bv[3] = {0, 0, 0};
+    int imgc = 0;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int v = it.home[d] + o[d];
+      const int n = g.size[d];
+      int I = 0, b = v;
+      if (v < 0) { b = v + n; I = 1; }
+      else if (v >= n) { b = v - n; I = -1; }
+      if (I != 0 && !g.periodic[d]) ok = false;
+      if (b < 0 || b >= n) ok = false;  // would need an image beyond +-1
+      bv[d] = b;
+      imgc |= (I + 1) << (2 * d);
+          }
+    if (ok) {
+      uint32_t index = 0, m = 1;
+#pragma unroll
+      for (int i = D - 1; i >= 0; --i) {
+        if (i != D - 1) m *= uint32_t(g.size[i + 1]);
+        index += m * uint32_t(bv[i]);
+      }
+      const int bidx = int(index);
+      const int beg = int(a.bbeg[bidx]);
+      const int end = int(a.bend[bidx]);
+      slots[s] = Slot{bidx, beg, end - beg, imgc};
+    } else {
+      slots[s] = Slot{-1, 0, 0, imgc};
+    }
+  }
+  __syncthreads();
+  // ascending bucket order (ties by slot index)
+  for (int s = lane; s < S; s += kGroup) {
+    const int bs = slots[s].b;
+    int rank = 0;
+    for (int t = 0; t < S; ++t) {
+      const int bt = slots[t].b;
+      rank += (bt < bs || (bt == bs && t < s)) ? 1 : 0;
+    }
+    sorder[rank] = s;
+  }
+  // per-lane visit multiplicities, one image at a time
+  bool escape = false;
+  for (int s = 0; s < S; ++s) mult[s * kGroup + lane] = 0;
+  {
+    int nimg = 1;
+#pragma unroll
+    for (int d = 0; d < D; ++d) nimg *= 3;
+    for (int ii = 0; ii < nimg; ++ii) {
+      int I[D];
+      bool img_ok = true;
+      int t = ii;
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        I[d] = t % 3 - 1;
+        t /= 3;
+        if (I[d] != 0 && !g.periodic[d]) img_ok = false;
+      }
+      if (!img_ok) continue;  // uniform
+      int pk = 0;
+#pragma unroll
+      for (int d = 0; d < D; ++d) pk |= (I[d] + 1) << (2 * d);
+      double qi[D];
+#pragma unroll
+      for (int d = 0; d < D; ++d) qi[d] = image_of(I[d] + 1, q[d], g.L[d]);
+      const bool in_range = active && !outside_domain<D>(g, qi, a.r2);
+      if (__ballot(in_range) == 0) continue;
+      QuadState<D> qs;
+      if (in_range) {
+        quad_state<D>(g, qi, a.r2, qs);
+      } else {
+        qs.valid = 0;
+      }
+      if (CHECK && in_range) {
+        int c[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) c[d] = it.home[d] + I[d] * g.size[d];
+        if (escapes_stencil<D>(g, qi, a.r2, qs, c, wd)) escape = true;
+      }
+      for (int s = 0; s < S; ++s) {
+        const Slot sl = slots[s];
+        if (sl.img != pk || sl.b < 0) continue;
+        int b[D];
+        int rem = sl.b;
+#pragma unroll
+        for (int d = D - 1; d >= 0; --d) {
+          b[d] = rem % g.size[d];
+          rem /= g.size[d];
+        }
+        const int m = in_range ? visit_count<D>(g, qi, a.r2, qs, b) : 0;
+        mult[s * kGroup + lane] = uint8_t(m);
+      }
+    }
+  }
+  __syncthreads();
+  return escape;
+}
+
 template <int D, int MODE>
-__global__ __launch_bounds__(kGroup) void k_search(SearchArgs a, GridParams g) {
+__global__ __launch_bounds__(kGroup) __attribute__((amdgpu_waves_per_eu(4))) void k_search(SearchArgs a, GridParams g) {
   extern __shared__ __align__(16) unsigned char lds[];
-  constexpr bool kMV = (MODE == kMatvec64 || MODE == kMatvec32);
   const int S = a.nslots;
   // fill passes: the output ring, [32][64] words in static LDS (a lane's
   // ring address is a constant plus (slot << 8) | (lane << 2))
@@ -465,335 +607,162 @@ __global__ __launch_bounds__(kGroup) void k_search(SearchArgs a, GridParams g) {
   uint8_t *mult = reinterpret_cast<uint8_t *>(sorder + S);  // [S][64]
   // count / list passes: staged candidates (coordinates [D][64], index [64])
   StageRec *st = reinterpret_cast<StageRec *>(
-      lds + ((size_t(S) * (sizeof(Slot) + 4 + kGroup) + 4 * size_t(S + 1) + 15) & ~size_t(15)));
-  double *xs = reinterpret_cast<double *>(st + kGroup);  // [64][kMaxRhs], matvec only
+      lds + ((size_t(S) * (sizeof(Slot) + 4 + kGroup) + 15) & ~size_t(15)));
   const int lane = threadIdx.x;
-  const int nwork = int(*a.nwork);
-  int wd[3] = {a.w[0], a.w[1], a.w[2]};
-  int span[3];
+  if (blockIdx.x >= *a.nwork) return;  // (the grid is an upper bound)
+  const WorkItem it = a.work[blockIdx.x];
+  const int qk = it.start + (lane < it.count ? lane : 0);
+  double q[D];
+  bool finite = true;
 #pragma unroll
-  for (int d = 0; d < 3; ++d) span[d] = 2 * wd[d] + 1;
-
-  // work items are taken dynamically: their cost varies by orders of
-  // magnitude between sparse and dense cells
-  for (;;) {
-    int wi = 0;
-    if (lane == 0) wi = int(atomicAdd(a.next, 1u));
-    wi = __shfl(wi, 0, 64);
-    if (wi >= nwork) break;
-    const WorkItem it = a.work[wi];
-    const int qk = it.start + (lane < it.count ? lane : 0);
-    double q[D];
-    bool finite = true;
+  for (int d = 0; d < D; ++d) {
+    q[d] = a.qpos[int64_t(qk) * D + d];
+    finite = finite && isfinite(q[d]);
+  }
+  // a centre with a non-finite coordinate has no neighbours
+  const bool active = lane < it.count && finite;
+  const bool has_row = lane < it.count;
+  // box of the work item's active centres (empty when none is active)
+  double qlo[3] = {0.0, 0.0, 0.0}, qhi[3] = {0.0, 0.0, 0.0};
+  if (MODE != kCapacity) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      q[d] = a.qpos[int64_t(qk) * D + d];
-      finite = finite && isfinite(q[d]);
+      qlo[d] = uniform_f64(wave_min_f64(active ? q[d] : INFINITY));
+      qhi[d] = uniform_f64(wave_max_f64(active ? q[d] : -INFINITY));
     }
-    // a centre with a non-finite coordinate has no neighbours
-    const bool active = lane < it.count && finite;
-    const bool has_row = lane < it.count;
-    // box of the work item's active centres (empty when none is active)
-    double qlo[3] = {0.0, 0.0, 0.0}, qhi[3] = {0.0, 0.0, 0.0};
-    if (MODE != kCapacity) {
+  }
+  const int64_t row = a.qperm ? int64_t(a.qperm[qk]) : int64_t(qk);
+  constexpr bool kCheck = MODE == kCount || MODE == kCapacity;
+  const bool escape = stencil_setup<D, kCheck>(a, g, it, q, active, slots, sorder, mult);
+  if (kCheck && escape) atomicOr(a.escape_flag, 1u);
+  if (MODE == kCapacity) {
+    // candidates of every visited bucket, with multiplicity: no distance
+    // test can accept more
+    int64_t cap = 0;
+    for (int s = 0; s < S; ++s) cap += int64_t(mult[s * kGroup + lane]) * slots[s].len;
+    // rounded up to 16 entries: every padded row then starts on a 64-byte
+    // boundary, where the fill's ring stores whole segments from the first
+    if (has_row) a.counts[row] = active ? ((cap + 15) & ~int64_t(15)) : 0;
+    return;
+  }
+  int cnt = 0;
+  int64_t out = 0;
+  constexpr bool kList = (MODE == kFill || MODE == kAssemble || MODE == kFillPadded);
+  if (kList && active) out = a.row_ptr[row];
+  // ring state: entries [fpos, out + cnt) of this lane's row are staged
+  int64_t fpos = out;
+  uint32_t *rl = ring + lane;  // slot k of this lane: rl[k * kGroup]
+  // store the segment holding fpos once it is complete (64-byte vector
+  // stores when it starts at its segment boundary, the row's first,
+  // partial segment entry by entry)
+  auto ring_segment = [&]() {
+    const int64_t pos = out + cnt;
+    const int64_t seg = fpos & ~int64_t(kSeg - 1);
+    if (pos >= seg + kSeg) {
+      if (fpos == seg) {
+        const uint32_t *src = rl + int(seg & (kRing - 1)) * kGroup;
+        uint32_t v[kSeg];
 #pragma unroll
-      for (int d = 0; d < D; ++d) {
-        qlo[d] = uniform_f64(wave_min_f64(active ? q[d] : INFINITY));
-        qhi[d] = uniform_f64(wave_max_f64(active ? q[d] : -INFINITY));
-      }
-    }
-    const int64_t row = a.qperm ? int64_t(a.qperm[qk]) : int64_t(qk);
-    // image points q + I*L for I = -1, 0, +1 (search_iterator,
-    // src/Search.h:188-190), formed where needed by image_of
-
-    // stencil slots: virtual cell v = home + o -> bucket b under image I
-    for (int s = lane; s < S; s += kGroup) {
-      int o[3] = {0, 0, 0};
-      int rem = s;
+        for (int k = 0; k < kSeg; ++k) v[k] = src[k * kGroup];
+        uint4 *dst = reinterpret_cast<uint4 *>(a.col + seg);
 #pragma unroll
-      for (int d = D - 1; d >= 0; --d) {
-        o[d] = rem % span[d] - wd[d];
-        rem /= span[d];
-      }
-      bool ok = true;
-      int bv[3] = {0, 0, 0};
-      int imgc = 0, p3 = 1;
-#pragma unroll
-      for (int d = 0; d < D; ++d) {
-        const int v = it.home[d] + o[d];
-        const int n = g.size[d];
-        int I = 0, b = v;
-        if (v < 0) { b = v + n; I = 1; }
-        else if (v >= n) { b = v - n; I = -1; }
-        if (I != 0 && !g.periodic[d]) ok = false;
-        if (b < 0 || b >= n) ok = false;  // would need an image beyond +-1
-        bv[d] = b;
-        imgc |= (I + 1) << (2 * d);
-        (void)p3;
-      }
-      if (ok) {
-        uint32_t index = 0, m = 1;
-#pragma unroll
-        for (int i = D - 1; i >= 0; --i) {
-          if (i != D - 1) m *= uint32_t(g.size[i + 1]);
-          index += m * uint32_t(bv[i]);
-        }
-        const int bidx = int(index);
-        const int beg = int(a.bbeg[bidx]);
-        const int end = int(a.bend[bidx]);
-        slots[s] = Slot{bidx, beg, end - beg, imgc};
+        for (int k = 0; k < kSeg / 4; ++k)
+          dst[k] = make_uint4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
       } else {
-        slots[s] = Slot{-1, 0, 0, imgc};
+        for (int64_t e = fpos; e < seg + kSeg; ++e)
+          a.col[e] = int32_t(rl[int(e & (kRing - 1)) * kGroup]);
       }
+      fpos = seg + kSeg;
     }
-    __syncthreads();
-    // ascending bucket order (ties by slot index)
-    for (int s = lane; s < S; s += kGroup) {
-      const int bs = slots[s].b;
-      int rank = 0;
-      for (int t = 0; t < S; ++t) {
-        const int bt = slots[t].b;
-        rank += (bt < bs || (bt == bs && t < s)) ? 1 : 0;
-      }
-      sorder[rank] = s;
-    }
-    // per-lane visit multiplicities, one image at a time
-    bool escape = false;
-    for (int s = 0; s < S; ++s) mult[s * kGroup + lane] = 0;
-    {
-      int nimg = 1;
+  };
+  // store everything staged (row end, or before a bucket written directly)
+  auto ring_drain = [&]() {
+    const int64_t pos = out + cnt;
+    for (int64_t e = fpos; e < pos; ++e) a.col[e] = int32_t(rl[int(e & (kRing - 1)) * kGroup]);
+    fpos = pos;
+  };
+  double wrow = 1.0;
+  if (MODE == kAssemble && (a.k.row_s || a.k.col_s)) {
+    wrow = a.k.w0;
+    if (a.k.row_s && active) wrow = wrow + a.k.wr * a.k.row_s[row];
+  }
+
+  for (int k = 0; k < S; ++k) {
+    const int s = abh::uniform_i32(sorder[k]);
+    const int len = abh::uniform_i32(slots[s].len);
+    if (len <= 0) continue;
+    const int m = active ? int(mult[s * kGroup + lane]) : 0;
+    if (__ballot(m != 0) == 0) continue;  // no lane visits this bucket
+    const int beg = abh::uniform_i32(slots[s].beg);
+    const int img = abh::uniform_i32(slots[s].img);
+    double qi[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-      for (int d = 0; d < D; ++d) nimg *= 3;
-      for (int ii = 0; ii < nimg; ++ii) {
-        int I[D];
-        bool img_ok = true;
-        int t = ii;
+    for (int d = 0; d < D; ++d) qi[d] = image_of((img >> (2 * d)) & 3, q[d], g.L[d]);
+    const int end = beg + len;
+
+    if (MODE == kCount || kList) {
+      // Candidates of this bucket in blocks of 64: each lane loads one and
+      // keeps it if it lies within r of the work item's query box (the
+      // same FP64 operations as the radius test, monotone in the query, so
+      // no accepted pair is dropped); the kept ones are compacted into LDS
+      // in index order and tested against every lane's centre.  acc <= r2
+      // equals the reference's !(acc > r2) for every finite centre (acc is
+      // never NaN there); lanes with m == 0 compare against -1.
+      double blo[3] = {0.0, 0.0, 0.0}, bhi[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const int dg = (img >> (2 * d)) & 3;
+        blo[d] = uniform_f64(
+            pick3(dg, qlo[d] + double(-1) * g.L[d], qlo[d], qlo[d] + double(1) * g.L[d]));
+        bhi[d] = uniform_f64(
+            pick3(dg, qhi[d] + double(-1) * g.L[d], qhi[d], qhi[d] + double(1) * g.L[d]));
+      }
+      const double r2m = m != 0 ? a.r2 : -1.0;
+      const bool single = __ballot(m > 1) == 0;
+      for (int c0 = beg; c0 < end; c0 += kGroup) {
+        const int jc = c0 + lane;
+        bool keep = jc < end;
+        double x[3] = {0.0, 0.0, 0.0};
+        if (keep) {
+#pragma unroll
+          for (int d = 0; d < D; ++d) x[d] = a.pos[int64_t(jc) * D + d];
+        }
+        double dd = 0.0;
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-          I[d] = t % 3 - 1;
-          t /= 3;
-          if (I[d] != 0 && !g.periodic[d]) img_ok = false;
+          double e = 0.0;
+          if (x[d] < blo[d]) e = blo[d] - x[d];
+          else if (x[d] > bhi[d]) e = x[d] - bhi[d];
+          dd = dd + e * e;
         }
-        if (!img_ok) continue;  // uniform
-        int pk = 0;
-#pragma unroll
-        for (int d = 0; d < D; ++d) pk |= (I[d] + 1) << (2 * d);
-        double qi[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d) qi[d] = image_of(I[d] + 1, q[d], g.L[d]);
-        const bool in_range = active && !outside_domain<D>(g, qi, a.r2);
-        if (__ballot(in_range) == 0) continue;
-        QuadState<D> qs;
-        if (in_range) {
-          quad_state<D>(g, qi, a.r2, qs);
-        } else {
-          qs.valid = 0;
+        keep = keep && dd <= a.r2;
+        const uint64_t km = __ballot(keep);
+        if (km == 0) continue;
+        const int nk = __popcll(km);
+        if (keep) {
+          const int sl = int(__builtin_amdgcn_mbcnt_hi(uint32_t(km >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo(uint32_t(km), 0u)));
+          st[sl] = StageRec{x[0], x[1], x[2], jc, 0};
         }
-        if ((MODE == kCount || MODE == kCapacity) && in_range) {
-          int c[D];
-#pragma unroll
-          for (int d = 0; d < D; ++d) c[d] = it.home[d] + I[d] * g.size[d];
-          if (escapes_stencil<D>(g, qi, a.r2, qs, c, wd)) escape = true;
-        }
-        for (int s = 0; s < S; ++s) {
-          const Slot sl = slots[s];
-          if (sl.img != pk || sl.b < 0) continue;
-          int b[D];
-          int rem = sl.b;
-#pragma unroll
-          for (int d = D - 1; d >= 0; --d) {
-            b[d] = rem % g.size[d];
-            rem /= g.size[d];
-          }
-          const int m = in_range ? visit_count<D>(g, qi, a.r2, qs, b) : 0;
-          mult[s * kGroup + lane] = uint8_t(m);
-        }
-      }
-    }
-    if ((MODE == kCount || MODE == kCapacity) && escape) atomicOr(a.escape_flag, 1u);
-    __syncthreads();
-    if (MODE == kCapacity) {
-      // candidates of every visited bucket, with multiplicity: no distance
-      // test can accept more
-      int64_t cap = 0;
-      for (int s = 0; s < S; ++s) cap += int64_t(mult[s * kGroup + lane]) * slots[s].len;
-      // rounded up to 16 entries: every padded row then starts on a 64-byte
-      // boundary, where the fill's ring stores whole segments from the first
-      if (has_row) a.counts[row] = active ? ((cap + 15) & ~int64_t(15)) : 0;
-      __syncthreads();
-      continue;
-    }
-    int cnt = 0;
-    int64_t out = 0;
-    constexpr bool kList = (MODE == kFill || MODE == kAssemble || MODE == kFillPadded);
-    if (kList && active) out = a.row_ptr[row];
-    // ring state: entries [fpos, out + cnt) of this lane's row are staged
-    int64_t fpos = out;
-    uint32_t *rl = ring + lane;  // slot k of this lane: rl[k * kGroup]
-    // store the segment holding fpos once it is complete (64-byte vector
-    // stores when it starts at its segment boundary, the row's first,
-    // partial segment entry by entry)
-    auto ring_segment = [&]() {
-      const int64_t pos = out + cnt;
-      const int64_t seg = fpos & ~int64_t(kSeg - 1);
-      if (pos >= seg + kSeg) {
-        if (fpos == seg) {
-          const uint32_t *src = rl + int(seg & (kRing - 1)) * kGroup;
-          uint32_t v[kSeg];
-#pragma unroll
-          for (int k = 0; k < kSeg; ++k) v[k] = src[k * kGroup];
-          uint4 *dst = reinterpret_cast<uint4 *>(a.col + seg);
-#pragma unroll
-          for (int k = 0; k < kSeg / 4; ++k)
-            dst[k] = make_uint4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
-        } else {
-          for (int64_t e = fpos; e < seg + kSeg; ++e)
-            a.col[e] = int32_t(rl[int(e & (kRing - 1)) * kGroup]);
-        }
-        fpos = seg + kSeg;
-      }
-    };
-    // store everything staged (row end, or before a bucket written directly)
-    auto ring_drain = [&]() {
-      const int64_t pos = out + cnt;
-      for (int64_t e = fpos; e < pos; ++e) a.col[e] = int32_t(rl[int(e & (kRing - 1)) * kGroup]);
-      fpos = pos;
-    };
-    double acc64[kMaxRhs];
-    float acc32[kMaxRhs], cmp32[kMaxRhs];
-    if (kMV) {
-#pragma unroll
-      for (int r = 0; r < kMaxRhs; ++r) {
-        acc64[r] = (has_row && r < a.nrhs) ? a.y[int64_t(r) * a.ldy + row] : 0.0;
-        acc32[r] = 0.0f;
-        cmp32[r] = 0.0f;
-      }
-    }
-    double wrow = 1.0;
-    if ((kMV || MODE == kAssemble) && (a.k.row_s || a.k.col_s)) {
-      wrow = a.k.w0;
-      if (a.k.row_s && active) wrow = wrow + a.k.wr * a.k.row_s[row];
-    }
-
-    for (int k = 0; k < S; ++k) {
-      const int s = abh::uniform_i32(sorder[k]);
-      const int len = abh::uniform_i32(slots[s].len);
-      if (len <= 0) continue;
-      const int m = active ? int(mult[s * kGroup + lane]) : 0;
-      if (__ballot(m != 0) == 0) continue;  // no lane visits this bucket
-      const int beg = abh::uniform_i32(slots[s].beg);
-      const int img = abh::uniform_i32(slots[s].img);
-      double qi[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-      for (int d = 0; d < D; ++d) qi[d] = image_of((img >> (2 * d)) & 3, q[d], g.L[d]);
-      const int end = beg + len;
-
-      if (MODE == kCount || kList) {
-        // Candidates of this bucket in blocks of 64: each lane loads one and
-        // keeps it if it lies within r of the work item's query box (the
-        // same FP64 operations as the radius test, monotone in the query, so
-        // no accepted pair is dropped); the kept ones are compacted into LDS
-        // in index order and tested against every lane's centre.  acc <= r2
-        // equals the reference's !(acc > r2) for every finite centre (acc is
-        // never NaN there); lanes with m == 0 compare against -1.
-        double blo[3] = {0.0, 0.0, 0.0}, bhi[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-          const int dg = (img >> (2 * d)) & 3;
-          blo[d] = uniform_f64(
-              pick3(dg, qlo[d] + double(-1) * g.L[d], qlo[d], qlo[d] + double(1) * g.L[d]));
-          bhi[d] = uniform_f64(
-              pick3(dg, qhi[d] + double(-1) * g.L[d], qhi[d], qhi[d] + double(1) * g.L[d]));
-        }
-        const double r2m = m != 0 ? a.r2 : -1.0;
-        const bool single = __ballot(m > 1) == 0;
-        for (int c0 = beg; c0 < end; c0 += kGroup) {
-          const int jc = c0 + lane;
-          bool keep = jc < end;
-          double x[3] = {0.0, 0.0, 0.0};
-          if (keep) {
-#pragma unroll
-            for (int d = 0; d < D; ++d) x[d] = a.pos[int64_t(jc) * D + d];
-          }
-          double dd = 0.0;
-#pragma unroll
-          for (int d = 0; d < D; ++d) {
-            double e = 0.0;
-            if (x[d] < blo[d]) e = blo[d] - x[d];
-            else if (x[d] > bhi[d]) e = x[d] - bhi[d];
-            dd = dd + e * e;
-          }
-          keep = keep && dd <= a.r2;
-          const uint64_t km = __ballot(keep);
-          if (km == 0) continue;
-          const int nk = __popcll(km);
-          if (keep) {
-            const int sl = int(__builtin_amdgcn_mbcnt_hi(uint32_t(km >> 32),
-                                                         __builtin_amdgcn_mbcnt_lo(uint32_t(km), 0u)));
-            st[sl] = StageRec{x[0], x[1], x[2], jc, 0};
-          }
-          __syncthreads();  // single-wave group: the staged block is complete
-          if (use_ring && single) {
-            // at most 16 appends per lane between segment stores: a block
-            // starts with the next entry in the segment of the first
-            // unstored one, so fewer than 32 entries are ever unstored and
-            // the slot of the next entry is free.  Every candidate is
-            // written there and the position advances on a hit only.
-            for (int t0 = 0; t0 < nk; t0 += kSeg) {
-              const int t1 = nk - t0 < kSeg ? nk : t0 + kSeg;
-              // byte offset of the next entry's ring slot in bits 8..12
-              const uint32_t k8s = uint32_t(out + cnt) << 8;
-              uint32_t k8 = k8s;
-              int t = t0;
-              for (; t + kStageUnroll <= t1; t += kStageUnroll) {
-                double e[kStageUnroll][3];
-                int jj[kStageUnroll];
-#pragma unroll
-                for (int u = 0; u < kStageUnroll; ++u) load_stage(st[t + u], e[u], jj[u]);
-                bool h[kStageUnroll];
-#pragma unroll
-                for (int u = 0; u < kStageUnroll; ++u) {
-                  double acc = 0.0;
-#pragma unroll
-                  for (int d = 0; d < D; ++d) {
-                    const double dx = e[u][d] - qi[d];
-                    acc = acc + dx * dx;
-                  }
-                  h[u] = acc <= r2m;
-                }
-#pragma unroll
-                for (int u = 0; u < kStageUnroll; ++u) {
-                  ring_put(ring, k8, lane, uint32_t(jj[u]));
-                  k8 += h[u] ? 256u : 0u;
-                }
-              }
-              for (; t < t1; ++t) {
-                double e1[3];
-                int j1;
-                load_stage(st[t], e1, j1);
-                double acc = 0.0;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                  const double dx = e1[d] - qi[d];
-                  acc = acc + dx * dx;
-                }
-                ring_put(ring, k8, lane, uint32_t(j1));
-                k8 += acc <= r2m ? 256u : 0u;
-              }
-              cnt += int((k8 - k8s) >> 8);
-              ring_segment();
-            }
-            __syncthreads();  // the next block overwrites the stage
-            continue;
-          }
-          if (MODE == kCount) {
-            // a hit adds m (1 whenever no lane visits the bucket twice)
-            int t = 0;
-            for (; t + kStageUnroll <= nk; t += kStageUnroll) {
+        __syncthreads();  // single-wave group: the staged block is complete
+        if (use_ring && single) {
+          // at most 16 appends per lane between segment stores: a block
+          // starts with the next entry in the segment of the first
+          // unstored one, so fewer than 32 entries are ever unstored and
+          // the slot of the next entry is free.  Every candidate is
+          // written there and the position advances on a hit only.
+          for (int t0 = 0; t0 < nk; t0 += kSeg) {
+            const int t1 = nk - t0 < kSeg ? nk : t0 + kSeg;
+            // byte offset of the next entry's ring slot in bits 8..12
+            const uint32_t k8s = uint32_t(out + cnt) << 8;
+            uint32_t k8 = k8s;
+            int t = t0;
+            for (; t + kStageUnroll <= t1; t += kStageUnroll) {
               double e[kStageUnroll][3];
               int jj[kStageUnroll];
 #pragma unroll
               for (int u = 0; u < kStageUnroll; ++u) load_stage(st[t + u], e[u], jj[u]);
+              bool h[kStageUnroll];
 #pragma unroll
               for (int u = 0; u < kStageUnroll; ++u) {
                 double acc = 0.0;
@@ -802,10 +771,15 @@ __global__ __launch_bounds__(kGroup) void k_search(SearchArgs a, GridParams g) {
                   const double dx = e[u][d] - qi[d];
                   acc = acc + dx * dx;
                 }
-                cnt += acc <= r2m ? m : 0;
+                h[u] = acc <= r2m;
+              }
+#pragma unroll
+              for (int u = 0; u < kStageUnroll; ++u) {
+                ring_put(ring, k8, lane, uint32_t(jj[u]));
+                k8 += h[u] ? 256u : 0u;
               }
             }
-            for (; t < nk; ++t) {
+            for (; t < t1; ++t) {
               double e1[3];
               int j1;
               load_stage(st[t], e1, j1);
@@ -815,31 +789,33 @@ __global__ __launch_bounds__(kGroup) void k_search(SearchArgs a, GridParams g) {
                 const double dx = e1[d] - qi[d];
                 acc = acc + dx * dx;
               }
-              cnt += acc <= r2m ? m : 0;
+              ring_put(ring, k8, lane, uint32_t(j1));
+              k8 += acc <= r2m ? 256u : 0u;
             }
-            __syncthreads();  // the next block overwrites the stage
-            continue;
+            cnt += int((k8 - k8s) >> 8);
+            ring_segment();
           }
-          if (use_ring) ring_drain();  // several visits of one bucket: direct stores
+          __syncthreads();  // the next block overwrites the stage
+          continue;
+        }
+        if (MODE == kCount) {
+          // a hit adds m (1 whenever no lane visits the bucket twice)
           int t = 0;
           for (; t + kStageUnroll <= nk; t += kStageUnroll) {
             double e[kStageUnroll][3];
             int jj[kStageUnroll];
 #pragma unroll
             for (int u = 0; u < kStageUnroll; ++u) load_stage(st[t + u], e[u], jj[u]);
-            double acc[kStageUnroll];
 #pragma unroll
             for (int u = 0; u < kStageUnroll; ++u) {
-              acc[u] = 0.0;
+              double acc = 0.0;
 #pragma unroll
               for (int d = 0; d < D; ++d) {
                 const double dx = e[u][d] - qi[d];
-                acc[u] = acc[u] + dx * dx;
+                acc = acc + dx * dx;
               }
+              cnt += acc <= r2m ? m : 0;
             }
-#pragma unroll
-            for (int u = 0; u < kStageUnroll; ++u)
-              staged_hit<MODE>(a, single, acc[u] <= r2m, acc[u], jj[u], m, wrow, out, cnt);
           }
           for (; t < nk; ++t) {
             double e1[3];
@@ -851,157 +827,55 @@ __global__ __launch_bounds__(kGroup) void k_search(SearchArgs a, GridParams g) {
               const double dx = e1[d] - qi[d];
               acc = acc + dx * dx;
             }
-            staged_hit<MODE>(a, single, acc <= r2m, acc, j1, m, wrow, out, cnt);
+            cnt += acc <= r2m ? m : 0;
           }
-          if (use_ring) fpos = out + cnt;
           __syncthreads();  // the next block overwrites the stage
+          continue;
         }
-      } else {
-        // matvec: the candidates are staged and culled as in the list
-        // passes, with their right-hand sides; every lane then evaluates the
-        // kernel for the staged candidates within its radius, in candidate
-        // order (y += f x for each of the m visits)
-        double blo[3] = {0.0, 0.0, 0.0}, bhi[3] = {0.0, 0.0, 0.0};
+        if (use_ring) ring_drain();  // several visits of one bucket: direct stores
+        int t = 0;
+        for (; t + kStageUnroll <= nk; t += kStageUnroll) {
+          double e[kStageUnroll][3];
+          int jj[kStageUnroll];
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-          const int dg = (img >> (2 * d)) & 3;
-          blo[d] = uniform_f64(
-              pick3(dg, qlo[d] + double(-1) * g.L[d], qlo[d], qlo[d] + double(1) * g.L[d]));
-          bhi[d] = uniform_f64(
-              pick3(dg, qhi[d] + double(-1) * g.L[d], qhi[d], qhi[d] + double(1) * g.L[d]));
-        }
-        const double r2m = m != 0 ? a.r2 : -1.0;
-        for (int c0 = beg; c0 < end; c0 += kGroup) {
-          const int jc = c0 + lane;
-          bool keep = jc < end;
-          double x[3] = {0.0, 0.0, 0.0};
-          if (keep) {
+          for (int u = 0; u < kStageUnroll; ++u) load_stage(st[t + u], e[u], jj[u]);
+          double acc[kStageUnroll];
 #pragma unroll
-            for (int d = 0; d < D; ++d) x[d] = a.pos[int64_t(jc) * D + d];
-          }
-          double dd = 0.0;
-#pragma unroll
-          for (int d = 0; d < D; ++d) {
-            double e = 0.0;
-            if (x[d] < blo[d]) e = blo[d] - x[d];
-            else if (x[d] > bhi[d]) e = x[d] - bhi[d];
-            dd = dd + e * e;
-          }
-          keep = keep && dd <= a.r2;
-          const uint64_t km = __ballot(keep);
-          if (km == 0) continue;
-          const int nk = __popcll(km);
-          if (keep) {
-            const int sl = int(__builtin_amdgcn_mbcnt_hi(uint32_t(km >> 32),
-                                                         __builtin_amdgcn_mbcnt_lo(uint32_t(km), 0u)));
-            st[sl] = StageRec{x[0], x[1], x[2], jc, 0};
-            if (MODE == kMatvec32) {
-              // the FP32 form stages its right-hand sides in FP32 (rounded
-              // once here instead of at every use)
-              float *xf = reinterpret_cast<float *>(xs);
-#pragma unroll
-              for (int r = 0; r < kMaxRhs; ++r)
-                xf[sl * kMaxRhs + r] = r < a.nrhs ? float(a.x[int64_t(r) * a.ldx + jc]) : 0.0f;
-            } else {
-#pragma unroll
-              for (int r = 0; r < kMaxRhs; ++r)
-                xs[sl * kMaxRhs + r] = r < a.nrhs ? a.x[int64_t(r) * a.ldx + jc] : 0.0;
-            }
-          }
-          __syncthreads();  // single-wave group: the staged block is complete
-          // radius tests of the whole block first, this lane's hits as bits
-          // (candidate t at bit nk - 1 - t), then the kernel for the hits
-          // only, in candidate order: a round evaluates one hit per lane,
-          // so lanes do not wait on the kernels of candidates they miss
-          uint64_t hm = 0;
-          {
-            int t = 0;
-            for (; t + kStageUnroll <= nk; t += kStageUnroll) {
-              double e[kStageUnroll][3];
-              int jj[kStageUnroll];
-#pragma unroll
-              for (int u = 0; u < kStageUnroll; ++u) load_stage(st[t + u], e[u], jj[u]);
-#pragma unroll
-              for (int u = 0; u < kStageUnroll; ++u) {
-                double acc = 0.0;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                  const double dx = e[u][d] - qi[d];
-                  acc = acc + dx * dx;
-                }
-                hm = (hm << 1) + (acc <= r2m ? 1ull : 0ull);
-              }
-            }
-            for (; t < nk; ++t) {
-              double e1[3];
-              int j1;
-              load_stage(st[t], e1, j1);
-              double acc = 0.0;
-#pragma unroll
-              for (int d = 0; d < D; ++d) {
-                const double dx = e1[d] - qi[d];
-                acc = acc + dx * dx;
-              }
-              hm = (hm << 1) + (acc <= r2m ? 1ull : 0ull);
-            }
-          }
-          // (a divergent loop: the wave runs as many rounds as its lane
-          // with the most hits)
-          while (hm != 0) {
-            const int p = 63 - __builtin_clzll(hm);
-            hm ^= 1ull << p;
-            const int t = nk - 1 - p;
-            double e1[3];
-            int j1;
-            load_stage(st[t], e1, j1);
-            double acc = 0.0;
+          for (int u = 0; u < kStageUnroll; ++u) {
+            acc[u] = 0.0;
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-              const double dx = e1[d] - qi[d];
-              acc = acc + dx * dx;
-            }
-            double w = wrow;
-            if (a.k.col_s) w = w + a.k.wc * a.k.col_s[j1];
-            const double *xr = xs + t * kMaxRhs;
-            if (MODE == kMatvec64) {
-              const double f = phi64(a.k, acc) * w;
-              for (int rep = 0; rep < m; ++rep) {
-#pragma unroll
-                for (int r = 0; r < kMaxRhs; ++r)
-                  if (r < a.nrhs) acc64[r] += f * xr[r];
-              }
-            } else {
-              const float f = phi32(a.k, float(acc)) * float(w);
-              const float *xf = reinterpret_cast<const float *>(xs) + t * kMaxRhs;
-              for (int rep = 0; rep < m; ++rep) {
-#pragma unroll
-                for (int r = 0; r < kMaxRhs; ++r)
-                  if (r < a.nrhs) kb_add(acc32[r], cmp32[r], f * xf[r]);
-              }
+              const double dx = e[u][d] - qi[d];
+              acc[u] = acc[u] + dx * dx;
             }
           }
-          __syncthreads();  // the next block overwrites the stage
+#pragma unroll
+          for (int u = 0; u < kStageUnroll; ++u)
+            staged_hit<MODE>(a, single, acc[u] <= r2m, acc[u], jj[u], m, wrow, out, cnt);
         }
+        for (; t < nk; ++t) {
+          double e1[3];
+          int j1;
+          load_stage(st[t], e1, j1);
+          double acc = 0.0;
+#pragma unroll
+          for (int d = 0; d < D; ++d) {
+            const double dx = e1[d] - qi[d];
+            acc = acc + dx * dx;
+          }
+          staged_hit<MODE>(a, single, acc <= r2m, acc, j1, m, wrow, out, cnt);
+        }
+        if (use_ring) fpos = out + cnt;
+        __syncthreads();  // the next block overwrites the stage
       }
     }
-    if (use_ring) ring_drain();
-    if (has_row) {
-      if (MODE == kCount || MODE == kFillPadded) a.counts[row] = cnt;
-      if (MODE == kMatvec64) {
-#pragma unroll
-        for (int r = 0; r < kMaxRhs; ++r)
-          if (r < a.nrhs) a.y[int64_t(r) * a.ldy + row] = acc64[r];
-      }
-      if (MODE == kMatvec32) {
-#pragma unroll
-        for (int r = 0; r < kMaxRhs; ++r)
-          if (r < a.nrhs)
-            a.y[int64_t(r) * a.ldy + row] = acc64[r] + (double(acc32[r]) + double(cmp32[r]));
-      }
-    }
-    __syncthreads();  // slots / mult reused by the next work item
   }
+  if (use_ring) ring_drain();
+  if (has_row && (MODE == kCount || MODE == kFillPadded)) a.counts[row] = cnt;
 }
+
+#include "search_matvec.hpp"
+#include "search_group.hpp"
 
 // xr[j][r] = x[r][j] (r < nrhs, zero beyond): the right-hand sides of one
 // column in one 64-byte segment for the CSR product's gathers
@@ -1135,11 +1009,18 @@ struct QueryPlan {
   bool self = false;      // centres are the cell list's own positions
   bool permuted = false;  // centres were sorted (perm / qbuf hold the order)
   int sub_levels = 0;     // Morton sub-cell levels inside a home cell
+  // every query goes to k_search_group, in the order given (no sort and no
+  // work lists); otherwise the two lists of k_plan_items
+  bool all_light = false;
+  double light_most = kLightSearch;
+  bool group = false;  // k_search_group serves some of the queries
   double radius = 0, r2 = 0;
   int w[3] = {0, 0, 0};
   int nslots = 1;
   const double *q_sorted = nullptr;
-  DevBuf qbuf, perm, keys, flags, ridx, run_start, chunks, choff, work, counters, escape, sched;
+  int64_t max_work = 0;  // work items, or an upper bound before the first count
+  DevBuf qbuf, perm, keys, work, light;
+  DevBuf counters;  // listed queries, work items, escape flag
 
   const int32_t *qperm() const { return permuted ? perm.as<int32_t>() : nullptr; }
 };
@@ -1168,19 +1049,89 @@ static void set_stencil(QueryPlan &p, int extra) {
               "use fewer particles per bucket or a smaller radius");
 }
 
+// k_search_group walks a stencil of at most kGlMaxSlots buckets in which no
+// bucket occurs twice.
+static bool group_fits(const QueryPlan &p) {
+  if (p.nslots > kGlMaxSlots) return false;
+  for (int d = 0; d < p.D; ++d)
+    if (p.cells->periodic[d] && int64_t(p.cells->size[d]) < 2 * p.w[d] + 1) return false;
+  return true;
+}
+
+// Whether the cells hold few particles: the mean occupancy of a particle's
+// bucket (the squared bucket counts over the particles, which is what the
+// candidate tests of the set against itself grow with) is at most `most`.
+// The sum is read back once per build.  Sets of up to kSmall particles are
+// served by k_search_group whatever their cells: in one bucket, 16,384 x
+// 16,384 tests take less there than the chains of a few work items.
+static bool cells_light(const abh_cells *c, double most) {
+  if (c->n_alive <= kSmall) return true;
+  if (!c->sq_known) {
+    BuildCounters h{};
+    ABH_HIP(hipMemcpyAsync(&h, c->counters.p, sizeof(h), hipMemcpyDeviceToHost, c->ctx->stream));
+    ABH_HIP(hipStreamSynchronize(c->ctx->stream));
+    c->sq_sum = h.sq_sum;
+    c->sq_known = true;
+  }
+  return double(c->sq_sum) <= most * double(c->n_alive);
+}
+
+template <int D> static void plan_items(QueryPlan &p) {
+  abh_context *ctx = p.ctx;
+  const int64_t n = p.nq;
+  p.work.ensure(size_t(n + 1) * sizeof(WorkItem));
+  p.light.ensure(size_t(n + 1) * 4);
+  uint32_t *ctr = p.counters.as<uint32_t>();  // [0] = listed queries, [1] = work items
+  ABH_HIP(hipMemsetAsync(ctr, 0, 8, ctx->stream));
+  k_plan_items<D><<<unsigned(ceil_div(n, kThreads)), kThreads, 0, ctx->stream>>>(
+      p.keys.as<uint32_t>(), n, p.sub_levels * D, p.group ? kHeavyMin : 1, p.q_sorted,
+      p.cells->params(), p.work.as<WorkItem>(), p.light.as<int32_t>(), ctr);
+  check_launch();
+  // every item holds kHeavyMin queries; without the list there may be as many
+  // items as queries, and it pays to wait for their number
+  p.max_work = n / kHeavyMin;
+  if (!p.group) {
+    uint32_t h = 0;
+    ABH_HIP(hipMemcpyAsync(&h, ctr + 1, 4, hipMemcpyDeviceToHost, ctx->stream));
+    ABH_HIP(hipStreamSynchronize(ctx->stream));
+    p.max_work = h;
+  }
+}
+
 template <int D> static void build_plan_d(QueryPlan &p, const double *q) {
   abh_context *ctx = p.ctx;
   hipStream_t s = ctx->stream;
   const GridParams g = p.cells->params();
   const int64_t n = p.nq;
   const unsigned blocks = unsigned(ceil_div(n, kThreads));
-  p.keys.ensure(size_t(n + 1) * 4);
-  uint32_t *keys = p.keys.as<uint32_t>();
   uint64_t maxkey = 1;
   for (int d = 0; d < D; ++d)
     maxkey *= uint64_t(g.periodic[d] ? 3 * g.size[d] : g.size[d] + 2);
   int bits = 0;
   while (bits < 64 && ((maxkey - 1) >> bits) != 0) ++bits;
+  ABH_REQUIRE(p.self || bits <= 32, ABH_ERR_UNSUPPORTED,
+              "too many buckets to group arbitrary centres; search from the particle "
+              "positions themselves");
+  p.group = group_fits(p);
+  p.counters.ensure(16);
+  p.max_work = 0;
+  // Without sorting: the particles lie in bucket order, and for centres in
+  // random order the reads that this scatters cost less than the sort (1 and
+  // 4 million random centres, 8 particles a cell in 3D: search 2.24 and
+  // 7.76 ms sorted, 1.33 and 6.63 ms as they come).  The plan keeps a copy of
+  // the centres.
+  p.all_light = p.group && cells_light(p.cells, p.light_most);
+  if (p.all_light) {
+    ABH_HIP(hipMemsetAsync(p.counters.p, 0, 8, s));
+    p.sub_levels = 0;
+    p.permuted = false;
+    p.qbuf.ensure(size_t(n + 1) * D * 8);
+    ABH_HIP(hipMemcpyAsync(p.qbuf.p, q, size_t(n) * D * 8, hipMemcpyDeviceToDevice, s));
+    p.q_sorted = p.qbuf.as<double>();
+    return;
+  }
+  p.keys.ensure(size_t(n + 1) * 4);
+  uint32_t *keys = p.keys.as<uint32_t>();
   // sub-cell levels that fit the 32-bit key (at most 2: 4^D sub-cells)
   int levels = 0;
   while (levels < 2 && bits + (levels + 1) * D <= 32) ++levels;
@@ -1191,9 +1142,6 @@ template <int D> static void build_plan_d(QueryPlan &p, const double *q) {
     k_home_keys<D><<<blocks, kThreads, 0, s>>>(q, n, g, 0, keys, nullptr);
     check_launch();
   } else {
-    ABH_REQUIRE(bits <= 32, ABH_ERR_UNSUPPORTED,
-                "too many buckets to group arbitrary centres; search from the particle "
-                "positions themselves");
     p.perm.ensure(size_t(n + 1) * 4);
     k_home_keys<D><<<blocks, kThreads, 0, s>>>(q, n, g, levels, keys, p.perm.as<int32_t>());
     check_launch();
@@ -1202,29 +1150,34 @@ template <int D> static void build_plan_d(QueryPlan &p, const double *q) {
     gather_bytes(ctx, p.perm.as<int32_t>(), n, q, p.qbuf.p, size_t(D) * 8);
     p.q_sorted = p.qbuf.as<double>();
   }
-  p.flags.ensure(size_t(n + 1) * 4);
-  p.ridx.ensure(size_t(n + 1) * 4);
-  p.run_start.ensure(size_t(n + 1) * 4);
-  p.chunks.ensure(size_t(n + 1) * 4);
-  p.choff.ensure(size_t(n + 1) * 4);
-  p.work.ensure(size_t(n + 1) * sizeof(WorkItem));
-  p.counters.ensure(16);
-  p.sched.ensure(16);
-  uint32_t *ctr = p.counters.as<uint32_t>();  // [0] = runs, [1] = work items
-  k_run_flags<<<blocks, kThreads, 0, s>>>(keys, n, p.sub_levels * D, p.flags.as<uint32_t>());
-  check_launch();
-  scan_exclusive(ctx, p.flags.as<uint32_t>(), p.ridx.as<uint32_t>(), n, ctr + 0);
-  k_run_starts<<<blocks, kThreads, 0, s>>>(p.flags.as<uint32_t>(), p.ridx.as<uint32_t>(), n,
-                                           p.run_start.as<uint32_t>());
-  check_launch();
-  k_run_chunks<<<blocks, kThreads, 0, s>>>(p.run_start.as<uint32_t>(), ctr + 0, n,
-                                           p.chunks.as<uint32_t>());
-  check_launch();
-  scan_exclusive(ctx, p.chunks.as<uint32_t>(), p.choff.as<uint32_t>(), n, ctr + 1);
-  k_fill_work<D><<<blocks, kThreads, 0, s>>>(p.run_start.as<uint32_t>(), ctr + 0, n,
-                                             p.choff.as<uint32_t>(), p.chunks.as<uint32_t>(),
-                                             p.q_sorted, g, p.work.as<WorkItem>());
-  check_launch();
+  plan_items<D>(p);
+}
+
+// The stencil was widened past what k_search_group walks: every query
+// becomes part of a work item of k_search.
+template <int D> static void all_heavy_d(QueryPlan &p) {
+  if (!p.all_light) {
+    p.group = false;
+    plan_items<D>(p);
+    return;
+  }
+  DevBuf own;
+  std::swap(own.p, p.qbuf.p);
+  std::swap(own.bytes, p.qbuf.bytes);
+  build_plan_d<D>(p, own.as<double>());
+  if (!p.permuted) {  // q_sorted is the copy itself
+    std::swap(own.p, p.qbuf.p);
+    std::swap(own.bytes, p.qbuf.bytes);
+  }
+  ABH_HIP(hipStreamSynchronize(p.ctx->stream));
+}
+
+static void widen_stencil(QueryPlan &p, int extra) {
+  set_stencil(p, extra);
+  if (!p.group || group_fits(p)) return;
+  if (p.D == 1) all_heavy_d<1>(p);
+  else if (p.D == 2) all_heavy_d<2>(p);
+  else all_heavy_d<3>(p);
 }
 
 static void build_plan(QueryPlan &p, abh_context *ctx, const abh_cells *cells, int64_t nq,
@@ -1263,36 +1216,57 @@ static SearchArgs base_args(const QueryPlan &p) {
 }
 
 // dynamic LDS of k_search (the fill passes add their static output ring)
-static size_t lds_bytes(int nslots, bool matvec) {
-  const size_t slots = size_t(nslots) * (sizeof(Slot) + 4 + kGroup) + 4 * size_t(nslots + 1);
-  return ((slots + 15) & ~size_t(15)) + size_t(kGroup) * sizeof(StageRec) +
-         (matvec ? size_t(kGroup) * kMaxRhs * sizeof(double) : 0);
+static size_t lds_bytes(int nslots) {
+  const size_t slots = size_t(nslots) * (sizeof(Slot) + 4 + kGroup);
+  return ((slots + 15) & ~size_t(15)) + size_t(kGroup) * sizeof(StageRec);
 }
 
-__global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
-
-template <int MODE> static void launch_search(const QueryPlan &p, const SearchArgs &a0) {
-  // persistent waves per CU: the list passes run best at 16 (measured on
-  // the 4M-particle mixture: 9.4 / 14.3 ms at 16 against 10.0 / 15.6 ms at
-  // 32; 8 leaves the scalar-load latency exposed)
-  const int wpc = (MODE == kMatvec64 || MODE == kMatvec32) ? 32 : 16;
-  const unsigned grid = unsigned(std::min<int64_t>(ceil_div(p.nq, kGroup), int64_t(p.ctx->n_cu) * wpc));
-  if (grid == 0) return;
-  SearchArgs a = a0;
-  a.next = p.sched.as<uint32_t>();
-  ABH_REQUIRE(a.next, ABH_ERR_INVALID_ARG, "search plan not built");
-  k_zero_u32<<<1, 1, 0, p.ctx->stream>>>(a.next);
+template <int D, int MODE>
+static void launch_group(const QueryPlan &p, const SearchArgs &a, const GridParams &g) {
+  // all queries, or the ones k_plan_items listed (how many is on the device:
+  // blocks past the end return at once)
+  const int32_t *list = p.all_light ? nullptr : p.light.as<int32_t>();
+  const uint32_t *nlist = p.all_light ? nullptr : p.counters.as<uint32_t>();
+  const unsigned grid = unsigned(ceil_div(p.nq, kGlGroups));
+  constexpr bool kMV = MODE == kMatvec64 || MODE == kMatvec32;
+  k_search_group<D, MODE><<<grid, kGlThreads, group_lds_bytes(a.nslots, kMV), p.ctx->stream>>>(
+      a, g, list, nlist, p.nq);
   check_launch();
+}
+
+template <int D, bool FP32>
+static void launch_matvec(const QueryPlan &p, const SearchArgs &a, const GridParams &g,
+                          unsigned grid) {
+  hipStream_t s = p.ctx->stream;
+  const int nr = a.nrhs == 1 ? 1 : (a.nrhs == 2 ? 2 : (a.nrhs <= 4 ? 4 : 8));
+  const size_t lds = matvec_lds_bytes(a.nslots, nr, FP32);
+  if (nr == 1) k_matvec<D, FP32, 1><<<grid, kGroup, lds, s>>>(a, g);
+  else if (nr == 2) k_matvec<D, FP32, 2><<<grid, kGroup, lds, s>>>(a, g);
+  else if (nr == 4) k_matvec<D, FP32, 4><<<grid, kGroup, lds, s>>>(a, g);
+  else k_matvec<D, FP32, 8><<<grid, kGroup, lds, s>>>(a, g);
+  check_launch();
+}
+
+template <int D, int MODE> static void launch_search_d(const QueryPlan &p, const SearchArgs &a) {
   const GridParams g = p.cells->params();
-  const size_t lds = lds_bytes(a.nslots, MODE == kMatvec64 || MODE == kMatvec32);
-  if (p.D == 1) k_search<1, MODE><<<grid, kGroup, lds, p.ctx->stream>>>(a, g);
-  else if (p.D == 2) k_search<2, MODE><<<grid, kGroup, lds, p.ctx->stream>>>(a, g);
-  else k_search<3, MODE><<<grid, kGroup, lds, p.ctx->stream>>>(a, g);
-  check_launch();
+  if (p.group) launch_group<D, MODE>(p, a, g);
+  if (p.all_light || p.max_work == 0) return;
+  const unsigned grid = unsigned(p.max_work);
+  if constexpr (MODE == kMatvec64 || MODE == kMatvec32) {
+    launch_matvec<D, MODE == kMatvec32>(p, a, g, grid);
+  } else {
+    k_search<D, MODE><<<grid, kGroup, lds_bytes(a.nslots), p.ctx->stream>>>(a, g);
+    check_launch();
+  }
 }
 
-// Counts neighbours into counts[nq] (device), widening the stencil until no
-// query's visited buckets escape it.
+template <int MODE> static void launch_search(const QueryPlan &p, const SearchArgs &a) {
+  if (p.nq == 0) return;
+  if (p.D == 1) launch_search_d<1, MODE>(p, a);
+  else if (p.D == 2) launch_search_d<2, MODE>(p, a);
+  else launch_search_d<3, MODE>(p, a);
+}
+
 // col[row_ptr[i] + e] = padded[pad_ptr[i] + e], one wavefront per row
 // (the row's body is stored 16 bytes per lane from its first 16-byte
 // aligned address, head and tail element by element)
@@ -1318,37 +1292,24 @@ __global__ __launch_bounds__(256) void k_compact_rows(const int64_t *__restrict_
   if (lane < rem) col[d0 + 4 * nb4 + lane] = padded[s0 + 4 * nb4 + lane];
 }
 
-// Like count_with_escape, with the capacity pass (no distance tests).
-static void capacity_with_escape(QueryPlan &p, int64_t *caps) {
-  p.escape.ensure(4);
+// Row counts (kCount) or upper bounds of them (kCapacity, no distance tests)
+// into counts[nq] (device), widening the stencil until no query's visited
+// buckets escape it.  Reading the escape flag back also tells how many work
+// items there are, for the launches that follow.
+template <int MODE> static void count_with_escape(QueryPlan &p, int64_t *counts) {
   for (int extra = 0;; ++extra) {
-    if (extra > 0) set_stencil(p, extra);
-    ABH_HIP(hipMemsetAsync(p.escape.p, 0, 4, p.ctx->stream));
-    SearchArgs a = base_args(p);
-    a.counts = caps;
-    a.escape_flag = p.escape.as<uint32_t>();
-    launch_search<kCapacity>(p, a);
-    uint32_t esc = 0;
-    ABH_HIP(hipMemcpyAsync(&esc, p.escape.p, 4, hipMemcpyDeviceToHost, p.ctx->stream));
-    ABH_HIP(hipStreamSynchronize(p.ctx->stream));
-    if (!esc) return;
-    ABH_REQUIRE(extra < 4, ABH_ERR_UNSUPPORTED, "search stencil failed to cover visited buckets");
-  }
-}
-
-static void count_with_escape(QueryPlan &p, int64_t *counts) {
-  p.escape.ensure(4);
-  for (int extra = 0;; ++extra) {
-    if (extra > 0) set_stencil(p, extra);
-    ABH_HIP(hipMemsetAsync(p.escape.p, 0, 4, p.ctx->stream));
+    if (extra > 0) widen_stencil(p, extra);
+    uint32_t *ctr = p.counters.as<uint32_t>();
+    ABH_HIP(hipMemsetAsync(ctr + 2, 0, 4, p.ctx->stream));
     SearchArgs a = base_args(p);
     a.counts = counts;
-    a.escape_flag = p.escape.as<uint32_t>();
-    launch_search<kCount>(p, a);
-    uint32_t esc = 0;
-    ABH_HIP(hipMemcpyAsync(&esc, p.escape.p, 4, hipMemcpyDeviceToHost, p.ctx->stream));
+    a.escape_flag = ctr + 2;
+    launch_search<MODE>(p, a);
+    uint32_t h[2] = {0, 0};
+    ABH_HIP(hipMemcpyAsync(h, ctr + 1, 8, hipMemcpyDeviceToHost, p.ctx->stream));
     ABH_HIP(hipStreamSynchronize(p.ctx->stream));
-    if (!esc) return;
+    p.max_work = h[0];
+    if (!h[1]) return;
     ABH_REQUIRE(extra < 4, ABH_ERR_UNSUPPORTED, "search stencil failed to cover visited buckets");
   }
 }
@@ -1440,7 +1401,7 @@ abh_status abh_search_update(abh_search *s, const abh_cells *cells, int64_t nq,
     s->total_buf.ensure(8);
     int64_t *rp = s->row_ptr.as<int64_t>();
     ABH_HIP(hipMemsetAsync(rp + nq, 0, 8, ctx->stream));
-    if (nq > 0) abh::count_with_escape(s->plan, rp);
+    if (nq > 0) abh::count_with_escape<kCount>(s->plan, rp);
     int64_t *total_dev = s->total_buf.as<int64_t>();
     abh::scan_exclusive(ctx, rp, rp, nq + 1, total_dev);
     int64_t total = 0;
@@ -1523,7 +1484,7 @@ abh_status abh_search_run_fused(abh_search *s, const abh_cells *cells, int64_t n
     ABH_HIP(hipMemsetAsync(rp + nq, 0, 8, st));
     int64_t padded_total = 0;
     if (nq > 0) {
-      abh::capacity_with_escape(s->plan, pp);
+      abh::count_with_escape<kCapacity>(s->plan, pp);
       abh::scan_exclusive(ctx, pp, pp, nq + 1, s->total_buf.as<int64_t>());
       ABH_HIP(hipMemcpyAsync(&padded_total, s->total_buf.p, 8, hipMemcpyDeviceToHost, st));
       ABH_HIP(hipStreamSynchronize(st));
@@ -1569,6 +1530,7 @@ abh_status abh_sparse_op_create(abh_context *ctx, const abh_cells *cols, int64_t
     ABH_REQUIRE(!ctx->closed, ABH_ERR_INVALID_ARG, "context already destroyed");
     ABH_REQUIRE(kernel->type >= ABH_KERNEL_CONSTANT && kernel->type <= ABH_KERNEL_SMOOTH_INV_R,
                 ABH_ERR_UNSUPPORTED, "unknown kernel type");
+    op->plan.light_most = kLightOp;
     abh::build_plan(op->plan, ctx, cols, nrows, row_pos, radius);
     op->ncols = cols->n_alive;
     op->k.type = kernel->type;
@@ -1586,7 +1548,7 @@ abh_status abh_sparse_op_create(abh_context *ctx, const abh_cells *cols, int64_t
       counts.ensure(size_t(nrows + 1) * 8);
       int64_t *c = counts.as<int64_t>();
       ABH_HIP(hipMemsetAsync(c + nrows, 0, 8, ctx->stream));
-      abh::count_with_escape(op->plan, c);
+      abh::count_with_escape<kCount>(op->plan, c);
       abh::DevBuf total_buf;
       total_buf.ensure(8);
       int64_t *total_dev = total_buf.as<int64_t>();
@@ -1625,7 +1587,7 @@ abh_status abh_sparse_op_assemble(abh_sparse_op *op, int64_t *row_ptr, int32_t *
     ABH_REQUIRE(op->nnz == 0 || (col && val), ABH_ERR_INVALID_ARG, "col or val is null");
     ABH_HIP(hipMemsetAsync(row_ptr + nq, 0, 8, ctx->stream));
     if (nq == 0) return;
-    abh::count_with_escape(op->plan, row_ptr);
+    abh::count_with_escape<kCount>(op->plan, row_ptr);
     abh::DevBuf total_buf;
     total_buf.ensure(8);
     abh::scan_exclusive(ctx, row_ptr, row_ptr, nq + 1, total_buf.as<int64_t>());
@@ -1696,7 +1658,7 @@ abh_status abh_sparse_op_cache(abh_sparse_op *op, abh_precision precision, int e
     }
     int64_t *rp = op->c_rp.as<int64_t>();
     ABH_HIP(hipMemsetAsync(rp + nq, 0, 8, ctx->stream));
-    abh::count_with_escape(op->plan, rp);
+    abh::count_with_escape<kCount>(op->plan, rp);
     abh::DevBuf total_buf;
     total_buf.ensure(8);
     abh::scan_exclusive(ctx, rp, rp, nq + 1, total_buf.as<int64_t>());
