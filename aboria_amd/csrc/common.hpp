@@ -53,6 +53,17 @@ struct DevBuf {
     ABH_HIP(hipMalloc(&p, alloc));
     bytes = alloc;
   }
+  // at least `want` bytes, without room to grow
+  void ensure_exact(size_t want) {
+    if (want <= bytes && p) return;
+    release();
+    ABH_HIP(hipMalloc(&p, want));
+    bytes = want;
+  }
+  void swap(DevBuf &o) {
+    std::swap(p, o.p);
+    std::swap(bytes, o.bytes);
+  }
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
@@ -78,6 +89,13 @@ struct abh_context {
   abh::DevBuf scan_blocks;                     // per-tile sums of scan_exclusive
   abh::DevBuf sort_keys, sort_vals, sort_hist;  // radix sort ping-pong + histograms
   abh::DevBuf dense_part;                       // column-split partial sums (abh_dense_apply)
+  // Schwarz set-up (schwarz.hip): the working set of a factorisation group (at
+  // most about 3 GB) and the inverse rows of the last preconditioner
+  // destroyed (at most 4 GB), kept for the next one until the context goes or
+  // memory runs out.  Once a process has cycled through the card's memory the
+  // driver clears what is freed, about 28 ms per GB.
+  abh::DevBuf factor_a, factor_d, factor_ds, factor_w, factor_sg;
+  abh::DevBuf factor_spare;
   int n_cu = 256;
   // device address of the static scratch of abh_dense_apply_noalloc on this
   // context's device (hipGetSymbolAddress at context creation)

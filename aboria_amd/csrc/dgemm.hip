@@ -14,8 +14,11 @@
 // of lane l holds C[m = l % 16][n = l / 16 + 4 v] and the 16 lanes of a
 // group store 16 consecutive rows of a column (128 contiguous bytes).
 //
-// lower_only skips the tiles that lie strictly above the diagonal (a
-// symmetric trailing update whose upper triangle is never read).
+// C may be A or B where a workgroup's tile reads only the rows or columns
+// that it writes (one tile across the other dimension): all its loads come
+// before its stores.  In large batches all tiles of one matrix run on one XCD
+// (blocks go to the 8 XCDs round robin), whose L2 then holds the operand they
+// share; a few matrices would leave XCDs idle that way.
 #include "common.hpp"
 #include "solvers.hpp"
 
@@ -29,16 +32,17 @@ constexpr int kLd = kT + 1;
 
 template <bool TA, bool TB>
 __global__ __launch_bounds__(256) void k_dgemm(int M, int N, int K, double alpha,
-                                               const double *__restrict__ A, int lda,
-                                               int64_t sA, const double *__restrict__ B, int ldb,
-                                               int64_t sB, double beta, double *__restrict__ C,
-                                               int ldc, int64_t sC, int tiles_m, int lower_only) {
+                                               const double *A, int lda, int64_t sA,
+                                               const double *B, int ldb, int64_t sB, double beta,
+                                               double *C, int ldc, int64_t sC, int tiles_m,
+                                               int tiles, int batch, int xcds, int from_c) {
   __shared__ double As[kK][kLd];  // op(A)[m][k] stored [k][m]
   __shared__ double Bs[kK][kLd];  // op(B)[k][n] stored [k][n]
-  const int g = blockIdx.y;
-  const int tm = int(blockIdx.x) % tiles_m, tn = int(blockIdx.x) / tiles_m;
+  const int q = int(blockIdx.x) / xcds;
+  const int g = (q / tiles) * xcds + int(blockIdx.x) % xcds;
+  if (g >= batch) return;  // uniform over the workgroup
+  const int tm = (q % tiles) % tiles_m, tn = (q % tiles) / tiles_m;
   const int m0 = tm * kT, n0 = tn * kT;
-  if (lower_only && m0 + kT - 1 < n0) return;  // uniform over the workgroup
   A += int64_t(g) * sA;
   B += int64_t(g) * sB;
   C += int64_t(g) * sC;
@@ -88,6 +92,24 @@ __global__ __launch_bounds__(256) void k_dgemm(int M, int N, int K, double alpha
     for (int j = 0; j < 2; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
 
   const int kl = lane >> 4, rl = lane & 15;
+  // acc[i][j][v] = C[m = m0 + wm + 16 i + rl][n = n0 + wn + 16 j + kl + 4 v].
+  // from_c: the sums start from beta C / alpha (alpha is 1 or -1), so that an
+  // update that nearly cancels C rounds at the size of what is left of it, not
+  // at the size of the whole product
+  if (from_c) {
+    const double f = beta * alpha;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int gm = m0 + wm + 16 * i + rl;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int gn = n0 + wn + 16 * j + kl + 4 * v;
+          if (gm < M && gn < N) acc[i][j][v] = f * C[int64_t(gn) * ldc + gm];
+        }
+    }
+  }
   load(0);
   for (int k0 = 0; k0 < K; k0 += kK) {
     __syncthreads();
@@ -109,7 +131,6 @@ __global__ __launch_bounds__(256) void k_dgemm(int M, int N, int K, double alpha
           acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[j], fb[i], acc[i][j], 0, 0, 0);
     }
   }
-  // acc[i][j][v] = C[m = m0 + wm + 16 i + rl][n = n0 + wn + 16 j + kl + 4 v]
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int gm = m0 + wm + 16 * i + rl;
@@ -122,7 +143,7 @@ __global__ __launch_bounds__(256) void k_dgemm(int M, int N, int K, double alpha
         if (gn >= N) continue;
         double *c = C + int64_t(gn) * ldc + gm;
         const double r = alpha * acc[i][j][v];
-        *c = beta == 0.0 ? r : r + beta * *c;
+        *c = beta == 0.0 || from_c ? r : r + beta * *c;
       }
   }
 }
@@ -134,32 +155,35 @@ namespace abh {
 void dgemm_strided_batched(hipStream_t st, bool ta, bool tb, int m, int n, int k, double alpha,
                            const double *A, int lda, int64_t sA, const double *B, int ldb,
                            int64_t sB, double beta, double *C, int ldc, int64_t sC, int batch,
-                           bool lower_only) {
+                           bool from_c) {
   if (m <= 0 || n <= 0 || batch <= 0) return;
   ABH_REQUIRE(k >= 0 && lda >= 1 && ldb >= 1 && ldc >= m, ABH_ERR_INVALID_ARG,
               "dgemm: bad leading dimension");
+  ABH_REQUIRE(!from_c || alpha == 1.0 || alpha == -1.0, ABH_ERR_INVALID_ARG,
+              "dgemm: alpha must be 1 or -1");
   ABH_REQUIRE(batch <= 65535, ABH_ERR_INVALID_ARG, "dgemm: batch too large");
   const int tm = int(ceil_div(m, kT)), tn = int(ceil_div(n, kT));
-  ABH_REQUIRE(int64_t(tm) * tn < (int64_t(1) << 31), ABH_ERR_INVALID_ARG, "dgemm: too many tiles");
   if (k == 0) {
     // C = beta C: the product is empty
     ABH_REQUIRE(beta == 1.0, ABH_ERR_INVALID_ARG, "dgemm: k == 0 needs beta == 1");
     return;
   }
-  dim3 grid(unsigned(tm * tn), unsigned(batch));
-  const int lo = lower_only ? 1 : 0;
+  const int tiles = tm * tn, xcds = batch >= 64 ? 8 : 1;
+  const int64_t blocks = int64_t(tiles) * (ceil_div(batch, xcds) * xcds);
+  ABH_REQUIRE(blocks < (int64_t(1) << 31), ABH_ERR_INVALID_ARG, "dgemm: too many tiles");
+  const dim3 grid{unsigned(blocks)};
   if (!ta && !tb)
     k_dgemm<false, false><<<grid, 256, 0, st>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                                                 ldc, sC, tm, lo);
+                                                 ldc, sC, tm, tiles, batch, xcds, from_c);
   else if (!ta && tb)
     k_dgemm<false, true><<<grid, 256, 0, st>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                                                ldc, sC, tm, lo);
+                                                ldc, sC, tm, tiles, batch, xcds, from_c);
   else if (ta && !tb)
     k_dgemm<true, false><<<grid, 256, 0, st>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                                                ldc, sC, tm, lo);
+                                                ldc, sC, tm, tiles, batch, xcds, from_c);
   else
     k_dgemm<true, true><<<grid, 256, 0, st>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                                               ldc, sC, tm, lo);
+                                               ldc, sC, tm, tiles, batch, xcds, from_c);
   check_launch();
 }
 

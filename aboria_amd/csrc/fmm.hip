@@ -1789,7 +1789,7 @@ template <int N> void compress_impl(abh_fmm *f, double eps) {
     if (ox >= -1 && ox <= 1 && oy >= -1 && oy <= 1 && oz >= -1 && oz <= 1) continue;
     abh::dgemm_strided_batched(s, true, false, NC, NC, NC, 1.0, M + int64_t(o) * NC * NC, NC,
                                per_lev, M + int64_t(o) * NC * NC, NC, per_lev, 1.0,
-                               gram.as<double>(), NC, int64_t(NC) * NC, nlev, false);
+                               gram.as<double>(), NC, int64_t(NC) * NC, nlev);
   }
   std::vector<double> gh(size_t(nlev) * NC * NC);
   ABH_HIP(hipMemcpyAsync(gh.data(), gram.p, gh.size() * 8, hipMemcpyDeviceToHost, s));
@@ -1856,10 +1856,10 @@ template <int N> void compress_impl(abh_fmm *f, double eps) {
     // T_o = K_o U (K_o = X_o^T), C_o = U^T T_o, both column-major
     abh::dgemm_strided_batched(s, true, false, NC, KP, NC, 1.0, M + li * per_lev, NC,
                                int64_t(NC) * NC, Ul, NC, 0, 0.0, T.as<double>(), NC,
-                               int64_t(NC) * KP, kOffsets, false);
+                               int64_t(NC) * KP, kOffsets);
     abh::dgemm_strided_batched(s, true, false, KP, KP, NC, 1.0, Ul, NC, 0, T.as<double>(), NC,
                                int64_t(NC) * KP, 0.0, Cm.as<double>(), KP, int64_t(KP) * KP,
-                               kOffsets, false);
+                               kOffsets);
     k_pack_frag<<<8192, 256, 0, s>>>(Cm.as<double>(), kOffsets, KP, KP, int64_t(KP) * KP, 1, KP,
                                      f->Cf.as<double>() + int64_t(li) * kOffsets *
                                                               frag_size(KP, KP));

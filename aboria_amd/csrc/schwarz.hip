@@ -6,14 +6,24 @@
 //
 // Factorise (device): domains are sorted by size and processed in groups of
 // equal padded size n (a multiple of 64).  Per group every local matrix
-// A_g = K + shift I (identity in the padding) is assembled in HBM,
-// factorised by a right-looking blocked Cholesky (64-wide panels: the
-// diagonal block in LDS, panel and trailing updates as strided-batched
-// FP64 MFMA GEMMs, dgemm.hip), and the interior columns of A_g^-1 (= the
-// interior rows, A_g is symmetric) are obtained by a blocked forward and
-// backward substitution on the unit columns.  They stay resident: R_g is
-// n x ni column-major, so row a of the local inverse is the contiguous
-// column a.
+// A_g = K + shift I (identity in the padding) is assembled in HBM with the
+// domain's list reversed: entry j at matrix index n - 1 - j, so the padding
+// comes first and the interior last (the signed form below keeps the list's
+// order).  It is factorised by a left-looking
+// blocked Cholesky (64-wide panels: a block column takes all earlier ones in
+// one strided-batched FP64 MFMA GEMM, dgemm.hip, the diagonal block is
+// factorised and inverted by one wavefront, the panel multiplied by that
+// inverse in place), and the interior columns of A_g^-1 (= the interior
+// rows, A_g is symmetric) are obtained by a blocked forward and backward
+// substitution on the last unit columns: since the interior comes last, the
+// forward one touches the last block rows only.  They stay resident: R_g is
+// n x ni column-major, so row a of the local inverse is the contiguous column
+// ni - 1 - a, backwards (signed: column a).
+// 400,056 points, 6,256 domains of 576 (the whole set-up and solve, 113 ms
+// before): diagonal blocks 36.9 -> 6.5 ms (256 threads and three barriers
+// per column before), products 48.6 -> 22.9 ms, copies 6.2 -> 0 ms; with
+// right-looking updates every trailing tile was read and written once per
+// panel, which HBM bounded.
 //
 // For the dense batch (every problem an independent particle set) the
 // domains come from a per-problem bucket grid instead of a cell list, the
@@ -28,6 +38,7 @@
 #include <cmath>
 #include <memory>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "cells.hpp"
@@ -46,15 +57,17 @@ constexpr int kApplyLds = 7936;    // max domain size staged in LDS by apply (62
 
 struct DomDev {
   int64_t idx_off;  // first entry in the index array
-  int64_t r_off;    // first double of the domain's inverse rows
+  int64_t r_off;    // interior row 0's column of R (row a: a columns on, reversed: before)
   int32_t m;        // interior + buffer
   int32_t ni;       // interior
   int32_t ld;       // padded size n of its group (leading dimension of R)
+  int32_t rev;      // the list is reversed in the matrix (see k_assemble)
   int32_t failed;   // factorisation broke down: apply leaves its rows at b
 };
 
-// A[g] (n x n, column-major) = K + shift I over the domain's particles,
-// identity on the padding.
+// A[g] (n x n, column-major) = K + shift I over the domain's particles, entry
+// j of the list at index j, reversed: n - 1 - j; identity on the padding; only
+// the tiles on and below the diagonal, the others are never read.
 template <int D>
 __global__ __launch_bounds__(256) void k_assemble(const DomDev *__restrict__ doms,
                                                   const int32_t *__restrict__ idx,
@@ -66,12 +79,13 @@ __global__ __launch_bounds__(256) void k_assemble(const DomDev *__restrict__ dom
   const DomDev dm = doms[g];
   const int i0 = blockIdx.x * 64, j0 = blockIdx.y * 64;
   const int t = threadIdx.x;
+  if (j0 > i0) return;
   if (t < 64) {
-    const int i = i0 + t;
+    const int i = dm.rev ? n - 1 - i0 - t : i0 + t;
 #pragma unroll
     for (int d = 0; d < D; ++d) pi[t][d] = i < dm.m ? pos[int64_t(idx[dm.idx_off + i]) * D + d] : 0.0;
   } else if (t < 128) {
-    const int j = j0 + t - 64;
+    const int j = dm.rev ? n - 1 - j0 - (t - 64) : j0 + t - 64;
 #pragma unroll
     for (int d = 0; d < D; ++d)
       pj[t - 64][d] = j < dm.m ? pos[int64_t(idx[dm.idx_off + j]) * D + d] : 0.0;
@@ -83,7 +97,7 @@ __global__ __launch_bounds__(256) void k_assemble(const DomDev *__restrict__ dom
   for (int lj = t >> 6; lj < 64; lj += 4) {
     const int j = j0 + lj;
     double v;
-    if (i < dm.m && j < dm.m) {
+    if ((dm.rev ? n - 1 - min(i, j) : max(i, j)) < dm.m) {
       double s = 0.0;
 #pragma unroll
       for (int d = 0; d < D; ++d) {
@@ -99,81 +113,97 @@ __global__ __launch_bounds__(256) void k_assemble(const DomDev *__restrict__ dom
   }
 }
 
+// One step of a 64 x 64 elimination on rows held in registers, N of them
+// left: v[k - 1] = v[k] - f c[k], so that v[0] is always the current column.
+template <int N>
+__device__ __forceinline__ void eliminate(double (&v)[kNb], double f, const double *c) {
+#pragma unroll
+  for (int k = 1; k < N; ++k) v[k - 1] = fma(-f, c[k], v[k]);
+}
+
 // Cholesky of the 64 x 64 diagonal block at (o, o) of every matrix of the
-// group, in LDS; writes L back and L^-1 to dinv (64 x 64 column-major).
+// group; writes L back and L^-1 to dinv (64 x 64 column-major).
 // Signed mode (symmetric matrices with negative eigenvalues, such as
 // multiquadric ones): A = L S L^T with S = diag(+-1); the signs go to
 // sg[g * sg_stride + o + j] and S L^-1 (the panel's right factor) to dinvs.
-__global__ __launch_bounds__(256) void k_potrf_diag(double *__restrict__ A, int n, int o,
-                                                    double *__restrict__ dinv,
-                                                    int64_t dinv_stride,
-                                                    uint8_t *__restrict__ failed, int signed_mode,
-                                                    double *__restrict__ sg, int64_t sg_stride,
-                                                    double *__restrict__ dinvs) {
-  __shared__ double L[kNb][kNb + 1];
-  __shared__ double X[kNb][kNb + 1];
+//
+// Bound by the latency of the pivot chain (square root, division, the
+// column through LDS), so one wavefront does a whole block without barriers:
+// lane r holds row r in registers, a step takes the pivot from lane j, puts
+// column j in LDS and subtracts it from the columns right of it, which every
+// lane reads by broadcast.  The inverse is the same elimination on the unit
+// columns, one per lane.  231 blocks: 152 us with 256 threads, the block in
+// LDS and three barriers per step; now 78 us for 1,000 blocks.
+__global__ __launch_bounds__(64) void k_potrf_diag(double *__restrict__ A, int n, int o,
+                                                   double *__restrict__ dinv,
+                                                   int64_t dinv_stride,
+                                                   uint8_t *__restrict__ failed, int signed_mode,
+                                                   double *__restrict__ sg, int64_t sg_stride,
+                                                   double *__restrict__ dinvs) {
+  constexpr int kLd = kNb + 2;
+  // column j of L in L[j]; a step reads up to 63 words past its column (their
+  // values reach no entry that is kept)
+  __shared__ double L[kNb + 1][kLd];
   __shared__ double S[kNb];
-  __shared__ int bad;
   const int g = blockIdx.x;
-  const int t = threadIdx.x;
+  const int r = threadIdx.x;
   double *Ag = A + int64_t(g) * n * n + int64_t(o) * n + o;
-  for (int e = t; e < kNb * kNb; e += 256) {
-    const int r = e & 63, c = e >> 6;
-    L[r][c] = Ag[int64_t(c) * n + r];
-  }
-  if (t == 0) bad = 0;
-  __syncthreads();
-  for (int j = 0; j < kNb; ++j) {
-    if (t == 0) {
-      double d = L[j][j];
-      double sj = 1.0;
-      if (signed_mode) {
-        if (!(d != 0.0) || !isfinite(d)) {
-          bad = 1;
-          d = 1.0;
-        }
-        sj = d > 0.0 ? 1.0 : -1.0;
-        d = fabs(d);
-      } else if (!(d > 0.0)) {
-        bad = 1;
+  double v[kNb];
+#pragma unroll
+  for (int c = 0; c < kNb; ++c) v[c] = Ag[int64_t(c) * n + r];
+  bool bad = false;
+  auto factor = [&](auto left, int j) {
+    const uint64_t pv = uint64_t(__double_as_longlong(v[0]));
+    const uint32_t plo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(pv)), j));
+    const uint32_t phi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(pv >> 32)), j));
+    double d = __longlong_as_double((long long)((uint64_t(phi) << 32) | plo));
+    double sj = 1.0;
+    if (signed_mode) {
+      if (!(d != 0.0) || !isfinite(d)) {
+        bad = true;
         d = 1.0;
       }
-      S[j] = sj;
-      L[j][j] = sqrt(d);
+      sj = d > 0.0 ? 1.0 : -1.0;
+      d = fabs(d);
+    } else if (!(d > 0.0)) {
+      bad = true;
+      d = 1.0;
     }
+    const double root = sqrt(d);
+    const double l = r > j ? v[0] / (root * sj) : (r == j ? root : 0.0);
+    L[j][r] = l;
+    if (r == 0) S[j] = sj;
+    __syncthreads();  // one wavefront: the column is in LDS
+    eliminate<decltype(left)::value>(v, l * sj, &L[j][j]);
+  };
+  // fewer and fewer columns are left
+  for (int j = 0; j < 16; ++j) factor(std::integral_constant<int, 64>{}, j);
+  for (int j = 16; j < 32; ++j) factor(std::integral_constant<int, 48>{}, j);
+  for (int j = 32; j < 48; ++j) factor(std::integral_constant<int, 32>{}, j);
+  for (int j = 48; j < 64; ++j) factor(std::integral_constant<int, 16>{}, j);
+  for (int c = 0; c < kNb; ++c) Ag[int64_t(c) * n + r] = L[c][r];
+  // X = L^-1: lane c eliminates column c of the identity; row j of X replaces
+  // column j of L, which no later step reads
+#pragma unroll
+  for (int k = 0; k < kNb; ++k) v[k] = k == r ? 1.0 : 0.0;
+  auto invert = [&](auto left, int j) {
+    const double x = v[0] / L[j][j];
+    eliminate<decltype(left)::value>(v, x, &L[j][j]);
     __syncthreads();
-    const double djj = L[j][j] * S[j];
-    if (t > j && t < kNb) L[t][j] = L[t][j] / djj;
-    __syncthreads();
-    // trailing update of the lower triangle, columns j+1..63
-    const double sj = S[j];
-    for (int e = t; e < kNb * kNb; e += 256) {
-      const int r = e & 63, c = e >> 6;
-      if (c > j && r >= c) L[r][c] = L[r][c] - (L[r][j] * L[c][j]) * sj;
-    }
-    __syncthreads();
-  }
-  // X = L^-1, one column per thread (forward substitution)
-  if (t < kNb) {
-    const int c = t;
-    for (int r = 0; r < c; ++r) X[r][c] = 0.0;
-    X[c][c] = 1.0 / L[c][c];
-    for (int r = c + 1; r < kNb; ++r) {
-      double s = 0.0;
-      for (int q = c; q < r; ++q) s = s + L[r][q] * X[q][c];
-      X[r][c] = -s / L[r][r];
-    }
-  }
+    L[j][r] = x;
+  };
+  for (int j = 0; j < 16; ++j) invert(std::integral_constant<int, 64>{}, j);
+  for (int j = 16; j < 32; ++j) invert(std::integral_constant<int, 48>{}, j);
+  for (int j = 32; j < 48; ++j) invert(std::integral_constant<int, 32>{}, j);
+  for (int j = 48; j < 64; ++j) invert(std::integral_constant<int, 16>{}, j);
   __syncthreads();
   double *Dg = dinv + int64_t(g) * dinv_stride;
-  for (int e = t; e < kNb * kNb; e += 256) {
-    const int r = e & 63, c = e >> 6;
-    Ag[int64_t(c) * n + r] = r >= c ? L[r][c] : 0.0;
-    Dg[c * kNb + r] = X[r][c];
-    if (signed_mode) dinvs[int64_t(g) * dinv_stride + c * kNb + r] = X[r][c] * S[r];
+  for (int c = 0; c < kNb; ++c) {
+    Dg[c * kNb + r] = L[r][c];
+    if (signed_mode) dinvs[int64_t(g) * dinv_stride + c * kNb + r] = L[r][c] * S[r];
   }
-  if (signed_mode && t < kNb) sg[int64_t(g) * sg_stride + o + t] = S[t];
-  if (t == 0 && bad) failed[g] = 1;
+  if (signed_mode) sg[int64_t(g) * sg_stride + o + r] = S[r];
+  if (r == 0 && bad) failed[g] = 1;
 }
 
 // dst[g] (rows x cols, ld ldd) = src[g] (ld lds) times cs[g * cs_stride + c]
@@ -200,13 +230,13 @@ __global__ void k_scale_rows(double *__restrict__ Y, int64_t stride, int n, int 
   Y[g * stride + e] = Y[g * stride + e] * sg[g * sg_stride + int(e % n)];
 }
 
-// Y[g] (n x ni) = the first ni columns of the identity
-__global__ void k_unit_cols(double *__restrict__ Y, int64_t stride, int n, int ni) {
+// Y[g] (n x ni) = ni columns of the identity, from column c0 on
+__global__ void k_unit_cols(double *__restrict__ Y, int64_t stride, int n, int ni, int c0) {
   const int g = blockIdx.y;
   const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (e >= int64_t(n) * ni) return;
   const int r = int(e % n), c = int(e / n);
-  Y[g * stride + e] = r == c ? 1.0 : 0.0;
+  Y[g * stride + e] = r == c0 + c ? 1.0 : 0.0;
 }
 
 struct ApplyChunk {
@@ -232,13 +262,17 @@ __global__ __launch_bounds__(256) void k_ras_apply(const ApplyChunk *__restrict_
   }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int rows = min(kApplyRows, dm.ni - ch.row0);
+  const int dir = dm.rev ? -1 : 1;
   for (int a = wave; a < rows; a += 4) {
-    const double *Ra = R + dm.r_off + int64_t(ch.row0 + a) * dm.ld;
+    // entry j of the list is row j of the column, reversed: ld - 1 - j
+    const int64_t row = ch.row0 + a;
+    const double *Ra = R + dm.r_off + (dm.rev ? dm.ld - 1 - row * dm.ld : row * dm.ld);
     double s = 0.0;
     int j = lane;
     // four row loads in flight per step, summed in the same order
     for (; j + 192 < dm.m; j += 256) {
-      const double r0 = Ra[j], r1 = Ra[j + 64], r2 = Ra[j + 128], r3 = Ra[j + 192];
+      const double r0 = Ra[j * dir], r1 = Ra[(j + 64) * dir], r2 = Ra[(j + 128) * dir],
+                   r3 = Ra[(j + 192) * dir];
       const double b0 = LDS ? bl[j] : b[id[j]];
       const double b1 = LDS ? bl[j + 64] : b[id[j + 64]];
       const double b2 = LDS ? bl[j + 128] : b[id[j + 128]];
@@ -248,7 +282,7 @@ __global__ __launch_bounds__(256) void k_ras_apply(const ApplyChunk *__restrict_
       s = s + r2 * b2;
       s = s + r3 * b3;
     }
-    for (; j < dm.m; j += 64) s = s + Ra[j] * (LDS ? bl[j] : b[id[j]]);
+    for (; j < dm.m; j += 64) s = s + Ra[j * dir] * (LDS ? bl[j] : b[id[j]]);
     s = abh::wave_sum(s);
     if (lane == 0) x[id[ch.row0 + a]] = s;
   }
@@ -334,6 +368,43 @@ void analyse_batch_into(abh_schwarz *s, int D, const std::vector<int64_t> &boff,
   take(s, dm);
 }
 
+void drop_factor_buffers(abh_context *ctx) {
+  for (DevBuf *b : {&ctx->factor_a, &ctx->factor_d, &ctx->factor_ds, &ctx->factor_w,
+                    &ctx->factor_sg, &ctx->factor_spare})
+    b->release();
+}
+
+constexpr size_t kSpareMax = size_t(4) << 30;
+
+// R of at least `want` bytes: its own, the context's spare one if that is not
+// more than twice as large, or a new allocation.
+void take_inverse(abh_schwarz *s, size_t want) {
+  abh_context *ctx = s->ctx;
+  DevBuf &spare = ctx->factor_spare;
+  if (s->R.bytes >= want) return;
+  if (spare.bytes >= want && spare.bytes / 2 <= want) {
+    s->R.swap(spare);
+    spare.release();
+    return;
+  }
+  try {
+    s->R.ensure_exact(want);
+  } catch (const abh::Error &e) {
+    if (e.status != ABH_ERR_OUT_OF_MEMORY) throw;
+    (void)hipGetLastError();
+    ABH_HIP(hipStreamSynchronize(ctx->stream));
+    drop_factor_buffers(ctx);
+    s->R.ensure_exact(want);
+  }
+}
+
+// gives R back to the context (nothing on its stream uses it any more)
+void give_inverse(abh_schwarz *s) {
+  DevBuf &spare = s->ctx->factor_spare;
+  if (s->coarse) give_inverse(s->coarse);
+  if (s->R.bytes <= kSpareMax && s->R.bytes > spare.bytes) s->R.swap(spare);
+}
+
 // sgn: local matrices may be indefinite; factorise A = L S L^T (S = +-1)
 // instead of requiring positive pivots.
 void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2, double shift,
@@ -342,6 +413,10 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
   hipStream_t st = ctx->stream;
   const int nd = int(s->nint.size());
   if (nd == 0) return;
+  // Signed factorisations run without pivoting on matrices with eigenvalues
+  // of both signs and keep the list's order, in which the interior comes first
+  // (reversed they lost accuracy on multiquadric domains).
+  const int rev = sgn ? 0 : 1;
   // domains by padded size, then interior count, largest first; a group
   // shares the padded size and the interior count of its first member
   std::vector<int> order(nd);
@@ -364,6 +439,7 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
   // inverse rows: n_pad x ni_pad per domain
   struct Group {
     int first, count, n, ni;
+    int64_t r_off;  // R of the first member
   };
   std::vector<Group> groups;
   int64_t r_total = 0;
@@ -371,13 +447,21 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
     int i = 0;
     while (i < nd) {
       const int n = npad(order[i]);
-      // working set per member: A (n^2) + panel copy (64 n) + dinv (n 64)
-      // (+ S L^-1 and the signs in signed mode)
-      const double per = double(n) * n * 8.0 + double(n) * kNb * (sgn ? 24.0 : 16.0) +
+      // working set per member: A (n^2) + dinv (64 n) (+ S L^-1, the scaled
+      // block row and the signs in signed mode)
+      const double per = double(n) * n * 8.0 + double(n) * kNb * (sgn ? 24.0 : 8.0) +
                          (sgn ? double(n) * 8.0 : 0.0);
-      const double budget = std::min(8.0e9, 0.35 * double(free_b));
-      int gmax = int(std::max(1.0, std::min(256.0, budget / per)));
-      Group gr{i, 0, n, 0};
+      // Large groups fill the chip with diagonal blocks and panels (at most a
+      // wavefront per SIMD): 6,256 domains of 576 take 69 ms in groups of
+      // 256, 57 in groups of 512, 53 in groups of 1,024 (2.7 GB).  A size's
+      // domains are spread evenly over its groups.
+      const double budget =
+          std::min(2.4e9, 0.35 * (double(free_b) + double(ctx->factor_a.bytes)));
+      int gmax = int(std::max(1.0, std::min(4.0 * ctx->n_cu, budget / per)));
+      int same = 0;
+      while (i + same < nd && npad(order[i + same]) == n) ++same;
+      gmax = int(abh::ceil_div(same, abh::ceil_div(same, gmax)));
+      Group gr{i, 0, n, 0, r_total};
       gr.ni = s->nint[order[i]];
       while (i < nd && gr.count < gmax && npad(order[i]) == n) {
         ++gr.count;
@@ -386,7 +470,8 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
       for (int q = 0; q < gr.count; ++q) {
         const int d = order[gr.first + q];
         dd[d].idx_off = s->off[d];
-        dd[d].r_off = r_total + int64_t(q) * n * gr.ni;
+        dd[d].r_off = r_total + int64_t(q) * n * gr.ni + (rev ? int64_t(gr.ni - 1) * n : 0);
+        dd[d].rev = rev;
         dd[d].m = msize(d);
         dd[d].ni = s->nint[d];
         dd[d].ld = n;
@@ -397,7 +482,7 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
     }
   }
   s->factor_bytes = size_t(r_total) * 8;
-  s->R.ensure(s->factor_bytes + 64);
+  take_inverse(s, s->factor_bytes + 64);
   s->d_idx.ensure(s->idx.size() * 4 + 64);
   ABH_HIP(hipMemcpyAsync(s->d_idx.p, s->idx.data(), s->idx.size() * 4, hipMemcpyHostToDevice, st));
   // domain table in group order (the group's members are contiguous)
@@ -418,20 +503,21 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
                          hipMemcpyHostToDevice, st));
   using abh::dgemm_strided_batched;
 
-  int gmax = 0, nmax = 0, nimax = 0;
+  size_t a_size = 0, d_size = 0, s_size = 0;
   for (const Group &gr : groups) {
-    gmax = std::max(gmax, gr.count);
-    nmax = std::max(nmax, gr.n);
-    nimax = std::max(nimax, gr.ni);
+    a_size = std::max(a_size, size_t(gr.count) * gr.n * gr.n);
+    d_size = std::max(d_size, size_t(gr.count) * gr.n * kNb);
+    s_size = std::max(s_size, size_t(gr.count) * gr.n);
   }
-  DevBuf A, W, Tm, Dinv, DinvS, Sg, fail;
-  A.ensure(size_t(gmax) * nmax * nmax * 8);
-  W.ensure(size_t(gmax) * nmax * kNb * 8);
-  Tm.ensure(size_t(gmax) * kNb * nimax * 8);
-  Dinv.ensure(size_t(gmax) * (nmax / kNb) * kNb * kNb * 8);
+  DevBuf &A = ctx->factor_a, &W = ctx->factor_w, &Dinv = ctx->factor_d;
+  DevBuf &DinvS = ctx->factor_ds, &Sg = ctx->factor_sg;
+  DevBuf fail;
+  A.ensure(a_size * 8);
+  Dinv.ensure(d_size * 8);
   if (sgn) {
-    DinvS.ensure(size_t(gmax) * (nmax / kNb) * kNb * kNb * 8);
-    Sg.ensure(size_t(gmax) * nmax * 8);
+    W.ensure(d_size * 8);
+    DinvS.ensure(d_size * 8);
+    Sg.ensure(s_size * 8);
   }
   fail.ensure(size_t(nd) + 64);
   ABH_HIP(hipMemsetAsync(fail.p, 0, size_t(nd), st));
@@ -442,14 +528,13 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
     const int64_t sA = int64_t(n) * n;
     const int64_t sD = int64_t(K) * kNb * kNb;
     const int64_t sW = int64_t(n) * kNb;
-    const int64_t sT = int64_t(kNb) * ni;
     const int64_t sY = int64_t(n) * ni;
-    double *Ap = A.as<double>(), *Wp = W.as<double>(), *Tp = Tm.as<double>();
+    double *Ap = A.as<double>(), *Wp = W.as<double>();
     double *Dp = Dinv.as<double>();
     // signed mode: panel right factor S L^-1, signs per member (stride n)
     double *DSp = sgn ? DinvS.as<double>() : Dp;
     double *Sp = sgn ? Sg.as<double>() : nullptr;
-    double *Y = s->R.as<double>() + dd[order[gr.first]].r_off;
+    double *Y = s->R.as<double>() + gr.r_off;
     uint8_t *fl = fail.as<uint8_t>() + gr.first;
     const DomDev *gd = d_dg.as<DomDev>() + gr.first;
     {
@@ -459,55 +544,50 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
       else k_assemble<3><<<grid, 256, 0, st>>>(gd, didx, pos, k, r2, shift, n, Ap);
       abh::check_launch();
     }
-    // blocked Cholesky, lower (signed: A = L S L^T)
+    // blocked Cholesky, lower (signed: A = L S L^T), one block column after
+    // the other
     for (int kb = 0; kb < K; ++kb) {
       const int o = kb * kNb;
-      k_potrf_diag<<<G, 256, 0, st>>>(Ap, n, o, Dp + int64_t(kb) * kNb * kNb, sD, fl,
-                                      sgn ? 1 : 0, Sp, n, DSp + int64_t(kb) * kNb * kNb);
-      abh::check_launch();
       const int r = n - o - kNb;
-      if (r == 0) break;
-      double *P = Ap + o + kNb + int64_t(o) * n;
-      // panel P = A[o+64:, o:o+64] L_kk^-T (S_k)
-      {
-        dim3 grid(unsigned(abh::ceil_div(int64_t(r) * kNb, 256)), G);
-        k_copy_block<<<grid, 256, 0, st>>>(P, sA, n, Wp, sW, n, r, kNb);
-        abh::check_launch();
+      double *Ck = Ap + o + int64_t(o) * n;  // A[o:, o:o+64]
+      if (kb > 0) {
+        // A[o:, o:o+64] -= A[o:, :o] (S) A[o:o+64, :o]^T
+        const double *Bk = Ap + o;
+        if (sgn) {
+          dim3 grid(unsigned(abh::ceil_div(int64_t(kNb) * o, 256)), G);
+          k_copy_block<<<grid, 256, 0, st>>>(Ap + o, sA, n, Wp, sW, kNb, kNb, o, Sp, n);
+          abh::check_launch();
+          Bk = Wp;
+        }
+        dgemm_strided_batched(st, false, true, n - o, kNb, o, -1.0, Ap + o, n, sA, Bk,
+                              sgn ? kNb : n, sgn ? sW : sA, 1.0, Ck, n, sA, G, true);
       }
-      dgemm_strided_batched(st, false, true, r, kNb, kNb, 1.0, Wp, n, sW,
-                            DSp + int64_t(kb) * kNb * kNb, kNb, sD, 0.0, P, n, sA, G);
-      // trailing A[o+64:, o+64:] -= P (S_k) P^T, lower triangle (the upper
-      // one is never read again)
-      const double *Pl = P;
-      if (sgn) {
-        dim3 grid(unsigned(abh::ceil_div(int64_t(r) * kNb, 256)), G);
-        k_copy_block<<<grid, 256, 0, st>>>(P, sA, n, Wp, sW, n, r, kNb, Sp + o, n);
-        abh::check_launch();
-        Pl = Wp;
-      }
-      dgemm_strided_batched(st, false, true, r, r, kNb, -1.0, Pl, n, sgn ? sW : sA, P, n, sA,
-                            1.0, Ap + o + kNb + int64_t(o + kNb) * n, n, sA, G, true);
+      k_potrf_diag<<<G, 64, 0, st>>>(Ap, n, o, Dp + int64_t(kb) * kNb * kNb, sD, fl, sgn ? 1 : 0,
+                                     Sp, n, DSp + int64_t(kb) * kNb * kNb);
+      abh::check_launch();
+      // panel A[o+64:, o:o+64] L_kk^-T (S_k), in place
+      if (r > 0)
+        dgemm_strided_batched(st, false, true, r, kNb, kNb, 1.0, Ck + kNb, n, sA,
+                              DSp + int64_t(kb) * kNb * kNb, kNb, sD, 0.0, Ck + kNb, n, sA, G);
     }
-    // Y = L^-1 E (E = first ni unit columns); Y is lower trapezoidal
+    // Y = L^-1 E (E = the interior's unit columns, the last ni or the first):
+    // rows before the block of the first unit stay zero, and so do columns of
+    // units past the block row at hand
     {
       dim3 grid(unsigned(abh::ceil_div(int64_t(n) * ni, 256)), G);
-      k_unit_cols<<<grid, 256, 0, st>>>(Y, sY, n, ni);
+      k_unit_cols<<<grid, 256, 0, st>>>(Y, sY, n, ni, rev ? n - ni : 0);
       abh::check_launch();
     }
-    for (int kb = 0; kb < K; ++kb) {
+    for (int kb = rev ? (n - ni) / kNb : 0; kb < K; ++kb) {
       const int o = kb * kNb;
-      const int nc = std::min(ni, o + kNb);  // columns >= o+64 are still zero
-      {
-        dim3 grid(unsigned(abh::ceil_div(int64_t(kNb) * nc, 256)), G);
-        k_copy_block<<<grid, 256, 0, st>>>(Y + o, sY, n, Tp, sT, kNb, kNb, nc);
-        abh::check_launch();
-      }
+      const int nc = rev ? ni : std::min(ni, o + kNb);
+      // in place, like every product with a diagonal block's inverse
       dgemm_strided_batched(st, false, false, kNb, nc, kNb, 1.0, Dp + int64_t(kb) * kNb * kNb,
-                            kNb, sD, Tp, kNb, sT, 0.0, Y + o, n, sY, G);
+                            kNb, sD, Y + o, n, sY, 0.0, Y + o, n, sY, G);
       const int r = n - o - kNb;
       if (r > 0)
         dgemm_strided_batched(st, false, false, r, nc, kNb, -1.0, Ap + o + kNb + int64_t(o) * n,
-                              n, sA, Y + o, n, sY, 1.0, Y + o + kNb, n, sY, G);
+                              n, sA, Y + o, n, sY, 1.0, Y + o + kNb, n, sY, G, true);
     }
     // Z = L^-T (S) Y, in place
     if (sgn) {
@@ -520,14 +600,9 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
       const int r = n - o - kNb;
       if (r > 0)
         dgemm_strided_batched(st, true, false, kNb, ni, r, -1.0, Ap + o + kNb + int64_t(o) * n,
-                              n, sA, Y + o + kNb, n, sY, 1.0, Y + o, n, sY, G);
-      {
-        dim3 grid(unsigned(abh::ceil_div(int64_t(kNb) * ni, 256)), G);
-        k_copy_block<<<grid, 256, 0, st>>>(Y + o, sY, n, Tp, sT, kNb, kNb, ni);
-        abh::check_launch();
-      }
+                              n, sA, Y + o + kNb, n, sY, 1.0, Y + o, n, sY, G, true);
       dgemm_strided_batched(st, true, false, kNb, ni, kNb, 1.0, Dp + int64_t(kb) * kNb * kNb,
-                            kNb, sD, Tp, kNb, sT, 0.0, Y + o, n, sY, G);
+                            kNb, sD, Y + o, n, sY, 0.0, Y + o, n, sY, G);
     }
   }
   ABH_HIP(hipMemcpyAsync(fh.data(), fail.p, size_t(nd), hipMemcpyDeviceToHost, st));
@@ -689,6 +764,7 @@ abh_status abh_schwarz_destroy(abh_schwarz *s) {
   abh_context *ctx = s->ctx;
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
+  give_inverse(s);
   delete s;
   abh::ctx_release(ctx);
   return ABH_OK;
