@@ -27,6 +27,16 @@ constexpr int kRows = 256;
 // problem), so every source staged in LDS serves RPT rows.
 constexpr int kVariants = 3;
 constexpr int kRptOf[kVariants] = {1, 2, 4};
+// The symmetric form (k_dense_sym) has tiles of 256 x kSymRpt rows and is used
+// where it saves at least a quarter of the kernel values (with most problems
+// within one tile there is nothing to share), has at least kSymTiles tiles per
+// CU (300 problems of 200 to 3,000 points, 500 tiles: 0.58 ms, 0.36 one-sided
+// with one row per thread; 512 of 1,000 to 64,000, 7,700 tiles: 73.8 and
+// 118.7 ms) and its partial sums fit 1.25 GB (that batch needs 1.0).  The rule
+// looks at the sizes only, so a batch gives the same bits in every run.
+constexpr int kSymRpt = 4, kSymVariant = 2;
+constexpr int kSymTiles = 8;
+constexpr int64_t kSymPart = int64_t(5) << 25;
 
 // MQ: the multiquadric sqrt(|dx|^2 + c^2) with fused multiply-adds (the
 // batched RBF systems' kernel), instead of the generic profile.
@@ -122,6 +132,169 @@ __global__ __launch_bounds__(kRows) void k_dense(const int2 *__restrict__ tiles,
     if (!act[q]) continue;
     const int64_t i = int64_t(tiles[t].y) + threadIdx.x + q * kRows;
     const double v = FP32 ? double(a32[q]) + double(c32[q]) : acc[q];
+    double *yp = &y[base + i];
+    *yp = (overwrite ? 0.0 : *yp) + alpha * v;
+  }
+}
+
+// The same product with every kernel value used twice: the operators of a
+// batch are symmetric (one point set, no per-particle weights).  A tile's 1,024
+// rows meet the columns of their own tile as above and the columns past it
+// once for both sides: f x_j joins row i's sum and f x_i column j's.  A lane
+// holds 4 rows and walks 64 columns starting at its own number, so that at
+// any step the lanes of a wave hold different columns and add to different
+// column sums in LDS.  A tile writes its rows' sums and its column sums to
+// `part` (poff: where its row 0 starts there; entry c - row0 for column c) and
+// k_dense_sym_sum adds them up in tile order: deterministic.  The FP32 form
+// adds its FP32 terms in FP64.
+// Bound by the vector instructions of the profile (multiquadric: 14 per pair
+// and row for both sides, against 2 x 13).  512 problems of 1,000 to 64,000
+// points: 118.7 -> 73.8 ms.  Shorter sums: against sums in double-double that
+// batch is 4.1e-15 off, one-sided 6.8e-15 (as is a plain sum by rows, which
+// therefore agrees with the one-sided form to 1.2e-15).
+template <int D, bool FP32, bool MQ>
+__device__ __forceinline__ double sym_phi(const KernelDesc &k, const double *a, const double *b,
+                                          double xj, double &row) {
+  // returns the profile's value as the column side uses it and adds f xj
+  if (FP32) {
+    float s = MQ ? float(k.param2) : 0.0f;
+#pragma unroll
+    for (int d = D - 1; d >= 0; --d) {
+      const float dx = float(a[d] - b[d]);
+      s = fmaf(dx, dx, s);
+    }
+    const float f = MQ ? __builtin_amdgcn_sqrtf(s) : abh::phi32(k, s);
+    row += double(f * float(xj));
+    return double(f);
+  }
+  double s = MQ ? k.param2 : 0.0;
+#pragma unroll
+  for (int d = D - 1; d >= 0; --d) {
+    const double dx = a[d] - b[d];
+    s = MQ ? fma(dx, dx, s) : s + dx * dx;
+  }
+  const double f = MQ ? abh::sqrt_pos(s) : abh::phi64(k, s);  // MQ: s >= c^2 >= 1e-280
+  row = fma(f, xj, row);
+  return f;
+}
+
+template <int D, bool FP32, bool MQ>
+__global__ __launch_bounds__(kRows) void k_dense_sym(const int2 *__restrict__ tiles,
+                                                     const int64_t *__restrict__ poff,
+                                                     const int64_t *__restrict__ off,
+                                                     const double *__restrict__ pos,
+                                                     const double *__restrict__ x,
+                                                     double *__restrict__ part,
+                                                     const uint8_t *__restrict__ active,
+                                                     KernelDesc k) {
+  constexpr int RPT = kSymRpt;
+  __shared__ double sp[D][kRows];
+  __shared__ double sx[kRows];
+  __shared__ double csum[kRows / 64][kRows];
+  const int t = blockIdx.x;
+  const int p = tiles[t].x;
+  if (active && !active[p]) return;
+  const int64_t base = off[p];
+  const int64_t n = off[p + 1] - base, row0 = tiles[t].y;
+  double *out = part + poff[t];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double xi[RPT][D], xr[RPT], acc[RPT];
+#pragma unroll
+  for (int q = 0; q < RPT; ++q) {
+    const int64_t i = row0 + threadIdx.x + q * kRows;
+    const bool act = i < n;
+#pragma unroll
+    for (int d = 0; d < D; ++d) xi[q][d] = act ? pos[(base + i) * D + d] : 0.0;
+    xr[q] = act ? x[base + i] : 0.0;
+    acc[q] = 0.0;
+  }
+  const int64_t own = min(n, row0 + RPT * kRows);  // columns of the tile itself
+  for (int64_t c0 = row0; c0 < n;) {
+    const bool diag = c0 < own;
+    const int m = int(min(int64_t(kRows), (diag ? own : n) - c0));
+    __syncthreads();
+    if (int(threadIdx.x) < m) {
+      const int64_t j = base + c0 + threadIdx.x;
+#pragma unroll
+      for (int d = 0; d < D; ++d) sp[d][threadIdx.x] = pos[j * D + d];
+      sx[threadIdx.x] = x[j];
+    }
+#pragma unroll
+    for (int w = 0; w < kRows / 64; ++w) csum[w][threadIdx.x] = 0.0;
+    __syncthreads();
+    if (diag) {
+      // (rows past the problem's end have sums that nobody reads)
+      for (int j = 0; j < m; ++j) {
+        double pj[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) pj[d] = sp[d][j];
+        const double xj = sx[j];
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) sym_phi<D, FP32, MQ>(k, pj, xi[q], xj, acc[q]);
+      }
+    } else {
+      // columns past a tile exist only if the tile is full: every row counts
+      for (int b = 0; b < m; b += 64) {
+        const int mm = min(64, m - b);
+        auto step = [&](int j) {
+          double pj[D];
+#pragma unroll
+          for (int d = 0; d < D; ++d) pj[d] = sp[d][j];
+          const double xj = sx[j];
+          double col = 0.0;
+#pragma unroll
+          for (int q = 0; q < RPT; ++q) {
+            const double f = sym_phi<D, FP32, MQ>(k, pj, xi[q], xj, acc[q]);
+            if (FP32) col += double(float(f) * float(xr[q]));
+            else col = fma(f, xr[q], col);
+          }
+          unsafeAtomicAdd(&csum[wave][j], col);  // this lane's column alone, in step order
+        };
+        if (mm == 64) {
+#pragma unroll 2
+          for (int s = 0; s < 64; ++s) step(b + ((lane + s) & 63));
+        } else {
+          for (int s = 0; s < 64; ++s) {
+            const int j = (lane + s) & 63;
+            if (j < mm) step(b + j);
+          }
+        }
+      }
+      __syncthreads();
+      if (int(threadIdx.x) < m) {
+        double v = csum[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < kRows / 64; ++w) v += csum[w][threadIdx.x];
+        out[c0 - row0 + threadIdx.x] = v;
+      }
+    }
+    c0 += m;
+  }
+#pragma unroll
+  for (int q = 0; q < RPT; ++q) {
+    const int64_t i = threadIdx.x + q * kRows;
+    if (row0 + i < n) out[i] = acc[q];
+  }
+}
+
+// y[i] = (overwrite ? 0 : y[i]) + alpha * the sums of row i over the tiles of
+// its problem up to its own (consecutive in the list, `rows` rows each)
+__global__ __launch_bounds__(kRows) void k_dense_sym_sum(const int2 *__restrict__ tiles, int rows,
+                                                         const int64_t *__restrict__ poff,
+                                                         const int64_t *__restrict__ off,
+                                                         const double *__restrict__ part,
+                                                         double *__restrict__ y,
+                                                         const uint8_t *__restrict__ active,
+                                                         double alpha, int overwrite) {
+  const int t = blockIdx.x;
+  const int p = tiles[t].x;
+  if (active && !active[p]) return;
+  const int64_t base = off[p], n = off[p + 1] - base, row0 = tiles[t].y;
+  const int own = int(row0 / rows);
+  for (int64_t i = row0 + threadIdx.x; i < min(n, row0 + rows); i += kRows) {
+    double v = 0.0;
+#pragma unroll 4
+    for (int b = 0; b <= own; ++b) v += part[poff[t - own + b] + i - int64_t(b) * rows];
     double *yp = &y[base + i];
     *yp = (overwrite ? 0.0 : *yp) + alpha * v;
   }
@@ -225,7 +398,9 @@ __global__ __launch_bounds__(kRows) void k_dense_resid_dd(const int2 *__restrict
 // chains overlap: with the profile chosen inside the loop a column cost a
 // wave 1,500 cycles.  60,000 x 60,000, before and now: multiquadric with
 // eight right-hand sides 9.7 -> 4.0 ms, 1/(r + p) in FP32 5.7 -> 2.3 ms,
-// Gaussian with sixteen 15.3 -> 6.1 ms (FP64 issue bound).
+// Gaussian with sixteen 15.3 -> 6.1 ms (FP64 issue bound).  Against 80-bit sums
+// the 5,000 x 4,001 Gaussian is 2.5e-16 off; one sum per row, here or as a
+// plain matrix product, 1.3e-15.
 constexpr int kRectRhs = 16;
 constexpr int kRectCols = 128;  // columns staged per step
 constexpr int kRectUnroll = 4;
@@ -381,7 +556,10 @@ struct abh_dense_batch {
   const double *pos = nullptr;
   DevBuf tiles[kVariants], off, active;
   int ntiles[kVariants] = {0, 0, 0};
+  bool sym = false;  // the symmetric form, unless a tile shape was forced
+  DevBuf poff, part;
   int choice[2] = {-1, -1};        // tuned variant per precision (FP64, FP32c)
+  bool forced[2] = {false, false};
   float tune_ms[2][kVariants] = {};
 
   template <int RPT>
@@ -407,6 +585,32 @@ struct abh_dense_batch {
     else { ABH_DENSE_LAUNCH(3) }
 #undef ABH_DENSE_LAUNCH
 #undef ABH_DENSE_LAUNCH2
+    abh::check_launch();
+  }
+
+  void run_sym(const double *x, double *y, bool fp32, double alpha, bool overwrite,
+               const uint8_t *act) {
+    hipStream_t s = ctx->stream;
+    const int2 *tl = tiles[kSymVariant].as<int2>();
+    const int64_t *o = off.as<int64_t>(), *po = poff.as<int64_t>();
+    double *pt = part.as<double>();
+    const int nt = ntiles[kSymVariant];
+    const bool mq =
+        k.type == ABH_KERNEL_MULTIQUADRIC && !k.row_s && !k.col_s && k.param2 >= 1e-280;
+#define ABH_DENSE_SYM2(DD, MQ)                                                             \
+  if (fp32) k_dense_sym<DD, true, MQ><<<nt, kRows, 0, s>>>(tl, po, o, pos, x, pt, act, k); \
+  else k_dense_sym<DD, false, MQ><<<nt, kRows, 0, s>>>(tl, po, o, pos, x, pt, act, k);
+#define ABH_DENSE_SYM(DD)             \
+  if (mq) { ABH_DENSE_SYM2(DD, true) } \
+  else { ABH_DENSE_SYM2(DD, false) }
+    if (dim == 1) { ABH_DENSE_SYM(1) }
+    else if (dim == 2) { ABH_DENSE_SYM(2) }
+    else { ABH_DENSE_SYM(3) }
+#undef ABH_DENSE_SYM
+#undef ABH_DENSE_SYM2
+    abh::check_launch();
+    k_dense_sym_sum<<<nt, kRows, 0, s>>>(tl, kSymRpt * kRows, po, o, pt, y, act, alpha,
+                                         overwrite ? 1 : 0);
     abh::check_launch();
   }
 
@@ -471,7 +675,9 @@ struct abh_dense_batch {
 
   void apply(const double *x, double *y, bool fp32, double alpha, bool overwrite,
              const uint8_t *act) {
-    run(tune(fp32), x, y, fp32, alpha, overwrite, act);
+    const int v = tune(fp32);
+    if (sym && !forced[fp32 ? 1 : 0]) run_sym(x, y, fp32, alpha, overwrite, act);
+    else run(v, x, y, fp32, alpha, overwrite, act);
   }
 };
 
@@ -623,16 +829,38 @@ abh_status abh_dense_batch_create(abh_context *ctx, int dim, int nprob, const in
     });
     hipStream_t s = ctx->stream;
     std::vector<int2> tl[kVariants];
+    std::vector<int64_t> po;
+    int64_t sums = 0;
+    double values = 0.0, shared = 0.0;  // kernel values one-sided and symmetric
     for (int v = 0; v < kVariants; ++v) {
       const int64_t rows = int64_t(kRows) * kRptOf[v];
       for (int p : order)
-        for (int64_t r = 0; r < offsets[p + 1] - offsets[p]; r += rows)
+        for (int64_t r = 0, np = offsets[p + 1] - offsets[p]; r < np; r += rows) {
           tl[v].push_back(make_int2(p, int(r)));
+          if (v != kSymVariant) continue;
+          po.push_back(sums);
+          sums += np - r;
+          values += double(std::min(rows, np - r)) * double(np);
+          shared += double(rows) * double(np - r);
+        }
       op->ntiles[v] = int(tl[v].size());
       op->tiles[v].ensure(tl[v].size() * sizeof(int2) + 16);
       if (!tl[v].empty())
         ABH_HIP(hipMemcpyAsync(op->tiles[v].p, tl[v].data(), tl[v].size() * sizeof(int2),
                                hipMemcpyHostToDevice, s));
+    }
+    op->sym = shared <= 0.75 * values && sums <= kSymPart &&
+              op->ntiles[kSymVariant] >= kSymTiles * ctx->n_cu;
+    if (op->sym) {
+      op->poff.ensure(po.size() * 8 + 16);
+      ABH_HIP(hipMemcpyAsync(op->poff.p, po.data(), po.size() * 8, hipMemcpyHostToDevice, s));
+      try {
+        op->part.ensure_exact(size_t(sums) * 8);
+      } catch (const abh::Error &e) {  // no room: k_dense needs none
+        if (e.status != ABH_ERR_OUT_OF_MEMORY) throw;
+        (void)hipGetLastError();
+        op->sym = false;
+      }
     }
     op->off.ensure(size_t(nprob + 1) * 8);
     op->active.ensure(size_t(nprob) + 16);
@@ -870,6 +1098,7 @@ abh_status abh_dense_batch_tune(abh_dense_batch *op, abh_precision precision, in
         if (kRptOf[q] == *rows_per_thread) v = q;
       ABH_REQUIRE(v >= 0, ABH_ERR_INVALID_ARG, "rows_per_thread must be 1, 2 or 4");
       op->choice[fp32 ? 1 : 0] = v;
+      op->forced[fp32 ? 1 : 0] = true;
       return;
     }
     const int v = op->tune(fp32);

@@ -592,7 +592,9 @@ abh_status abh_dense_apply_noalloc(abh_context *ctx, int dim, int64_t nrows,
  * this batch once and keeps the fastest for the precision; apply and gmres
  * tune on first use.  rows_per_thread (host, may be NULL) gets the choice,
  * variant_ms (host, 3 floats, may be NULL) the measured times.  A positive
- * *rows_per_thread on entry (1, 2 or 4) sets that shape instead of tuning. */
+ * *rows_per_thread on entry (1, 2 or 4) sets that shape instead of tuning.
+ * Batches of many tiles use every kernel value for its row and its column
+ * (a choice by the sizes alone) unless a shape is set. */
 abh_status abh_dense_batch_tune(abh_dense_batch *op, abh_precision precision,
                                 int *rows_per_thread, float *variant_ms);
 
