@@ -556,6 +556,156 @@ __global__ __launch_bounds__(128 * m2l_row_groups(DIM)) void k_m2l_mfma64(const 
   }  // pass
 }
 
+// The M2L for at most eight right-hand sides.  k_m2l_mfma64 gives each child
+// its own 16 columns, the right-hand sides padded to 16; here a block's 16 CB
+// columns are the children of 2 CB / NRP neighbouring sibling tiles times NRP
+// right-hand sides (NRP: nrhs rounded up to 1, 2, 4 or 8), so that no product
+// is formed for padding and an operator fragment serves 16 CB columns.  The
+// offsets are split over blockIdx.y (few tiles on the coarse levels: one block
+// walked all 316 offsets, 0.5 to 1.5 ms a level), each split writing its sums
+// to part, which k_m2l_few_sum adds to G in split order (deterministic).  The
+// expansions are read from Wp, packed without padding (k_pack_w).  Bound by
+// the operators' fragments out of L2.  Order 4, 100,000 points, one
+// right-hand side, three levels: 4.65 ms before, now 1.1 ms with the packing
+// and the sums.
+constexpr int kFewSplits = 8;
+constexpr int kFewSpan = (kOffsets + kFewSplits - 1) / kFewSplits;  // offsets per split
+
+template <int CB> __device__ __host__ constexpr int few_tiles(int nrp) { return 2 * CB / nrp; }
+
+// Wp[(box NC + k) nrp + r] = W[(box NC + k) 16 + r], r < nrp
+__global__ __launch_bounds__(256) void k_pack_w(const double *__restrict__ W, int64_t rows, int nrp,
+                                                double *__restrict__ Wp) {
+  const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (e < rows * nrp) Wp[e] = W[(e / nrp) * kRhs + e % nrp];
+}
+
+template <int DIM, int CB>
+__global__ __launch_bounds__(256) void k_m2l_few(const int32_t *__restrict__ tile_parent,
+                                                 int ntiles, const int32_t *__restrict__ child0,
+                                                 const int32_t *__restrict__ coord,
+                                                 const int32_t *__restrict__ map, int side,
+                                                 const double *__restrict__ Mf,
+                                                 const double *__restrict__ Wp, int nrp,
+                                                 double *__restrict__ part) {
+  using F = Mfma64<DIM>;
+  constexpr int NC = F::NC, RB = F::RB, KS = F::KS;
+  constexpr int NP = (RB + 7) / 8;           // passes over the offsets (registers)
+  constexpr int RBP = (RB + NP - 1) / NP;    // row blocks per pass
+  constexpr int RPW = (RBP + 3) / 4;         // row blocks per wave and pass
+  constexpr int kMaxChild = 16 * CB;
+  __shared__ int32_t src[kFewSpan][kMaxChild];
+  const int tt = few_tiles<CB>(nrp), nchild = 8 * tt;
+  const int tile0 = int(blockIdx.x) * tt;
+  const int o0 = int(blockIdx.y) * kFewSpan;
+  // source node of every (offset, child) of the block, -1 = none
+  for (int e = threadIdx.x; e < kFewSpan * nchild; e += 256) {
+    const int o = o0 + e / nchild, q = e % nchild, ch = q & 7, tile = tile0 + (q >> 3);
+    int s = -1;
+    const int ox = o / 49 - 3, oy = (o / 7) % 7 - 3, oz = o % 7 - 3;
+    const bool near = ox >= -1 && ox <= 1 && oy >= -1 && oy <= 1 && oz >= -1 && oz <= 1;
+    if (o < kOffsets && !near && tile < ntiles) {
+      const int qx = ((ch >> 2) & 1) + ox, qy = ((ch >> 1) & 1) + oy, qz = (ch & 1) + oz;
+      if (qx >= -2 && qx <= 3 && qy >= -2 && qy <= 3 && qz >= -2 && qz <= 3) {
+        const int parent = tile_parent[tile];
+        const int sx = 2 * coord[parent * 3 + 0] + qx, sy = 2 * coord[parent * 3 + 1] + qy,
+                  sz = 2 * coord[parent * 3 + 2] + qz;
+        if (sx >= 0 && sx < side && sy >= 0 && sy < side && sz >= 0 && sz < side)
+          s = map[(int64_t(sx) * side + sy) * side + sz];
+      }
+    }
+    src[e / nchild][q] = s;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int kl = lane >> 4, rl = lane & 15;
+  int child[CB], rhs[CB];
+#pragma unroll
+  for (int c = 0; c < CB; ++c) {
+    child[c] = (16 * c + rl) / nrp;
+    rhs[c] = (16 * c + rl) % nrp;
+  }
+  for (int pass = 0; pass < NP; ++pass) {
+    f64x4 acc[RPW][CB];
+#pragma unroll
+    for (int i = 0; i < RPW; ++i)
+#pragma unroll
+      for (int c = 0; c < CB; ++c) acc[i][c] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int d = 0; d < kFewSpan; ++d) {
+      int sc[CB];
+      bool any = false;
+#pragma unroll
+      for (int c = 0; c < CB; ++c) {
+        sc[c] = src[d][child[c]];
+        any = any || sc[c] >= 0;
+      }
+      if (__ballot(any) == 0) continue;
+      const double *Mo = Mf + int64_t(o0 + d) * F::PER_OFFSET;
+      // (a child without this source reads box 0 and multiplies by nothing)
+      const double *wb[CB];
+#pragma unroll
+      for (int c = 0; c < CB; ++c)
+        wb[c] = Wp + (int64_t(sc[c] >= 0 ? sc[c] : 0) * NC) * nrp + rhs[c];
+#pragma unroll 2
+      for (int ks = 0; ks < KS; ++ks) {
+        double av[RPW], bv[CB];
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) {
+          const int rb = pass * RBP + wave + 4 * i;
+          av[i] = Mo[(int64_t(ks) * RB + (rb < RB ? rb : RB - 1)) * 64 + lane];
+        }
+        const int k = ks * 4 + kl < NC ? ks * 4 + kl : NC - 1;  // (A is zero past NC)
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+          const double w = wb[c][int64_t(k) * nrp];
+          bv[c] = sc[c] >= 0 ? w : 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < RPW; ++i)
+          if (wave + 4 * i < RBP)
+#pragma unroll
+            for (int c = 0; c < CB; ++c)
+              acc[i][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[i], bv[c], acc[i][c], 0, 0, 0);
+      }
+    }
+    double *out = part + int64_t(blockIdx.y) * ntiles * 8 * NC * nrp;
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      const int rb = pass * RBP + wave + 4 * i;
+      if (wave + 4 * i >= RBP || rb >= RB) continue;
+#pragma unroll
+      for (int c = 0; c < CB; ++c) {
+        if (tile0 + (child[c] >> 3) >= ntiles) continue;
+        const int64_t q = int64_t(tile0) * 8 + child[c];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = rb * 16 + kl + 4 * v;
+          if (row < NC) out[(q * NC + row) * nrp + rhs[c]] = acc[i][c][v];
+        }
+      }
+    }
+  }
+}
+
+// G of every child += its splits' sums, in order
+__global__ __launch_bounds__(256) void k_m2l_few_sum(const int32_t *__restrict__ tile_parent,
+                                                     int ntiles, const int32_t *__restrict__ child0,
+                                                     int NC, int nrp,
+                                                     const double *__restrict__ part,
+                                                     double *__restrict__ G) {
+  const int64_t total = int64_t(ntiles) * 8 * NC * nrp;
+  const int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (e >= total) return;
+  const int r = int(e % nrp);
+  const int64_t qr = e / nrp;  // child of the list, row
+  const int64_t q = qr / NC, row = qr % NC;
+  double v = 0.0;
+#pragma unroll
+  for (int s = 0; s < kFewSplits; ++s) v += part[s * total + e];
+  const int64_t node = int64_t(child0[tile_parent[q >> 3]]) + (q & 7);
+  G[(node * NC + row) * kRhs + r] += v;
+}
+
 // ---------------------------------------------------------------------------
 // M2L on the matrix cores: BF16 MFMA with a three-term split
 // (a = a_hi + a_lo, ab ~ a_hi b_hi + a_hi b_lo + a_lo b_hi, FP32 accumulation)
@@ -1584,6 +1734,10 @@ struct abh_fmm {
   DevBuf Mh, Ml, Wh, Wl;  // BF16 hi / lo parts for the MFMA M2L
   bool split_ready = false;
   DevBuf Mf;              // FP64 M2L operators in the MFMA fragment layout
+  // k_m2l_few: packed expansions and the splits' sums, for up to few_max
+  // right-hand sides; allocated once (a captured apply keeps their addresses)
+  DevBuf Wp, part;
+  int few_max = -1;
   bool pack_ready = false;
   // compressed M2L (abh_fmm_compress): per level an orthonormal basis U
   // (NC x comp_kp, the leading eigenvectors of the level's stacked
@@ -1948,6 +2102,39 @@ void tune_m2l16(abh_fmm *f, hipStream_t s) {
   ABH_HIP(hipMemsetAsync(f->Gc.p, 0, size_t(f->n_nodes) * f->comp_kp * kRhs * 8, s));
 }
 
+// Right-hand sides (1, 2, 4, 8 or none) that k_m2l_few's buffers hold: the
+// most that fit 2 GB, allocated at the first apply that asks, outside a stream
+// capture.
+int few_limit(abh_fmm *f, int NC) {
+  if (f->few_max >= 0) return f->few_max;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(f->ctx->stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  if (st != hipStreamCaptureStatusNone) return 0;
+  size_t widest = 0;
+  for (int l = 2; l <= f->nlevels; ++l)
+    widest = std::max(widest, size_t(f->tree.par_off[l] - f->tree.par_off[l - 1]));
+  const size_t pack = size_t(f->n_nodes) * NC * 8, sums = size_t(kFewSplits) * widest * 8 * NC * 8;
+  int nrp = 8;
+  while (nrp > 0 && (pack + sums) * nrp > (size_t(2) << 30)) nrp /= 2;
+  if (nrp > 0) {
+    try {
+      f->Wp.ensure_exact(pack * nrp + 64);
+      f->part.ensure_exact(sums * nrp + 64);
+    } catch (const abh::Error &e) {  // no room: the sixteen-column form
+      if (e.status != ABH_ERR_OUT_OF_MEMORY) throw;
+      (void)hipGetLastError();
+      f->Wp.release();
+      f->part.release();
+      nrp = 0;
+    }
+  }
+  f->few_max = nrp;
+  return nrp;
+}
+
 template <int N> void apply_impl(abh_fmm *f, int nrhs, const double *x, int64_t ldx, double *y,
                                  int64_t ldy, abh_precision prec) {
   constexpr int NC = Cheb<N>::NC;
@@ -1999,6 +2186,17 @@ template <int N> void apply_impl(abh_fmm *f, int nrhs, const double *x, int64_t 
       abh::check_launch();
     }
     const int KP = f->comp_kp;
+    // FP64, uncompressed, few right-hand sides: packed columns
+    int nrp = 16;
+    if (KP == 0 && !(mixed && NC <= kPad) && f->nlevels >= 2 && nr <= 8) {
+      nrp = nr <= 2 ? nr : (nr <= 4 ? 4 : 8);
+      if (nrp > few_limit(f, NC)) nrp = 16;
+    }
+    if (nrp <= 8) {
+      k_pack_w<<<unsigned(abh::ceil_div(nn * NC * nrp, int64_t(256))), 256, 0, s>>>(
+          f->W.as<double>(), nn * NC, nrp, f->Wp.as<double>());
+      abh::check_launch();
+    }
     if (KP > 0) {
       // compressed expansions of every level's boxes (tiles = the parents
       // one level up), zeroed compressed locals
@@ -2073,11 +2271,30 @@ template <int N> void apply_impl(abh_fmm *f, int nrhs, const double *x, int64_t 
           abh::check_launch();
           f->pack_ready = true;
         }
-        k_m2l_mfma64<NC><<<xcd_grid(npar(l - 1)), 128 * m2l_row_groups(NC), 0, s>>>(
-            par + f->tree.par_off[l - 1], npar(l - 1), f->tree.nodes.as<int32_t>(), f->coord.as<int32_t>(),
-            f->maps.as<int32_t>() + f->map_off[l], 1 << l,
-            f->Mf.as<double>() + int64_t(l - 2) * kOffsets * F::PER_OFFSET, f->W.as<double>(),
-            f->G.as<double>());
+        const int32_t *pl = par + f->tree.par_off[l - 1];
+        const int nt = npar(l - 1);
+        const int32_t *map = f->maps.as<int32_t>() + f->map_off[l];
+        const double *Ml = f->Mf.as<double>() + int64_t(l - 2) * kOffsets * F::PER_OFFSET;
+        if (nrp <= 8) {
+          const int tt = nrp <= 4 ? few_tiles<2>(nrp) : few_tiles<4>(nrp);
+          const dim3 grid(unsigned(abh::ceil_div(nt, tt)), kFewSplits);
+          if (nrp <= 4)
+            k_m2l_few<NC, 2><<<grid, 256, 0, s>>>(pl, nt, f->tree.nodes.as<int32_t>(),
+                                                  f->coord.as<int32_t>(), map, 1 << l, Ml,
+                                                  f->Wp.as<double>(), nrp, f->part.as<double>());
+          else
+            k_m2l_few<NC, 4><<<grid, 256, 0, s>>>(pl, nt, f->tree.nodes.as<int32_t>(),
+                                                  f->coord.as<int32_t>(), map, 1 << l, Ml,
+                                                  f->Wp.as<double>(), nrp, f->part.as<double>());
+          abh::check_launch();
+          k_m2l_few_sum<<<unsigned(abh::ceil_div(int64_t(nt) * 8 * NC * nrp, 256)), 256, 0, s>>>(
+              pl, nt, f->tree.nodes.as<int32_t>(), NC, nrp, f->part.as<double>(),
+              f->G.as<double>());
+        } else {
+          k_m2l_mfma64<NC><<<xcd_grid(nt), 128 * m2l_row_groups(NC), 0, s>>>(
+              pl, nt, f->tree.nodes.as<int32_t>(), f->coord.as<int32_t>(), map, 1 << l, Ml,
+              f->W.as<double>(), f->G.as<double>());
+        }
       }
       abh::check_launch();
     }
