@@ -6,9 +6,11 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <new>
 #include <string>
 #include <utility>
+#include <vector>
 
 #include "../../include/aboria_hip.h"
 
@@ -88,7 +90,14 @@ struct abh_context {
   // every primitive is enqueued on the one context stream)
   abh::DevBuf scan_blocks;                     // per-tile sums of scan_exclusive
   abh::DevBuf sort_keys, sort_vals, sort_hist;  // radix sort ping-pong + histograms
-  abh::DevBuf dense_part;                       // column-split partial sums (abh_dense_apply)
+  // Column-split partial sums of abh_dense_apply: the coarse split's and the
+  // fine split's (dense.hip).  Captured applies use the coarse split alone, so
+  // the fine one's buffer is in no graph.  A coarse buffer that a capture has
+  // seen is set aside when the context needs a larger one and freed with the
+  // context: its graph may be replayed at any time.
+  abh::DevBuf dense_part, dense_fine;
+  bool dense_part_captured = false;
+  std::vector<std::unique_ptr<abh::DevBuf>> dense_part_kept;
   // Schwarz set-up (schwarz.hip): the working set of a factorisation group (at
   // most about 3 GB) and the inverse rows of the last preconditioner
   // destroyed (at most 4 GB), kept for the next one until the context goes or

@@ -692,9 +692,37 @@ bool stream_capturing(hipStream_t s) {
   return st != hipStreamCaptureStatusNone;
 }
 
+// The context's buffer for the coarse split's partial sums, at least `doubles`
+// long.  Growing keeps a buffer that a graph may still use.
+double *coarse_part(abh_context *ctx, size_t doubles, bool capturing) {
+  DevBuf &b = ctx->dense_part;
+  if (b.bytes < doubles * 8 && ctx->dense_part_captured) {
+    ctx->dense_part_kept.emplace_back(new DevBuf());
+    ctx->dense_part_kept.back()->swap(b);
+    ctx->dense_part_captured = false;
+  }
+  b.ensure(doubles * 8);
+  ctx->dense_part_captured = ctx->dense_part_captured || capturing;
+  return b.as<double>();
+}
+
+// The context's buffer for the fine split's partial sums, as large as the
+// static scratch, so that it is allocated once; false if there is no room
+// (the coarse split's shapes of one range need none).
+bool fine_part(abh_context *ctx) {
+  try {
+    ctx->dense_fine.ensure_exact(kNoAllocScratchDoubles * 8);
+  } catch (const abh::Error &e) {
+    if (e.status != ABH_ERR_OUT_OF_MEMORY) throw;
+    (void)hipGetLastError();
+    return false;
+  }
+  return true;
+}
+
 // y += K x for the rectangular operator.  part_ext == nullptr: the column
-// split's partial sums live in the context's grow-only buffer; otherwise in
-// part_ext (part_cap doubles), and a split that needs more is refused.
+// split's partial sums live in the context's buffers; otherwise in part_ext
+// (part_cap doubles), and a split that needs more is refused.
 void dense_apply_impl(abh_context *ctx, int dim, int64_t nrows, const double *row_pos,
                       int64_t ncols, const double *col_pos, const abh_kernel *kernel, int nrhs,
                       const double *x, int64_t ldx, double *y, int64_t ldy,
@@ -727,8 +755,8 @@ void dense_apply_impl(abh_context *ctx, int dim, int64_t nrows, const double *ro
   // 5,000 x 4,001 Gaussian took 1,313 us in one range (20 blocks), 26 us in
   // 126 ranges; 300 x 50,000 760 us in 24, 52 us in 1,563.  A captured
   // abh_dense_apply keeps the coarse split, which needs no buffer of the
-  // context for the shapes that never needed one (the context may replace
-  // its buffer before the graph is replayed).
+  // context for the shapes that never needed one: a graph may be replayed on
+  // any stream, beside calls that use the context's buffers.
   int64_t ns = 1;
   const int64_t want = int64_t(ctx->n_cu) * 8;
   if (grows < want && ncols > 0)
@@ -736,21 +764,14 @@ void dense_apply_impl(abh_context *ctx, int dim, int64_t nrows, const double *ro
   int64_t cspan =
       ncols > 0 ? abh::ceil_div(abh::ceil_div(ncols, ns), int64_t(kRows)) * kRows : 1;
   ns = ncols > 0 ? abh::ceil_div(ncols, cspan) : 1;
-  const int64_t fit =
-      int64_t(kNoAllocScratchDoubles) / (int64_t(std::min(nrhs, kRectRhs)) * nrows);
-  if (grows < want && ns <= fit && (part_ext || !stream_capturing(s))) {
-    const int64_t fine = std::min({abh::ceil_div(want, grows), fit, ncols / 32});
-    if (fine > ns) {
-      cspan = abh::ceil_div(abh::ceil_div(ncols, fine), int64_t(32)) * 32;
-      ns = abh::ceil_div(ncols, cspan);
-    }
-  }
+  // part[s][r][i] for the ranges s, the right-hand sides r of one pass and
+  // the rows i; every entry is written by k_dense_rect before k_rect_reduce
+  // reads it, so the buffer needs no clearing
+  const size_t row_part = size_t(std::min(nrhs, kRectRhs)) * size_t(nrows);
+  const bool capturing = !part_ext && stream_capturing(s);
   double *part = nullptr;
   if (ns > 1) {
-    // part[s][r][i] for the ranges s, the right-hand sides r of one pass and
-    // the rows i; every entry is written by k_dense_rect before k_rect_reduce
-    // reads it, so the buffer needs no clearing
-    const size_t need = size_t(ns) * size_t(std::min(nrhs, kRectRhs)) * size_t(nrows);
+    const size_t need = size_t(ns) * row_part;
     if (part_ext) {
       ABH_REQUIRE(need <= part_cap, ABH_ERR_CAPACITY,
                   "column split needs " + std::to_string(need * 8) +
@@ -759,8 +780,18 @@ void dense_apply_impl(abh_context *ctx, int dim, int64_t nrows, const double *ro
                       "abh_dense_apply, or fewer right-hand sides per call)");
       part = part_ext;
     } else {
-      ctx->dense_part.ensure(need * sizeof(double));
-      part = ctx->dense_part.as<double>();
+      // (allocated also where the fine split follows: a later capture of this
+      // shape then finds it)
+      part = coarse_part(ctx, need, capturing);
+    }
+  }
+  const int64_t fit = int64_t(kNoAllocScratchDoubles / row_part);
+  if (grows < want && ns <= fit && !capturing) {
+    const int64_t fine = std::min({abh::ceil_div(want, grows), fit, ncols / 32});
+    if (fine > ns && (part_ext || fine_part(ctx))) {
+      cspan = abh::ceil_div(abh::ceil_div(ncols, fine), int64_t(32)) * 32;
+      ns = abh::ceil_div(ncols, cspan);
+      part = part_ext ? part_ext : ctx->dense_fine.as<double>();
     }
   }
   const dim3 grid{unsigned(grows), unsigned(ns), 1u};

@@ -560,8 +560,12 @@ abh_status abh_dense_batch_apply(abh_dense_batch *op, const double *x, double *y
  * x: column-major ncols x nrhs (leading dimension ldx); y: nrows x nrhs
  * (ldy).  precision: ABH_FP64 or ABH_FP32_COMPENSATED.  With fewer rows
  * than 2,048 per CU the columns are split into ranges whose partial sums the
- * context keeps in a device buffer (ranges x 16 x nrows doubles, kept for
- * later calls) and adds in range order: results are deterministic. */
+ * context keeps in device buffers (at most 32 MiB, or ranges of 2,048 columns
+ * and more x 16 x nrows doubles; kept for later calls) and adds in range
+ * order: results are deterministic.  A call under stream capture splits into
+ * ranges of at least 2,048 columns only, so that a graph of a smaller operator
+ * uses no buffer of the context: its result differs from an uncaptured call's
+ * in rounding. */
 abh_status abh_dense_apply(abh_context *ctx, int dim, int64_t nrows,
                            const double *row_pos, int64_t ncols,
                            const double *col_pos, const abh_kernel *kernel,
@@ -571,7 +575,8 @@ abh_status abh_dense_apply(abh_context *ctx, int dim, int64_t nrows,
 /* abh_dense_apply without any device allocation: no counterpart in the
  * reference; for callers that cannot allocate (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc).  Same arguments,
- * kernels and results as abh_dense_apply (bit for bit); the column split's
+ * kernels and results as an uncaptured abh_dense_apply (bit for bit, under
+ * capture too); the column split's
  * partial sums live in a static 32 MiB device array (one per device, held
  * until the process ends) instead of the context's grow-only buffer.  A
  * shape whose split needs more (ranges x min(nrhs, 16) x nrows doubles

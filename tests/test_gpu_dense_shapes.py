@@ -67,3 +67,37 @@ def test_dense_apply_captured(ctx):
             assert torch.allclose(y, k * ref, rtol=1e-12, atol=1e-12)
             assert torch.isfinite(big).all()
         c.close()
+
+
+@pytest.mark.parametrize("nrows,ncols,nrhs", [(300, 50_000, 2), (40, 9_000, 16)])
+def test_captured_split_keeps_its_buffer(ctx, nrows, ncols, nrhs):
+    """A captured apply that splits its columns (ranges of 2,048 and more) while
+    later calls need larger buffers of the context: no buffer that the graph
+    knows is freed, and every replay adds K x.  Bar: each replay's sum and ref
+    are within ncols roundings of the exact one."""
+    g = torch.Generator(device="cuda").manual_seed(nrows)
+    rand = lambda *s: torch.rand(*s, generator=g, device="cuda", dtype=torch.float64)  # noqa: E731
+    rows, cols, x = rand(nrows, 3), rand(ncols, 3), rand(nrhs, ncols) - 0.5
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        c = ab.Context(0, stream)
+        kernel = ab.Kernel.gaussian(0.2)
+        y = torch.zeros(nrhs, nrows, dtype=torch.float64, device="cuda")
+        ref = ab.dense_apply(c, rows, cols, kernel, x)
+        scale = ab.dense_apply(c, rows, cols, kernel, x.abs())
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            ab.dense_apply(c, rows, cols, kernel, x, y)
+        # fine splits of up to 32 MiB, then a coarse one of 82 MiB
+        shapes = [(5_000, 4_001, 1), (4_000, 5_000, 3), (20_000, 65_536, 16), (300, 60_000, 4)]
+        for k, (m, n, r) in enumerate(shapes, 1):
+            print("replay", k, flush=True)
+            big = ab.dense_apply(c, rand(m, 3), rand(n, 3), kernel, rand(r, n))
+            stream.synchronize()
+            graph.replay()
+            stream.synchronize()
+            assert torch.all((y - k * ref).abs() <= (k + 1) * (ncols + 64) * 2.0 ** -52 * scale)
+            assert torch.isfinite(big).all()
+        del graph
+        c.close()

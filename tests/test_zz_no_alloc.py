@@ -74,3 +74,28 @@ def test_noalloc_refuses_oversized_split(ctx):
     assert b"static scratch" in lib.abh_last_error(ctx.handle)
     torch.cuda.synchronize()
     assert torch.count_nonzero(y) == 0
+
+
+def test_noalloc_captured(ctx):
+    """Captured, the allocation-free entry point gives the bits of its (and
+    abh_dense_apply's) uncaptured call, in every replay."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda *s: torch.rand(*s, generator=g, device="cuda", dtype=torch.float64)  # noqa: E731
+    rows, cols, x = rand(500, 3), rand(9_000, 3), rand(2, 9_000) - 0.5
+    lib, kernel = C.lib(), ab.Kernel.gaussian(0.2)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        c = ab.Context(0, stream)
+        y = torch.zeros(2, 500, dtype=torch.float64, device="cuda")
+        ref = torch.zeros_like(y)
+        assert _call(lib.abh_dense_apply, c, rows, cols, kernel, x, ref, ab.FP64) == 0
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            assert _call(lib.abh_dense_apply_noalloc, c, rows, cols, kernel, x, y, ab.FP64) == 0
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            stream.synchronize()
+            assert torch.equal(y, ref)
+        c.close()
