@@ -80,6 +80,12 @@ class Context:
     def sync(self):
         check(C.lib().abh_context_sync(self.handle), self.handle)
 
+    def trim(self):
+        """Frees device memory that the context only keeps for later calls
+        (at most 7 GiB, from Schwarz preconditioners); for when torch's own
+        allocator runs out.  The library's allocations do it by themselves."""
+        check(C.lib().abh_context_trim(self.handle), self.handle)
+
     def close(self):
         if getattr(self, "handle", None):
             C.lib().abh_context_destroy(self.handle)

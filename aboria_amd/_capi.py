@@ -147,6 +147,7 @@ SIGNATURES = {
     "abh_context_create": (c_int, [c_int, c_void_p, P(c_void_p)]),
     "abh_context_destroy": (c_int, [c_void_p]),
     "abh_context_sync": (c_int, [c_void_p]),
+    "abh_context_trim": (c_int, [c_void_p]),
     "abh_status_string": (ctypes.c_char_p, [c_int]),
     "abh_last_error": (ctypes.c_char_p, [c_void_p]),
     "abh_malloc": (c_int, [c_void_p, P(c_void_p), c_size_t]),

@@ -24,6 +24,34 @@ using abh::DevBuf;
 using abh::GridParams;
 
 namespace abh {
+hipError_t device_alloc(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && entry_context && idle_bytes(entry_context) > 0) {
+    release_idle(entry_context);
+    e = hipMalloc(p, bytes);
+  }
+  // a failure is reported by its status alone, not to the next launch check
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
+size_t idle_bytes(const abh_context *ctx) {
+  size_t sum = ctx->factor_spare.bytes;
+  if (!ctx->factor_busy)
+    for (const DevBuf *b : {&ctx->factor_a, &ctx->factor_d, &ctx->factor_ds, &ctx->factor_w,
+                            &ctx->factor_sg})
+      sum += b->bytes;
+  return sum;
+}
+
+void release_idle(abh_context *ctx) {
+  ctx->factor_spare.release();
+  if (ctx->factor_busy) return;
+  for (DevBuf *b : {&ctx->factor_a, &ctx->factor_d, &ctx->factor_ds, &ctx->factor_w,
+                    &ctx->factor_sg})
+    b->release();
+}
+
 void context_free(abh_context *ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
@@ -256,8 +284,18 @@ abh_status abh_context_create(int device, void *stream, abh_context **out) {
 abh_status abh_context_destroy(abh_context *ctx) {
   if (!ctx || ctx->closed) return ABH_OK;
   ctx->closed = true;
-  if (ctx->refs == 0) abh::context_free(ctx);
+  if (ctx->refs == 0) {
+    abh::context_free(ctx);
+  } else {  // the handles left make no new ones
+    (void)hipSetDevice(ctx->device);
+    abh::release_idle(ctx);
+  }
   return ABH_OK;
+}
+
+abh_status abh_context_trim(abh_context *ctx) {
+  if (!ctx) return ABH_ERR_INVALID_ARG;
+  return abh::guard(ctx, [&] { abh::release_idle(ctx); });
 }
 
 abh_status abh_context_sync(abh_context *ctx) {
@@ -284,7 +322,7 @@ const char *abh_last_error(const abh_context *ctx) { return ctx ? ctx->last_erro
 
 abh_status abh_malloc(abh_context *ctx, void **ptr, size_t bytes) {
   if (!ctx || !ptr) return ABH_ERR_INVALID_ARG;
-  return abh::guard(ctx, [&] { ABH_HIP(hipMalloc(ptr, bytes ? bytes : 1)); });
+  return abh::guard(ctx, [&] { ABH_HIP(abh::device_alloc(ptr, bytes ? bytes : 1)); });
 }
 abh_status abh_free(abh_context *ctx, void *ptr) {
   if (!ctx) return ABH_ERR_INVALID_ARG;

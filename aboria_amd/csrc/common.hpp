@@ -34,6 +34,11 @@ struct Error {
     if (!(cond)) throw ::abh::Error{status, std::string(message)}; \
   } while (0)
 
+// hipMalloc.  When there is no room, the memory that the calling thread's
+// context (the one of the entry point it is in) only keeps for later calls is
+// released and the allocation tried once more.
+hipError_t device_alloc(void **p, size_t bytes);  // cells.hip
+
 // Grow-only device buffer.  Growing frees the old allocation (hipFree
 // synchronises the device, so pending kernels that used it have finished).
 struct DevBuf {
@@ -52,14 +57,14 @@ struct DevBuf {
     if (want <= bytes && p) return;
     release();
     size_t alloc = want + want / 4 + 256;
-    ABH_HIP(hipMalloc(&p, alloc));
+    ABH_HIP(device_alloc(&p, alloc));
     bytes = alloc;
   }
   // at least `want` bytes, without room to grow
   void ensure_exact(size_t want) {
     if (want <= bytes && p) return;
     release();
-    ABH_HIP(hipMalloc(&p, want));
+    ABH_HIP(device_alloc(&p, want));
     bytes = want;
   }
   void swap(DevBuf &o) {
@@ -98,13 +103,15 @@ struct abh_context {
   abh::DevBuf dense_part, dense_fine;
   bool dense_part_captured = false;
   std::vector<std::unique_ptr<abh::DevBuf>> dense_part_kept;
-  // Schwarz set-up (schwarz.hip): the working set of a factorisation group (at
-  // most about 3 GB) and the inverse rows of the last preconditioner
-  // destroyed (at most 4 GB), kept for the next one until the context goes or
-  // memory runs out.  Once a process has cycled through the card's memory the
-  // driver clears what is freed, about 28 ms per GB.
+  // Schwarz set-up (schwarz.hip): the working set of a factorisation group (a
+  // larger one than kFactorKeep is freed at once) and the inverse rows of the
+  // last preconditioner destroyed (at most kSpareKeep), kept for the next one
+  // until the context is destroyed or trimmed or an allocation of its entry
+  // points finds no room.  Once a process has cycled through the card's memory
+  // the driver clears what is freed, about 28 ms per GB.
   abh::DevBuf factor_a, factor_d, factor_ds, factor_w, factor_sg;
   abh::DevBuf factor_spare;
+  bool factor_busy = false;  // a factorisation is using factor_a .. factor_sg
   int n_cu = 256;
   // device address of the static scratch of abh_dense_apply_noalloc on this
   // context's device (hipGetSymbolAddress at context creation)
@@ -117,8 +124,27 @@ struct abh_context {
 
 namespace abh {
 
+constexpr size_t kFactorKeep = size_t(3) << 30;
+constexpr size_t kSpareKeep = size_t(4) << 30;
+
+// What the context keeps for later calls and no call is using, and its
+// release (device work that used it has finished when hipFree returns).
+size_t idle_bytes(const abh_context *ctx);
+void release_idle(abh_context *ctx);
+
+// The context of the entry point that this thread is in.
+inline thread_local abh_context *entry_context = nullptr;
+struct EntryScope {
+  abh_context *before = entry_context;
+  explicit EntryScope(abh_context *ctx) { entry_context = ctx; }
+  EntryScope(const EntryScope &) = delete;
+  EntryScope &operator=(const EntryScope &) = delete;
+  ~EntryScope() { entry_context = before; }
+};
+
 // Runs f() and converts internal errors to a status at the C ABI.
 template <class F> abh_status guard(abh_context *ctx, F &&f) {
+  EntryScope scope(ctx);
   try {
     if (ctx) ABH_HIP(hipSetDevice(ctx->device));
     f();

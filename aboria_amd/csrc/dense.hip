@@ -714,7 +714,6 @@ bool fine_part(abh_context *ctx) {
     ctx->dense_fine.ensure_exact(kNoAllocScratchDoubles * 8);
   } catch (const abh::Error &e) {
     if (e.status != ABH_ERR_OUT_OF_MEMORY) throw;
-    (void)hipGetLastError();
     return false;
   }
   return true;
@@ -889,7 +888,6 @@ abh_status abh_dense_batch_create(abh_context *ctx, int dim, int nprob, const in
         op->part.ensure_exact(size_t(sums) * 8);
       } catch (const abh::Error &e) {  // no room: k_dense needs none
         if (e.status != ABH_ERR_OUT_OF_MEMORY) throw;
-        (void)hipGetLastError();
         op->sym = false;
       }
     }

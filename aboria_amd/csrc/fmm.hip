@@ -2125,7 +2125,6 @@ int few_limit(abh_fmm *f, int NC) {
       f->part.ensure_exact(sums * nrp + 64);
     } catch (const abh::Error &e) {  // no room: the sixteen-column form
       if (e.status != ABH_ERR_OUT_OF_MEMORY) throw;
-      (void)hipGetLastError();
       f->Wp.release();
       f->part.release();
       nrp = 0;

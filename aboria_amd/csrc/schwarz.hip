@@ -368,42 +368,50 @@ void analyse_batch_into(abh_schwarz *s, int D, const std::vector<int64_t> &boff,
   take(s, dm);
 }
 
-void drop_factor_buffers(abh_context *ctx) {
-  for (DevBuf *b : {&ctx->factor_a, &ctx->factor_d, &ctx->factor_ds, &ctx->factor_w,
-                    &ctx->factor_sg, &ctx->factor_spare})
-    b->release();
-}
-
-constexpr size_t kSpareMax = size_t(4) << 30;
-
 // R of at least `want` bytes: its own, the context's spare one if that is not
 // more than twice as large, or a new allocation.
 void take_inverse(abh_schwarz *s, size_t want) {
-  abh_context *ctx = s->ctx;
-  DevBuf &spare = ctx->factor_spare;
+  DevBuf &spare = s->ctx->factor_spare;
   if (s->R.bytes >= want) return;
   if (spare.bytes >= want && spare.bytes / 2 <= want) {
+    // (as a new allocation would be: not in use on any stream)
+    ABH_HIP(hipDeviceSynchronize());
     s->R.swap(spare);
     spare.release();
     return;
   }
-  try {
-    s->R.ensure_exact(want);
-  } catch (const abh::Error &e) {
-    if (e.status != ABH_ERR_OUT_OF_MEMORY) throw;
-    (void)hipGetLastError();
-    ABH_HIP(hipStreamSynchronize(ctx->stream));
-    drop_factor_buffers(ctx);
-    s->R.ensure_exact(want);
-  }
+  s->R.ensure_exact(want);
 }
 
-// gives R back to the context (nothing on its stream uses it any more)
+// gives R back to the context, unless no preconditioner can follow
 void give_inverse(abh_schwarz *s) {
   DevBuf &spare = s->ctx->factor_spare;
+  if (s->ctx->closed) return;
   if (s->coarse) give_inverse(s->coarse);
-  if (s->R.bytes <= kSpareMax && s->R.bytes > spare.bytes) s->R.swap(spare);
+  if (s->R.bytes <= abh::kSpareKeep && s->R.bytes > spare.bytes) s->R.swap(spare);
 }
+
+// The context's factorisation workspaces while one runs; afterwards they stay
+// unless a large domain made them larger than what is kept.
+struct FactorScope {
+  abh_context *ctx;
+  explicit FactorScope(abh_context *c) : ctx(c) { ctx->factor_busy = true; }
+  FactorScope(const FactorScope &) = delete;
+  FactorScope &operator=(const FactorScope &) = delete;
+  ~FactorScope() {
+    ctx->factor_busy = false;
+    if (ctx->factor_a.bytes + ctx->factor_d.bytes + ctx->factor_ds.bytes + ctx->factor_w.bytes +
+            ctx->factor_sg.bytes > abh::kFactorKeep)
+      release();
+  }
+  void release() {
+    for (DevBuf *b : {&ctx->factor_a, &ctx->factor_d, &ctx->factor_ds, &ctx->factor_w,
+                      &ctx->factor_sg})
+      b->release();
+  }
+};
+
+constexpr double kGroupBudget = 2.4e9;  // bytes of work memory a group may take
 
 // sgn: local matrices may be indefinite; factorise A = L S L^T (S = +-1)
 // instead of requiring positive pivots.
@@ -456,7 +464,7 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
       // 256, 57 in groups of 512, 53 in groups of 1,024 (2.7 GB).  A size's
       // domains are spread evenly over its groups.
       const double budget =
-          std::min(2.4e9, 0.35 * (double(free_b) + double(ctx->factor_a.bytes)));
+          std::min(kGroupBudget, 0.35 * (double(free_b) + double(abh::idle_bytes(ctx))));
       int gmax = int(std::max(1.0, std::min(4.0 * ctx->n_cu, budget / per)));
       int same = 0;
       while (i + same < nd && npad(order[i + same]) == n) ++same;
@@ -512,12 +520,25 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
   DevBuf &A = ctx->factor_a, &W = ctx->factor_w, &Dinv = ctx->factor_d;
   DevBuf &DinvS = ctx->factor_ds, &Sg = ctx->factor_sg;
   DevBuf fail;
-  A.ensure(a_size * 8);
-  Dinv.ensure(d_size * 8);
-  if (sgn) {
-    W.ensure(d_size * 8);
-    DinvS.ensure(d_size * 8);
-    Sg.ensure(s_size * 8);
+  FactorScope scope(ctx);
+  auto room = [](DevBuf &b, size_t want) {
+    if (double(want) > kGroupBudget) b.ensure_exact(want);  // one large domain
+    else b.ensure(want);
+  };
+  auto workspace = [&] {
+    room(A, a_size * 8);
+    room(Dinv, d_size * 8);
+    if (!sgn) return;
+    room(W, d_size * 8);
+    room(DinvS, d_size * 8);
+    room(Sg, s_size * 8);
+  };
+  try {
+    workspace();
+  } catch (const abh::Error &e) {  // room taken by buffers of another shape
+    if (e.status != ABH_ERR_OUT_OF_MEMORY) throw;
+    scope.release();
+    workspace();
   }
   fail.ensure(size_t(nd) + 64);
   ABH_HIP(hipMemsetAsync(fail.p, 0, size_t(nd), st));

@@ -1666,6 +1666,7 @@ abh_status abh_sparse_op_cache(abh_sparse_op *op, abh_precision precision, int e
                         (have ? 0 : size_t(op->nnz) * 4 + size_t(nq + 1) * 8);
     size_t free_b = 0, total_b = 0;
     ABH_HIP(hipMemGetInfo(&free_b, &total_b));
+    free_b += abh::idle_bytes(ctx);
     ABH_REQUIRE(double(need) <= 0.8 * double(free_b), ABH_ERR_OUT_OF_MEMORY,
                 "not enough device memory to cache the operator");
     op->c_rp.ensure(size_t(nq + 1) * 8);

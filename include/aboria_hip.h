@@ -53,6 +53,12 @@ typedef struct abh_context abh_context;
 abh_status abh_context_create(int device, void *stream, abh_context **out);
 abh_status abh_context_destroy(abh_context *ctx);
 abh_status abh_context_sync(abh_context *ctx);
+/* Frees the device memory that the context only keeps for later calls: the
+ * Schwarz set-up's work memory (at most 3 GiB) and the inverse of the last
+ * preconditioner destroyed (at most 4 GiB).  The library does this by itself
+ * when one of its allocations on this context finds no room; this is for a
+ * caller whose own allocator ran out.  Waits for the device. */
+abh_status abh_context_trim(abh_context *ctx);
 const char *abh_status_string(abh_status s);
 const char *abh_last_error(const abh_context *ctx);
 

@@ -49,6 +49,7 @@ class Context {
   Context &operator=(const Context &) = delete;
   abh_context *get() const { return h_; }
   void sync() const { check(abh_context_sync(h_), h_); }
+  void trim() const { check(abh_context_trim(h_), h_); }
 
   // owning device buffer of T
   template <class T> struct Buffer {
