@@ -33,7 +33,8 @@ constexpr int kRptOf[kVariants] = {1, 2, 4};
 // CU (300 problems of 200 to 3,000 points, 500 tiles: 0.58 ms, 0.36 one-sided
 // with one row per thread; 512 of 1,000 to 64,000, 7,700 tiles: 73.8 and
 // 118.7 ms) and its partial sums fit 1.25 GB (that batch needs 1.0).  The rule
-// looks at the sizes only, so a batch gives the same bits in every run.
+// looks at the sizes and the number of CUs, so a batch gives the same bits in
+// every run on a device with room for its partial sums.
 constexpr int kSymRpt = 4, kSymVariant = 2;
 constexpr int kSymTiles = 8;
 constexpr int64_t kSymPart = int64_t(5) << 25;
@@ -556,10 +557,9 @@ struct abh_dense_batch {
   const double *pos = nullptr;
   DevBuf tiles[kVariants], off, active;
   int ntiles[kVariants] = {0, 0, 0};
-  bool sym = false;  // the symmetric form, unless a tile shape was forced
+  bool sym = false;  // the symmetric form, unless another tile shape was set
   DevBuf poff, part;
-  int choice[2] = {-1, -1};        // tuned variant per precision (FP64, FP32c)
-  bool forced[2] = {false, false};
+  int choice[2] = {-1, -1};        // tuned or set variant per precision (FP64, FP32c)
   float tune_ms[2][kVariants] = {};
 
   template <int RPT>
@@ -641,11 +641,26 @@ struct abh_dense_batch {
     else launch<4>(v, x, y, fp32, alpha, overwrite, act);
   }
 
+  bool symmetric(bool fp32) const {
+    const int c = choice[fp32 ? 1 : 0];
+    return sym && (c < 0 || c == kSymVariant);
+  }
+
+  // Before an apply: picks the one-sided form's tile shape.  The symmetric
+  // form has one shape and nothing to time (512 problems of 1,000 to 64,000
+  // points: six one-sided products, 0.7 s).
+  void prepare(bool fp32) {
+    if (!symmetric(fp32)) tune(fp32);
+  }
+
   // Autotuner: times every variant once (after a warm-up) on the batch
-  // itself and keeps the fastest for this precision.
+  // itself and keeps the fastest for this precision; in the symmetric form
+  // times that alone.
   int tune(bool fp32) {
     const int pi = fp32 ? 1 : 0;
-    if (choice[pi] >= 0) return choice[pi];
+    const bool one = symmetric(fp32);
+    if (one ? tune_ms[pi][kSymVariant] > 0.0f : choice[pi] >= 0)
+      return one ? kSymVariant : choice[pi];
     const int64_t n = L.total();
     DevBuf xs, ys;
     xs.ensure(size_t(n) * 8 + 64);
@@ -655,11 +670,15 @@ struct abh_dense_batch {
     hipEvent_t e0, e1;
     ABH_HIP(hipEventCreate(&e0));
     ABH_HIP(hipEventCreate(&e1));
-    int best = 0;
-    for (int v = 0; v < kVariants; ++v) {
-      run(v, xs.as<double>(), ys.as<double>(), fp32, 1.0, true, nullptr);
+    auto product = [&](int v) {
+      if (one) run_sym(xs.as<double>(), ys.as<double>(), fp32, 1.0, true, nullptr);
+      else run(v, xs.as<double>(), ys.as<double>(), fp32, 1.0, true, nullptr);
+    };
+    int best = one ? kSymVariant : 0;
+    for (int v = best; v < (one ? kSymVariant + 1 : kVariants); ++v) {
+      product(v);
       ABH_HIP(hipEventRecord(e0, s));
-      run(v, xs.as<double>(), ys.as<double>(), fp32, 1.0, true, nullptr);
+      product(v);
       ABH_HIP(hipEventRecord(e1, s));
       ABH_HIP(hipEventSynchronize(e1));
       float ms = 0.0f;
@@ -669,15 +688,15 @@ struct abh_dense_batch {
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    choice[pi] = best;
+    if (!one) choice[pi] = best;
     return best;
   }
 
   void apply(const double *x, double *y, bool fp32, double alpha, bool overwrite,
              const uint8_t *act) {
-    const int v = tune(fp32);
-    if (sym && !forced[fp32 ? 1 : 0]) run_sym(x, y, fp32, alpha, overwrite, act);
-    else run(v, x, y, fp32, alpha, overwrite, act);
+    prepare(fp32);
+    if (symmetric(fp32)) run_sym(x, y, fp32, alpha, overwrite, act);
+    else run(choice[fp32 ? 1 : 0], x, y, fp32, alpha, overwrite, act);
   }
 };
 
@@ -977,8 +996,8 @@ abh_status abh_dense_batch_gmres_precond(abh_dense_batch *op, const abh_schwarz 
       abh::schwarz_apply(prec, in, out);
     };
     // tiles tuned before any graph capture (the tuner allocates and times)
-    op->tune(fp32);
-    op->tune(false);
+    op->prepare(fp32);
+    op->prepare(false);
     abh::GmresResult res;
     abh::batch_gmres(ctx, op->L, f_op, f_true, prec ? &f_prec : nullptr, b, x, *opts,
                      opts->graph != 0, res);
@@ -1033,8 +1052,8 @@ abh_status abh_dense_batch_refine(abh_dense_batch *op, const abh_schwarz *prec,
     abh::BatchPrec f_prec = [&](const double *in, double *out) {
       abh::schwarz_apply(prec, in, out);
     };
-    op->tune(fp32);
-    op->tune(false);
+    op->prepare(fp32);
+    op->prepare(false);
     const int ld = 2;
     DevBuf r, d, partial, hdev, sdev;
     r.ensure(size_t(n) * 8 + 64);
@@ -1127,7 +1146,6 @@ abh_status abh_dense_batch_tune(abh_dense_batch *op, abh_precision precision, in
         if (kRptOf[q] == *rows_per_thread) v = q;
       ABH_REQUIRE(v >= 0, ABH_ERR_INVALID_ARG, "rows_per_thread must be 1, 2 or 4");
       op->choice[fp32 ? 1 : 0] = v;
-      op->forced[fp32 ? 1 : 0] = true;
       return;
     }
     const int v = op->tune(fp32);

@@ -602,10 +602,13 @@ abh_status abh_dense_apply_noalloc(abh_context *ctx, int dim, int64_t nrows,
  * workgroup, each source staged in LDS serving 1, 2 or 4 rows per thread) on
  * this batch once and keeps the fastest for the precision; apply and gmres
  * tune on first use.  rows_per_thread (host, may be NULL) gets the choice,
- * variant_ms (host, 3 floats, may be NULL) the measured times.  A positive
- * *rows_per_thread on entry (1, 2 or 4) sets that shape instead of tuning.
- * Batches of many tiles use every kernel value for its row and its column
- * (a choice by the sizes alone) unless a shape is set. */
+ * variant_ms (host, 3 floats, may be NULL) the measured times, 0 for shapes
+ * not timed.  A positive *rows_per_thread on entry (1, 2 or 4) sets that
+ * shape instead of tuning.
+ * Batches of many tiles (a choice by the sizes) use every kernel value for its
+ * row and its column; that form has 4 rows per thread and is not tuned: the
+ * call reports 4 and its time alone, setting 4 keeps or restores it, setting
+ * 1 or 2 selects the one-sided form. */
 abh_status abh_dense_batch_tune(abh_dense_batch *op, abh_precision precision,
                                 int *rows_per_thread, float *variant_ms);
 

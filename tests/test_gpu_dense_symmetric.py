@@ -41,5 +41,12 @@ def test_symmetric_matches_one_sided(ctx, name, dim):
     if name == "multiquadric":  # no further off the double-double sums
         exact = -op.residual_dd(torch.zeros_like(x), x)
         assert (y - exact).norm() <= 1.02 * (ref - exact).norm()
+    # nothing was timed on the way: the tuner reports the symmetric form, whose
+    # shape passed back keeps it and restores it after another was set
+    rpt, ms = op.tune(ab.FP64)
+    assert rpt == 4 and ms[4] > 0 and ms[1] == 0 and ms[2] == 0
+    assert torch.equal(op.apply(x, torch.zeros_like(x)), y)
+    one.tune(ab.FP64, force=rpt)
+    assert torch.equal(one.apply(x, torch.zeros_like(x)), y)
     y32 = op.apply(x, torch.full_like(x, 0.25), ab.FP32_COMPENSATED) - 0.25
     assert torch.all((y32 - ref).abs() <= 2e-6 * scale + 2.0 ** -52)
