@@ -14,7 +14,9 @@
 // of lane l holds C[m = l % 16][n = l / 16 + 4 v] and the 16 lanes of a
 // group store 16 consecutive rows of a column (128 contiguous bytes).
 //
-// C may be A or B where a workgroup's tile reads only the rows or columns
+// lower_only skips the tiles that lie strictly above the diagonal (a
+// symmetric trailing update whose upper triangle is never read).  C may be A
+// or B where a workgroup's tile reads only the rows or columns
 // that it writes (one tile across the other dimension): all its loads come
 // before its stores.  In large batches all tiles of one matrix run on one XCD
 // (blocks go to the 8 XCDs round robin), whose L2 then holds the operand they
@@ -35,7 +37,8 @@ __global__ __launch_bounds__(256) void k_dgemm(int M, int N, int K, double alpha
                                                const double *A, int lda, int64_t sA,
                                                const double *B, int ldb, int64_t sB, double beta,
                                                double *C, int ldc, int64_t sC, int tiles_m,
-                                               int tiles, int batch, int xcds, int from_c) {
+                                               int tiles, int batch, int xcds, int from_c,
+                                               int lower_only) {
   __shared__ double As[kK][kLd];  // op(A)[m][k] stored [k][m]
   __shared__ double Bs[kK][kLd];  // op(B)[k][n] stored [k][n]
   const int q = int(blockIdx.x) / xcds;
@@ -43,6 +46,7 @@ __global__ __launch_bounds__(256) void k_dgemm(int M, int N, int K, double alpha
   if (g >= batch) return;  // uniform over the workgroup
   const int tm = (q % tiles) % tiles_m, tn = (q % tiles) / tiles_m;
   const int m0 = tm * kT, n0 = tn * kT;
+  if (lower_only && m0 + kT - 1 < n0) return;  // uniform over the workgroup
   A += int64_t(g) * sA;
   B += int64_t(g) * sB;
   C += int64_t(g) * sC;
@@ -155,7 +159,7 @@ namespace abh {
 void dgemm_strided_batched(hipStream_t st, bool ta, bool tb, int m, int n, int k, double alpha,
                            const double *A, int lda, int64_t sA, const double *B, int ldb,
                            int64_t sB, double beta, double *C, int ldc, int64_t sC, int batch,
-                           bool from_c) {
+                           bool from_c, bool lower_only) {
   if (m <= 0 || n <= 0 || batch <= 0) return;
   ABH_REQUIRE(k >= 0 && lda >= 1 && ldb >= 1 && ldc >= m, ABH_ERR_INVALID_ARG,
               "dgemm: bad leading dimension");
@@ -174,16 +178,20 @@ void dgemm_strided_batched(hipStream_t st, bool ta, bool tb, int m, int n, int k
   const dim3 grid{unsigned(blocks)};
   if (!ta && !tb)
     k_dgemm<false, false><<<grid, 256, 0, st>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                                                 ldc, sC, tm, tiles, batch, xcds, from_c);
+                                                 ldc, sC, tm, tiles, batch, xcds, from_c,
+                                                 lower_only);
   else if (!ta && tb)
     k_dgemm<false, true><<<grid, 256, 0, st>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                                                ldc, sC, tm, tiles, batch, xcds, from_c);
+                                                ldc, sC, tm, tiles, batch, xcds, from_c,
+                                                lower_only);
   else if (ta && !tb)
     k_dgemm<true, false><<<grid, 256, 0, st>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                                                ldc, sC, tm, tiles, batch, xcds, from_c);
+                                                ldc, sC, tm, tiles, batch, xcds, from_c,
+                                                lower_only);
   else
     k_dgemm<true, true><<<grid, 256, 0, st>>>(m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C,
-                                               ldc, sC, tm, tiles, batch, xcds, from_c);
+                                               ldc, sC, tm, tiles, batch, xcds, from_c,
+                                               lower_only);
   check_launch();
 }
 

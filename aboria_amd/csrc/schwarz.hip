@@ -9,21 +9,23 @@
 // A_g = K + shift I (identity in the padding) is assembled in HBM with the
 // domain's list reversed: entry j at matrix index n - 1 - j, so the padding
 // comes first and the interior last (the signed form below keeps the list's
-// order).  It is factorised by a left-looking
-// blocked Cholesky (64-wide panels: a block column takes all earlier ones in
-// one strided-batched FP64 MFMA GEMM, dgemm.hip, the diagonal block is
-// factorised and inverted by one wavefront, the panel multiplied by that
-// inverse in place), and the interior columns of A_g^-1 (= the interior
-// rows, A_g is symmetric) are obtained by a blocked forward and backward
-// substitution on the last unit columns: since the interior comes last, the
-// forward one touches the last block rows only.  They stay resident: R_g is
+// order).  It is factorised by a blocked Cholesky in panels of 512 columns (up
+// to 1,536, in one panel):
+// within a panel a 64-wide block column takes the panel's earlier ones in one
+// strided-batched FP64 MFMA GEMM (dgemm.hip), its diagonal block is factorised
+// and inverted by one wavefront, the rows below multiplied by that inverse in
+// place; a finished panel updates what lies right of it.  The interior
+// columns of A_g^-1 (= the interior rows, A_g is symmetric) are obtained by a
+// blocked forward and backward substitution on the last unit columns: since
+// the interior comes last, the forward one touches the last block rows only,
+// and of those the columns that are not zero yet.  They stay resident: R_g is
 // n x ni column-major, so row a of the local inverse is the contiguous column
 // ni - 1 - a, backwards (signed: column a).
 // 400,056 points, 6,256 domains of 576 (the whole set-up and solve, 113 ms
 // before): diagonal blocks 36.9 -> 6.5 ms (256 threads and three barriers
-// per column before), products 48.6 -> 22.9 ms, copies 6.2 -> 0 ms; with
-// right-looking updates every trailing tile was read and written once per
-// panel, which HBM bounded.
+// per column before), products 48.6 -> 22.9 ms, copies 6.2 -> 0 ms; with an
+// update of the whole trailing matrix per block column every trailing tile was
+// read and written once for each, which HBM bounded.
 //
 // For the dense batch (every problem an independent particle set) the
 // domains come from a per-problem bucket grid instead of a cell list, the
@@ -411,7 +413,32 @@ struct FactorScope {
   }
 };
 
-constexpr double kGroupBudget = 2.4e9;  // bytes of work memory a group may take
+// Bytes of work memory a group of domains may take.  Up to kGroupBudget the
+// context keeps it.  Domains of which that holds fewer than kFewMembers leave
+// the chip idle in the diagonal blocks and in the products of few tiles and
+// get more, which is freed again: 400 domains of up to 4,654 take 715 ms in
+// groups of 13 and 517 in groups of 40, 49 of up to 11,192 (not all in full
+// groups) 2,181 ms in groups of 2 and about 960 in groups of 7, with the
+// panels of kPanel in place of whole columns in the latter.
+constexpr double kGroupBudget = 2.4e9, kLargeBudget = 8.0e9;
+constexpr int kFewMembers = 16;
+// Columns per panel of the factorisation: within a panel a block column takes
+// the panel's earlier ones (left-looking), a finished panel updates everything
+// right of it at once.  One panel (left-looking throughout) leaves a block
+// column of a few large matrices few tiles with long sums; panels of 64
+// (right-looking) read and write the trailing matrix for every block column.
+// Columns per panel 64 / 256 / 512 / 1,024 / all, ms: one domain of 20,500 546
+// / 485 / 484 / 487 / 609, 400 of up to 4,654 746 / 520 / 517 / 497 / -, 961
+// of up to 1,986 187 / 142 / 140 / 142 / 145, 3,025 of up to 685 31.0 / 26.5 /
+// 26.4 / 26.3 / 26.5.  Matrices of up to three panels come in large groups and
+// are one panel: in the signed form, which copies and scales an update's
+// right factor, 8,192 domains of up to 1,193 take 210 ms in panels of 512
+// and 199 in one.  The bits are the same in all of them: every element's sum
+// starts from the element and takes its terms in one order.
+constexpr int kPanel = 512;
+int panel_of(int n) { return n <= 3 * kPanel ? n : kPanel; }
+// rows of L times columns in the largest copy of a right factor
+int64_t panel_copy(int n) { return int64_t(n) * (panel_of(n) < n ? kPanel : kNb); }
 
 // sgn: local matrices may be indefinite; factorise A = L S L^T (S = +-1)
 // instead of requiring positive pivots.
@@ -456,15 +483,16 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
     while (i < nd) {
       const int n = npad(order[i]);
       // working set per member: A (n^2) + dinv (64 n) (+ S L^-1, the scaled
-      // block row and the signs in signed mode)
-      const double per = double(n) * n * 8.0 + double(n) * kNb * (sgn ? 24.0 : 8.0) +
-                         (sgn ? double(n) * 8.0 : 0.0);
+      // rows of a panel and the signs in signed mode)
+      const double per = double(n) * n * 8.0 + double(n) * kNb * 8.0 +
+                         (sgn ? 8.0 * (double(n) * (kNb + 1) + double(panel_copy(n))) : 0.0);
       // Large groups fill the chip with diagonal blocks and panels (at most a
       // wavefront per SIMD): 6,256 domains of 576 take 69 ms in groups of
       // 256, 57 in groups of 512, 53 in groups of 1,024 (2.7 GB).  A size's
       // domains are spread evenly over its groups.
+      const double room_b = 0.35 * (double(free_b) + double(abh::idle_bytes(ctx)));
       const double budget =
-          std::min(kGroupBudget, 0.35 * (double(free_b) + double(abh::idle_bytes(ctx))));
+          std::min(per * kFewMembers > kGroupBudget ? kLargeBudget : kGroupBudget, room_b);
       int gmax = int(std::max(1.0, std::min(4.0 * ctx->n_cu, budget / per)));
       int same = 0;
       while (i + same < nd && npad(order[i + same]) == n) ++same;
@@ -511,25 +539,26 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
                          hipMemcpyHostToDevice, st));
   using abh::dgemm_strided_batched;
 
-  size_t a_size = 0, d_size = 0, s_size = 0;
+  size_t a_size = 0, d_size = 0, s_size = 0, w_size = 0;
   for (const Group &gr : groups) {
     a_size = std::max(a_size, size_t(gr.count) * gr.n * gr.n);
     d_size = std::max(d_size, size_t(gr.count) * gr.n * kNb);
     s_size = std::max(s_size, size_t(gr.count) * gr.n);
+    w_size = std::max(w_size, size_t(gr.count) * size_t(panel_copy(gr.n)));
   }
   DevBuf &A = ctx->factor_a, &W = ctx->factor_w, &Dinv = ctx->factor_d;
   DevBuf &DinvS = ctx->factor_ds, &Sg = ctx->factor_sg;
   DevBuf fail;
   FactorScope scope(ctx);
   auto room = [](DevBuf &b, size_t want) {
-    if (double(want) > kGroupBudget) b.ensure_exact(want);  // one large domain
+    if (double(want) > kGroupBudget) b.ensure_exact(want);  // freed afterwards
     else b.ensure(want);
   };
   auto workspace = [&] {
     room(A, a_size * 8);
     room(Dinv, d_size * 8);
     if (!sgn) return;
-    room(W, d_size * 8);
+    room(W, w_size * 8);
     room(DinvS, d_size * 8);
     room(Sg, s_size * 8);
   };
@@ -548,7 +577,6 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
     const int G = gr.count, n = gr.n, ni = gr.ni, K = n / kNb;
     const int64_t sA = int64_t(n) * n;
     const int64_t sD = int64_t(K) * kNb * kNb;
-    const int64_t sW = int64_t(n) * kNb;
     const int64_t sY = int64_t(n) * ni;
     double *Ap = A.as<double>(), *Wp = W.as<double>();
     double *Dp = Dinv.as<double>();
@@ -566,23 +594,32 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
       abh::check_launch();
     }
     // blocked Cholesky, lower (signed: A = L S L^T), one block column after
-    // the other
+    // the other.  C = A[row:, col:col+cols] takes the columns from..to of L:
+    // C -= L[row:, from:to] (S) L[col:col+cols, from:to]^T
+    const int64_t sW = panel_copy(n);
+    const int panel = panel_of(n);
+    auto update = [&](int row, int cols, int from, int to, bool lower) {
+      const double *B = Ap + row + int64_t(from) * n;
+      int ldb = n;
+      int64_t sB = sA;
+      if (sgn) {
+        dim3 grid(unsigned(abh::ceil_div(int64_t(cols) * (to - from), 256)), G);
+        k_copy_block<<<grid, 256, 0, st>>>(B, sA, n, Wp, sW, cols, cols, to - from, Sp + from, n);
+        abh::check_launch();
+        B = Wp;
+        ldb = cols;
+        sB = sW;
+      }
+      dgemm_strided_batched(st, false, true, n - row, cols, to - from, -1.0,
+                            Ap + row + int64_t(from) * n, n, sA, B, ldb, sB, 1.0,
+                            Ap + row + int64_t(row) * n, n, sA, G, true, lower);
+    };
     for (int kb = 0; kb < K; ++kb) {
       const int o = kb * kNb;
       const int r = n - o - kNb;
+      const int p0 = o / panel * panel;      // the panel's first column
       double *Ck = Ap + o + int64_t(o) * n;  // A[o:, o:o+64]
-      if (kb > 0) {
-        // A[o:, o:o+64] -= A[o:, :o] (S) A[o:o+64, :o]^T
-        const double *Bk = Ap + o;
-        if (sgn) {
-          dim3 grid(unsigned(abh::ceil_div(int64_t(kNb) * o, 256)), G);
-          k_copy_block<<<grid, 256, 0, st>>>(Ap + o, sA, n, Wp, sW, kNb, kNb, o, Sp, n);
-          abh::check_launch();
-          Bk = Wp;
-        }
-        dgemm_strided_batched(st, false, true, n - o, kNb, o, -1.0, Ap + o, n, sA, Bk,
-                              sgn ? kNb : n, sgn ? sW : sA, 1.0, Ck, n, sA, G, true);
-      }
+      if (o > p0) update(o, kNb, p0, o, false);
       k_potrf_diag<<<G, 64, 0, st>>>(Ap, n, o, Dp + int64_t(kb) * kNb * kNb, sD, fl, sgn ? 1 : 0,
                                      Sp, n, DSp + int64_t(kb) * kNb * kNb);
       abh::check_launch();
@@ -590,6 +627,7 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
       if (r > 0)
         dgemm_strided_batched(st, false, true, r, kNb, kNb, 1.0, Ck + kNb, n, sA,
                               DSp + int64_t(kb) * kNb * kNb, kNb, sD, 0.0, Ck + kNb, n, sA, G);
+      if (r > 0 && (o + kNb) % panel == 0) update(o + kNb, r, p0, o + kNb, true);
     }
     // Y = L^-1 E (E = the interior's unit columns, the last ni or the first):
     // rows before the block of the first unit stay zero, and so do columns of
@@ -601,7 +639,7 @@ void factorise(abh_schwarz *s, const double *pos, const KernelDesc &k, double r2
     }
     for (int kb = rev ? (n - ni) / kNb : 0; kb < K; ++kb) {
       const int o = kb * kNb;
-      const int nc = rev ? ni : std::min(ni, o + kNb);
+      const int nc = std::min(ni, o + kNb - (rev ? n - ni : 0));
       // in place, like every product with a diagonal block's inverse
       dgemm_strided_batched(st, false, false, kNb, nc, kNb, 1.0, Dp + int64_t(kb) * kNb * kNb,
                             kNb, sD, Y + o, n, sY, 0.0, Y + o, n, sY, G);

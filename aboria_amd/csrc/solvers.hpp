@@ -32,13 +32,14 @@ abh_schwarz *schwarz_create_batch(abh_context *ctx, int dim, const std::vector<i
 // Strided-batched FP64 GEMM on the matrix cores, column-major
 // (dgemm.hip): C[g] = alpha op(A[g]) op(B[g]) + beta C[g] for g < batch;
 // beta == 0 does not read C.  from_c (alpha 1 or -1): the sums start from
-// beta C / alpha instead of joining it at the end.  C may be A when n <= 64, or B when m <= 64, with
-// the same leading dimension and stride, k no larger than that dimension.
-// Enqueued on st; throws abh::Error.
+// beta C / alpha instead of joining it at the end.  lower_only skips the
+// 64 x 64 tiles of C that lie strictly above its diagonal.  C may be A when
+// n <= 64, or B when m <= 64, with the same leading dimension and stride, k no
+// larger than that dimension.  Enqueued on st; throws abh::Error.
 void dgemm_strided_batched(hipStream_t st, bool ta, bool tb, int m, int n, int k, double alpha,
                            const double *A, int lda, int64_t sA, const double *B, int ldb,
                            int64_t sB, double beta, double *C, int ldc, int64_t sC, int batch,
-                           bool from_c = false);
+                           bool from_c = false, bool lower_only = false);
 
 // x = W b with W the approximate-inverse rows (learned.hip).
 void ainv_apply(const abh_ainv *a, const double *b, double *x);

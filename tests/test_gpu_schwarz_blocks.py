@@ -56,3 +56,25 @@ def test_domains_against_dense_solves(ctx, dim, n, leaf):
             err = np.abs(x[i[:nint[d]]] - ref[:nint[d]]).max()
             assert err <= 8 * len(i) * 2.0 ** -52 * np.linalg.cond(a) * np.linalg.norm(ref)
         del sw
+
+
+@pytest.mark.parametrize("n", [511, 577, 1_024, 1_536, 1_537, 2_048, 2_049, 2_111])
+def test_panel_sizes(ctx, n):
+    """One domain of one 512-column panel of the factorisation and of several, in
+    the Cholesky form and in the signed form of a batch.  Bound as above."""
+    print("panel", n, flush=True)
+    rng = np.random.default_rng(n)
+    pos, b = rng.random((n, 2)), rng.standard_normal(n)
+    cl = cells(ctx, pos, 4.0 * n)
+    batch = ab.DenseBatchOperator(ctx, [0, n], torch.tensor(pos, device="cuda"),
+                                  ab.Kernel.gaussian(0.05))
+    for p, sw in ((cl.positions().cpu().numpy(),
+                   ab.SchwartzPreconditioner(ctx, cl, ab.Kernel.gaussian(0.05), 0.0, 0.1)),
+                  (pos, ab.SchwartzPreconditioner.for_dense_batch(
+                      batch, [0.0] * 2, [1.0] * 2, 4.0 * n, 0.1))):
+        assert sw.info["n_domains"] == 1 and sw.info["failed_domains"] == 0
+        a = np.exp(-((p[:, None] - p[None]) ** 2).sum(-1) / 0.05 ** 2) + 0.1 * np.eye(n)
+        x = sw.solve(torch.tensor(b, device="cuda")).cpu().numpy()
+        ref = np.linalg.solve(a, b)
+        bound = 8 * n * 2.0 ** -52 * np.linalg.cond(a) * np.linalg.norm(ref)
+        assert np.linalg.norm(x - ref) <= bound
