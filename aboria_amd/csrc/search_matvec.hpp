@@ -13,9 +13,14 @@
 // sides is a template argument and a block serves one work item, which keeps
 // the grid's and the kernel's parameters out of the loops (the compiler had
 // moved 180 scalar registers into vector lanes and read 16 of them back in
-// every round).
-// 4M-particle mixture, Wendland, eight right-hand sides: 38.2 -> 25.1 ms;
-// one: 25.7 -> 20.8 ms.
+// every round).  The tests and the rounds are compiled with and without
+// periodic images (the rounds also for buckets visited more than once): chosen
+// at run time, the choice was a branch in every test and round, which kept their
+// dependent chains from overlapping.  An item of a crowded cell, alone on its
+// SIMD, then took twice as long as one candidate block after another had.
+// 4M-particle mixture, Wendland, eight right-hand sides: 38.2 -> 25.1 ms, now
+// 21.5; one: 25.7 -> 20.8, 17.4 ms.  1,000,000 points at 60 a cell, Gaussian, one
+// right-hand side: 3.40 -> 2.04, 1.69 ms.
 
 constexpr int kMix = 4;
 
@@ -160,7 +165,7 @@ __global__ __launch_bounds__(kGroup) __attribute__((amdgpu_waves_per_eu(3))) voi
   // (28.9 ms): what is left is that evaluation's own rounding.  One running
   // sum per row is 1.9e-15 off (1.4e-15 when it runs in bucket order, close to
   // the plain evaluation's order).
-  auto eval = [&](auto profile) {
+  auto eval = [&](auto profile, auto plain) {
     double part[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) part[r] = 0.0;
@@ -173,16 +178,17 @@ __global__ __launch_bounds__(kGroup) __attribute__((amdgpu_waves_per_eu(3))) voi
       load_stage(st[t], e1, j1);
       T x[NR];
       Pool::load(xs, t, x);
-      const int pinfo = images || multi ? st[t].pad : 0;
+      const int pinfo = decltype(plain)::value ? 0 : st[t].pad;
       double acc = 0.0;
 #pragma unroll
       for (int d = 0; d < D; ++d) {
-        const double dx = e1[d] - centre(pinfo >> 16, d);
+        const double dx = e1[d] - (decltype(plain)::value ? q[d] : centre(pinfo >> 16, d));
         acc = acc + dx * dx;
       }
       double w = wrow;
       if (a.k.col_s) w = w + a.k.wc * a.k.col_s[j1];
-      const int m = multi ? int(mult[(pinfo & 0xffff) * kGroup + lane]) : 1;
+      const int m = !decltype(plain)::value && multi
+                        ? int(mult[(pinfo & 0xffff) * kGroup + lane]) : 1;
       if constexpr (FP32) {
         const float fv = abh::phi32t<decltype(profile)::value>(a.k, float(acc)) * float(w);
         for (int rep = 0; rep < m; ++rep)
@@ -235,13 +241,17 @@ __global__ __launch_bounds__(kGroup) __attribute__((amdgpu_waves_per_eu(3))) voi
     if (km == 0 && !last) continue;
     const int nk = __popcll(km);
     if (np + nk > kGroup || last) {
-      switch (a.k.type) {
-        case ABH_KERNEL_CONSTANT: eval(Profile<ABH_KERNEL_CONSTANT>{}); break;
-        case ABH_KERNEL_GAUSSIAN: eval(Profile<ABH_KERNEL_GAUSSIAN>{}); break;
-        case ABH_KERNEL_WENDLAND_C2: eval(Profile<ABH_KERNEL_WENDLAND_C2>{}); break;
-        case ABH_KERNEL_MULTIQUADRIC: eval(Profile<ABH_KERNEL_MULTIQUADRIC>{}); break;
-        case ABH_KERNEL_SMOOTH_INV_R: eval(Profile<ABH_KERNEL_SMOOTH_INV_R>{}); break;
-      }
+      auto evals = [&](auto plain) {
+        switch (a.k.type) {
+          case ABH_KERNEL_CONSTANT: eval(Profile<ABH_KERNEL_CONSTANT>{}, plain); break;
+          case ABH_KERNEL_GAUSSIAN: eval(Profile<ABH_KERNEL_GAUSSIAN>{}, plain); break;
+          case ABH_KERNEL_WENDLAND_C2: eval(Profile<ABH_KERNEL_WENDLAND_C2>{}, plain); break;
+          case ABH_KERNEL_MULTIQUADRIC: eval(Profile<ABH_KERNEL_MULTIQUADRIC>{}, plain); break;
+          case ABH_KERNEL_SMOOTH_INV_R: eval(Profile<ABH_KERNEL_SMOOTH_INV_R>{}, plain); break;
+        }
+      };
+      if (images || multi) evals(std::false_type{});
+      else evals(std::true_type{});
       if (last) break;
       np = 0;
       __syncthreads();  // the next block overwrites the pool
@@ -260,30 +270,36 @@ __global__ __launch_bounds__(kGroup) __attribute__((amdgpu_waves_per_eu(3))) voi
     __syncthreads();  // single-wave group: the pooled block is complete
     // radius tests of the new candidates; a lane that does not visit a
     // candidate's bucket has no hit there
-    auto test = [&](int t) {
-      double e[3];
-      int j;
-      load_stage(st[t], e, j);
-      const int pinfo = abh::uniform_i32(st[t].pad);
-      const int mv = mult[(pinfo & 0xffff) * kGroup + lane];
-      double acc = 0.0;
+    auto tests = [&](auto img) {
+      auto test = [&](int t) {
+        double e[3];
+        int j;
+        load_stage(st[t], e, j);
+        const int pinfo = abh::uniform_i32(st[t].pad);
+        const int mv = mult[(pinfo & 0xffff) * kGroup + lane];
+        double acc = 0.0;
 #pragma unroll
-      for (int d = 0; d < D; ++d) {
-        const double dx = e[d] - centre(pinfo >> 16, d);
-        acc = acc + dx * dx;
+        for (int d = 0; d < D; ++d) {
+          const double dx =
+              e[d] - (decltype(img)::value ? image_of((pinfo >> (16 + 2 * d)) & 3, q[d], L[d])
+                                           : q[d]);
+          acc = acc + dx * dx;
+        }
+        return acc <= a.r2 && mv != 0;
+      };
+      int t = np;
+      np += nk;
+      for (; t + kStageUnroll <= np; t += kStageUnroll) {
+        bool h[kStageUnroll];
+#pragma unroll
+        for (int u = 0; u < kStageUnroll; ++u) h[u] = test(t + u);
+#pragma unroll
+        for (int u = 0; u < kStageUnroll; ++u) hm = (hm << 1) + (h[u] ? 1ull : 0ull);
       }
-      return acc <= a.r2 && mv != 0;
+      for (; t < np; ++t) hm = (hm << 1) + (test(t) ? 1ull : 0ull);
     };
-    int t = np;
-    np += nk;
-    for (; t + kStageUnroll <= np; t += kStageUnroll) {
-      bool h[kStageUnroll];
-#pragma unroll
-      for (int u = 0; u < kStageUnroll; ++u) h[u] = test(t + u);
-#pragma unroll
-      for (int u = 0; u < kStageUnroll; ++u) hm = (hm << 1) + (h[u] ? 1ull : 0ull);
-    }
-    for (; t < np; ++t) hm = (hm << 1) + (test(t) ? 1ull : 0ull);
+    if (images) tests(std::true_type{});
+    else tests(std::false_type{});
   }
   if (!has_row) return;
 #pragma unroll
