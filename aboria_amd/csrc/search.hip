@@ -50,7 +50,13 @@ constexpr int kGroup = 64;  // queries per work item = lanes per wave
 //  - otherwise the cells with kHeavyMin queries and more have work items: the
 //    4M-particle mixture takes 16.6 ms (search) and 24.6 (operator, eight
 //    right-hand sides) with 8, 16.4 and 25.1 with 12, 16.6 and 25.7 with 16.
+//    In cells of many queries the last few have one too: they would walk their
+//    long candidate lists alone before the work items start (100,000 points at
+//    300 a cell: fill 1,088 us, now 732, operator 3,038 and 1,334; the mixture's
+//    operator 21.5 and 19.7 ms).  For lists from 128 queries on: 1,000,000
+//    points at 60 a cell take 1,262 us to fill from 64 on, 1,195 from 128 on.
 constexpr int kHeavyMin = 12;
+constexpr int kCrowdedSearch = 128, kCrowdedOp = kGroup;
 constexpr double kLightSearch = 40.0;  // mean occupancy a particle sees, list passes
 constexpr double kLightOp = 13.0;      // the same for an operator's plan
 constexpr int64_t kSmall = 16384;      // particle sets that k_search_group always serves
@@ -128,9 +134,9 @@ __global__ __launch_bounds__(kThreads) void k_home_keys(const double *__restrict
 }
 
 // Runs of equal home cell (the key without its sub-cell bits) cut into work.
-// A run's whole groups of 64, and a remainder of at least heavy_min queries,
-// become work items of k_search; the queries of a smaller remainder go to the
-// list that k_search_group serves.  One thread per run (its first query),
+// A run's whole groups of 64, and a remainder of at least heavy_min queries or
+// of a run of at least `crowded`, become work items of k_search; the queries of
+// another remainder go to the list that k_search_group serves.  One thread per run (its first query),
 // which finds the run's end by doubling steps and a binary search; a block of
 // 1,024 takes its places in both lists with one atomic each (one per
 // wavefront: 0.65 ms at 4,000,000 queries, now 0.061 ms), so the lists stay
@@ -142,6 +148,7 @@ constexpr int kPlanThreads = 1024;
 template <int D>
 __global__ __launch_bounds__(kPlanThreads) void k_plan_items(const uint32_t *__restrict__ keys,
                                                          int64_t n, int shift, int heavy_min,
+                                                         int crowded,
                                                          const double *__restrict__ q_sorted,
                                                          GridParams g, WorkItem *__restrict__ work,
                                                          int32_t *__restrict__ light,
@@ -164,8 +171,9 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_items(const uint32_t *__r
     ++e;
     const int64_t c = e - k;
     const int rem = int(c % kGroup);
-    nw = uint32_t(c / kGroup) + (rem >= heavy_min ? 1u : 0u);
-    nl = rem < heavy_min ? uint32_t(rem) : 0u;
+    const bool list = rem < heavy_min && c < crowded;
+    nw = uint32_t(c / kGroup) + (rem > 0 && !list ? 1u : 0u);
+    nl = list ? uint32_t(rem) : 0u;
   }
   const uint32_t iw = abh::wave_incl_scan(nw), il = abh::wave_incl_scan(nl);
   const int wave = threadIdx.x >> 6;
@@ -1031,7 +1039,7 @@ struct QueryPlan {
   // every query goes to k_search_group, in the order given (no sort and no
   // work lists); otherwise the two lists of k_plan_items
   bool all_light = false;
-  double light_most = kLightSearch;
+  bool op = false;     // an operator's plan
   bool group = false;  // k_search_group serves some of the queries
   double radius = 0, r2 = 0;
   int w[3] = {0, 0, 0};
@@ -1103,11 +1111,13 @@ template <int D> static void plan_items(QueryPlan &p) {
   uint32_t *ctr = p.counters.as<uint32_t>();  // [0] = listed queries, [1] = work items
   ABH_HIP(hipMemsetAsync(ctr, 0, 8, ctx->stream));
   k_plan_items<D><<<unsigned(ceil_div(n, kPlanThreads)), kPlanThreads, 0, ctx->stream>>>(
-      p.keys.as<uint32_t>(), n, p.sub_levels * D, p.group ? kHeavyMin : 1, p.q_sorted,
-      p.cells->params(), p.work.as<WorkItem>(), p.light.as<int32_t>(), ctr);
+      p.keys.as<uint32_t>(), n, p.sub_levels * D, p.group ? kHeavyMin : 1,
+      p.op ? kCrowdedOp : kCrowdedSearch, p.q_sorted, p.cells->params(), p.work.as<WorkItem>(),
+      p.light.as<int32_t>(), ctr);
   check_launch();
-  // every item holds kHeavyMin queries; without the list there may be as many
-  // items as queries, and it pays to wait for their number
+  // every item holds kHeavyMin queries, or is the last of at least two of a
+  // run of 64 and more; without the list there may be as many items as queries,
+  // and it pays to wait for their number
   p.max_work = n / kHeavyMin;
   if (!p.group) {
     uint32_t h = 0;
@@ -1139,7 +1149,7 @@ template <int D> static void build_plan_d(QueryPlan &p, const double *q) {
   // 4 million random centres, 8 particles a cell in 3D: search 2.24 and
   // 7.76 ms sorted, 1.33 and 6.63 ms as they come).  The plan keeps a copy of
   // the centres.
-  p.all_light = p.group && cells_light(p.cells, p.light_most);
+  p.all_light = p.group && cells_light(p.cells, p.op ? kLightOp : kLightSearch);
   if (p.all_light) {
     ABH_HIP(hipMemsetAsync(p.counters.p, 0, 8, s));
     p.sub_levels = 0;
@@ -1549,7 +1559,7 @@ abh_status abh_sparse_op_create(abh_context *ctx, const abh_cells *cols, int64_t
     ABH_REQUIRE(!ctx->closed, ABH_ERR_INVALID_ARG, "context already destroyed");
     ABH_REQUIRE(kernel->type >= ABH_KERNEL_CONSTANT && kernel->type <= ABH_KERNEL_SMOOTH_INV_R,
                 ABH_ERR_UNSUPPORTED, "unknown kernel type");
-    op->plan.light_most = kLightOp;
+    op->plan.op = true;
     abh::build_plan(op->plan, ctx, cols, nrows, row_pos, radius);
     op->ncols = cols->n_alive;
     op->k.type = kernel->type;

@@ -47,6 +47,13 @@ CASES = [
 ]
 
 
+# Runs of 100 to 160 and of 64 to 70 queries: their last few.
+CASES += [
+    ("uniform", 17_003, 2, False, 130.0, 0.5, 0),
+    ("uniform", 17_003, 3, True, 65.0, 0.6, 0),
+]
+
+
 @pytest.mark.parametrize("case", CASES, ids=["%s-%d-%dd-%s-%g-%g-%d" % c for c in CASES])
 def test_routes(ctx, case):
     kind, n, dim, per, n_leaf, cells_r, other = case
