@@ -40,14 +40,25 @@ constexpr int kThreads = 256;
 constexpr int kMaxSlots = 343;
 constexpr int kGroup = 64;  // queries per work item = lanes per wave
 // Which queries get a wavefront per home cell (k_search, k_matvec) and which
-// eight lanes each (k_search_group).  Measured with a radius of 0.95 cells,
-// search (build, count and fill) and one application of the operator:
-//  - where all cells hold few particles every query is served by
-//    k_search_group, without sorting: at 32 a cell 1,000,000 points in 3D take
-//    2.50 ms (2.52 with work items), at 64 4.04 (2.77); 100,000 0.51 (0.65)
-//    and 0.67 (0.91).  A wave per cell applies the operator faster from about
-//    12 on: at 8 a cell 1.23 ms (1.32), at 16 2.12 (1.70).
-//  - otherwise the cells with kHeavyMin queries and more have work items: the
+// eight lanes each (k_search_group).  Measured in 3D with a radius of 0.95
+// cells; lists: count and fill with the plan, operator: one application.
+//  - Particles searched against themselves, in cells that hold few particles:
+//    every query is served by k_search_group, without sorting.  Lists of
+//    1,000,000 points at 30 a cell 2.21 ms (2.32 with work items), at 40 2.66
+//    (2.08); 100,000 at 40 0.37 (0.58).  A wave per cell applies the operator
+//    faster from about 10 on: 1,000,000 points at 8 a cell 1.29 ms (1.32), at 13
+//    1.83 (1.47), at 16 2.26 (1.42); 100,000 at 13 0.227 (0.233), at 20 0.300
+//    (0.268).
+//  - Other centres: what counts besides is how many of them share a cell, and
+//    whether the tests are enough to pay for the plan.  Lists (us, eight lanes /
+//    work items) over 300,000 particles at 20 a cell: 20 centres a cell 611 /
+//    1,043, 40 1,109 / 1,090, 64 1,744 / 1,211.  20,000 particles at 20 a cell:
+//    200 centres a cell (146,000, 8e7 tests) 388 / 442, 1,000 a cell (729,000)
+//    1,512 / 843; at 400 a cell 27,000 centres 1,412 / 1,493.  Operator: 300,000
+//    particles at 20 a cell, 10 centres a cell 435 / 470, 20 823 / 519, 40 1,605
+//    / 461; 20,000 at 5 a cell, 20 centres a cell 76 / 124, 40 127 / 88, 200 555
+//    / 204.
+//  - Otherwise the cells with kHeavyMin queries and more have work items: the
 //    4M-particle mixture takes 16.6 ms (search) and 24.6 (operator, eight
 //    right-hand sides) with 8, 16.4 and 25.1 with 12, 16.6 and 25.7 with 16.
 //    In cells of many queries the last few have one too: they would walk their
@@ -59,7 +70,13 @@ constexpr int kHeavyMin = 12;
 constexpr int kCrowdedSearch = 128, kCrowdedOp = kGroup;
 constexpr double kLightSearch = 40.0;  // mean occupancy a particle sees, list passes
 constexpr double kLightOp = 13.0;      // the same for an operator's plan
-constexpr int64_t kSmall = 16384;      // particle sets that k_search_group always serves
+constexpr double kSharedSearch = 40.0, kSharedOp = 20.0;  // centres a centre sees in its cell
+constexpr int64_t kSmall = 16384;  // this few queries over as few particles: always light
+// Operators: 16,000 points in one bucket (r = 0.2, 2D) take 2.12 ms with eight
+// lanes, 1.25 with work items; 10,000 (r = 0.05, 3D) 0.27 and 0.48.
+constexpr int64_t kSmallOp = 12288;
+constexpr int64_t kFewCentres = 32768;                // lists: half a wave per SIMD as items
+constexpr double kFewTests = 2e8, kFewTestsOp = 3e7;  // tests that a plan does not pay for
 
 struct WorkItem {
   int32_t home[3];
@@ -211,6 +228,55 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_items(const uint32_t *__r
     }
   }
   for (uint32_t c = 0; c < nl; ++c) light[bl + c] = int32_t(at + c);
+}
+
+// Pairs of equal home cells among kSample centres (chosen by a hash of their
+// number, so that no regular order of the centres shows), into *pairs: one
+// block counts the sample's cells in a hash table in LDS.
+constexpr int kSample = 2048;
+constexpr int kSampleSlots = 4 * kSample;  // a quarter full at most: a probe ends
+__device__ __forceinline__ uint32_t mix32(uint32_t h) {
+  h = (h ^ (h >> 16)) * 0x85ebca6bu;
+  h = (h ^ (h >> 13)) * 0xc2b2ae35u;
+  return h ^ (h >> 16);
+}
+template <int D>
+__global__ __launch_bounds__(1024) void k_shared_cells(const double *__restrict__ q, int64_t n,
+                                                       GridParams g, uint32_t *__restrict__ pairs) {
+  __shared__ uint32_t keys[kSampleSlots], counts[kSampleSlots], sums[16];
+  for (int i = threadIdx.x; i < kSampleSlots; i += 1024) {
+    keys[i] = 0xffffffffu;
+    counts[i] = 0;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kSample; i += 1024) {
+    const int64_t j = int64_t((uint64_t(mix32(uint32_t(i) + 1u)) * uint64_t(n)) >> 32);
+    double p[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) p[d] = q[j * D + d];
+    uint32_t key = 0;
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      key = key * uint32_t(home_span(g, d)) + uint32_t(home_of<D>(g, p, d) - home_lo(g, d));
+    // (the largest key shares the free slots' mark: its pairs are still counted)
+    uint32_t slot = mix32(key) % kSampleSlots;
+    for (int probe = 0; probe < kSampleSlots; ++probe) {
+      const uint32_t was = atomicCAS(&keys[slot], 0xffffffffu, key);
+      if (was == 0xffffffffu || was == key) break;
+      slot = (slot + 1) % kSampleSlots;
+    }
+    atomicAdd(&counts[slot], 1u);
+  }
+  __syncthreads();
+  uint32_t c = 0;
+  for (int i = threadIdx.x; i < kSampleSlots; i += 1024) c += counts[i] * (counts[i] - 1u);
+  c = abh::wave_sum(c);
+  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) c += sums[w];
+    *pairs = c;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1047,7 +1113,7 @@ struct QueryPlan {
   const double *q_sorted = nullptr;
   int64_t max_work = 0;  // work items, or an upper bound before the first count
   DevBuf qbuf, perm, keys, work, light;
-  DevBuf counters;  // listed queries, work items, escape flag
+  DevBuf counters;  // listed queries, work items, escape flag, sampled pairs
 
   const int32_t *qperm() const { return permuted ? perm.as<int32_t>() : nullptr; }
 };
@@ -1085,14 +1151,10 @@ static bool group_fits(const QueryPlan &p) {
   return true;
 }
 
-// Whether the cells hold few particles: the mean occupancy of a particle's
-// bucket (the squared bucket counts over the particles, which is what the
-// candidate tests of the set against itself grow with) is at most `most`.
-// The sum is read back once per build.  Sets of up to kSmall particles are
-// served by k_search_group whatever their cells: in one bucket, 16,384 x
-// 16,384 tests take less there than the chains of a few work items.
-static bool cells_light(const abh_cells *c, double most) {
-  if (c->n_alive <= kSmall) return true;
+// Whether the mean occupancy of a particle's bucket (the squared bucket counts
+// over the particles, which is what the candidate tests of the set against
+// itself grow with) is at most `most`.  The sum is read back once per build.
+static bool occupancy_within(const abh_cells *c, double most) {
   if (!c->sq_known) {
     BuildCounters h{};
     ABH_HIP(hipMemcpyAsync(&h, c->counters.p, sizeof(h), hipMemcpyDeviceToHost, c->ctx->stream));
@@ -1101,6 +1163,25 @@ static bool cells_light(const abh_cells *c, double most) {
     c->sq_known = true;
   }
   return double(c->sq_sum) <= most * double(c->n_alive);
+}
+
+// Whether k_search_group serves every query (see the constants).
+template <int D> static bool light_route(QueryPlan &p, const double *q) {
+  const abh_cells *c = p.cells;
+  const int64_t n = c->n_alive, nq = p.nq;
+  if (n > kSmall && !occupancy_within(c, p.op ? kLightOp : kLightSearch)) return false;
+  if (p.self && n > kSmall) return true;
+  if (nq <= kSmall) return !p.op || nq <= kSmallOp || occupancy_within(c, double(kSmallOp));
+  if (!p.op && nq <= kFewCentres) return true;
+  const double seen = std::min(double(n), double(p.nslots) * double(n) / double(c->nb));
+  if (double(nq) * seen <= (p.op ? kFewTestsOp : kFewTests)) return true;
+  uint32_t *pairs = p.counters.as<uint32_t>() + 3, h = 0;
+  k_shared_cells<D><<<1, 1024, 0, p.ctx->stream>>>(q, nq, c->params(), pairs);
+  check_launch();
+  ABH_HIP(hipMemcpyAsync(&h, pairs, 4, hipMemcpyDeviceToHost, p.ctx->stream));
+  ABH_HIP(hipStreamSynchronize(p.ctx->stream));
+  const double shared = double(nq) * double(h) / (double(kSample) * double(kSample - 1));
+  return shared <= (p.op ? kSharedOp : kSharedSearch);
 }
 
 template <int D> static void plan_items(QueryPlan &p) {
@@ -1149,7 +1230,7 @@ template <int D> static void build_plan_d(QueryPlan &p, const double *q) {
   // 4 million random centres, 8 particles a cell in 3D: search 2.24 and
   // 7.76 ms sorted, 1.33 and 6.63 ms as they come).  The plan keeps a copy of
   // the centres.
-  p.all_light = p.group && cells_light(p.cells, p.op ? kLightOp : kLightSearch);
+  p.all_light = p.group && light_route<D>(p, q);
   if (p.all_light) {
     ABH_HIP(hipMemsetAsync(p.counters.p, 0, 8, s));
     p.sub_levels = 0;

@@ -54,6 +54,19 @@ CASES += [
 ]
 
 
+# Many centres: few tests in all, centres that share cells or do not, a radius
+# well below a cell's side; most particles of a set of 12,300 in one bucket.
+CASES += [
+    ("uniform", 300, 2, False, 5.0, 1.0, 40_001),
+    ("uniform", 8_000, 2, True, 900.0, 0.3, 33_003),   # 1,500 centres a cell
+    ("uniform", 8_000, 2, False, 900.0, 0.3, 33_003),
+    ("uniform", 16_000, 3, True, 60.0, 0.6, 17_111),
+    ("uniform", 60_000, 2, False, 9.0, 0.95, 130_001),  # 20 to 30 centres a cell
+    ("uniform", 300, 1, False, 3.0, 1.0, 1_000_003),
+    ("uniform", 12_300, 2, False, 1e6, 0.1, 0),
+]
+
+
 @pytest.mark.parametrize("case", CASES, ids=["%s-%d-%dd-%s-%g-%g-%d" % c for c in CASES])
 def test_routes(ctx, case):
     kind, n, dim, per, n_leaf, cells_r, other = case
