@@ -39,8 +39,20 @@ constexpr int kSymRpt = 4, kSymVariant = 2;
 constexpr int kSymTiles = 8;
 constexpr int64_t kSymPart = int64_t(5) << 25;
 
+template <int V> struct Profile { static constexpr int value = V; };
+
 // MQ: the multiquadric sqrt(|dx|^2 + c^2) with fused multiply-adds (the
 // batched RBF systems' kernel), instead of the generic profile.
+//
+// Bound by the vector instructions of the profile, with few tiles by the
+// latency of their chains.  The profile is chosen outside the column loop (as a
+// switch inside it a branch kept the columns' chains apart, and the time hung
+// on how the switch was written: 4 to 8% either way).  One-sided, us, before and
+// now: one problem of 60,000 points in 3D, 1/(r + p) 11,006 -> 4,325, Gaussian
+// 10,818 -> 4,853; 2,000 of 1,000 points in 2D, 1/(r + p) 1,864 -> 1,687, in
+// FP32 1,052 -> 906.  Columns in flight: four; in FP32 two (3,000 problems of
+// 700 points in 3D: 802 us with two, 891 with four), for the FP32 Gaussian one
+// (1,068, 1,079 with two, 1,191 with four).
 template <int D, bool FP32, int RPT, bool MQ>
 __global__ __launch_bounds__(kRows) void k_dense(const int2 *__restrict__ tiles, int ntiles,
                                                  const int64_t *__restrict__ off,
@@ -85,46 +97,67 @@ __global__ __launch_bounds__(kRows) void k_dense(const int2 *__restrict__ tiles,
     }
     __syncthreads();
     if (!any) continue;
-    for (int j = 0; j < m; ++j) {
-      double pj[D];
+    auto columns = [&](auto profile) {
+      constexpr int kType = decltype(profile)::value;
+      constexpr int kUnroll = !FP32 ? 4 : (kType == ABH_KERNEL_GAUSSIAN ? 1 : 2);
+      auto column = [&](int j) {
+        double pj[D];
 #pragma unroll
-      for (int d = 0; d < D; ++d) pj[d] = sp[j][d];
-      const double xj = sx[j];
+        for (int d = 0; d < D; ++d) pj[d] = sp[j][d];
+        const double xj = sx[j];
 #pragma unroll
-      for (int q = 0; q < RPT; ++q) {
-        if (MQ && FP32) {
-          float s = float(k.param2);
+        for (int q = 0; q < RPT; ++q) {
+          if (MQ && FP32) {
+            float s = float(k.param2);
 #pragma unroll
-          for (int d = D - 1; d >= 0; --d) {
-            const float dx = float(pj[d] - xi[q][d]);
-            s = fmaf(dx, dx, s);
+            for (int d = D - 1; d >= 0; --d) {
+              const float dx = float(pj[d] - xi[q][d]);
+              s = fmaf(dx, dx, s);
+            }
+            abh::kb_add(a32[q], c32[q], __builtin_amdgcn_sqrtf(s) * float(xj));
+          } else if (MQ) {
+            double s = k.param2;
+#pragma unroll
+            for (int d = D - 1; d >= 0; --d) {
+              const double dx = pj[d] - xi[q][d];
+              s = fma(dx, dx, s);
+            }
+            acc[q] = fma(abh::sqrt_pos(s), xj, acc[q]);  // s >= c^2 >= 1e-280
+          } else if (FP32) {
+            float s = 0.0f;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+              const float dx = float(pj[d] - xi[q][d]);
+              s = s + dx * dx;
+            }
+            abh::kb_add(a32[q], c32[q], abh::phi32t<kType>(k, s) * float(xj));
+          } else {
+            double s = 0.0;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+              const double dx = pj[d] - xi[q][d];
+              s = s + dx * dx;
+            }
+            acc[q] += abh::phi64t<kType>(k, s) * xj;
           }
-          abh::kb_add(a32[q], c32[q], __builtin_amdgcn_sqrtf(s) * float(xj));
-        } else if (MQ) {
-          double s = k.param2;
-#pragma unroll
-          for (int d = D - 1; d >= 0; --d) {
-            const double dx = pj[d] - xi[q][d];
-            s = fma(dx, dx, s);
-          }
-          acc[q] = fma(abh::sqrt_pos(s), xj, acc[q]);  // s >= c^2 >= 1e-280
-        } else if (FP32) {
-          float s = 0.0f;
-#pragma unroll
-          for (int d = 0; d < D; ++d) {
-            const float dx = float(pj[d] - xi[q][d]);
-            s = s + dx * dx;
-          }
-          abh::kb_add(a32[q], c32[q], abh::phi32(k, s) * float(xj));
-        } else {
-          double s = 0.0;
-#pragma unroll
-          for (int d = 0; d < D; ++d) {
-            const double dx = pj[d] - xi[q][d];
-            s = s + dx * dx;
-          }
-          acc[q] += abh::phi64(k, s) * xj;
         }
+      };
+      if (MQ) {
+        for (int j = 0; j < m; ++j) column(j);
+      } else {
+#pragma unroll kUnroll
+        for (int j = 0; j < m; ++j) column(j);
+      }
+    };
+    if (MQ) {
+      columns(Profile<ABH_KERNEL_MULTIQUADRIC>{});
+    } else {
+      switch (k.type) {
+        case ABH_KERNEL_CONSTANT: columns(Profile<ABH_KERNEL_CONSTANT>{}); break;
+        case ABH_KERNEL_GAUSSIAN: columns(Profile<ABH_KERNEL_GAUSSIAN>{}); break;
+        case ABH_KERNEL_WENDLAND_C2: columns(Profile<ABH_KERNEL_WENDLAND_C2>{}); break;
+        case ABH_KERNEL_MULTIQUADRIC: columns(Profile<ABH_KERNEL_MULTIQUADRIC>{}); break;
+        case ABH_KERNEL_SMOOTH_INV_R: columns(Profile<ABH_KERNEL_SMOOTH_INV_R>{}); break;
       }
     }
   }
@@ -150,10 +183,12 @@ __global__ __launch_bounds__(kRows) void k_dense(const int2 *__restrict__ tiles,
 // adds its FP32 terms in FP64.
 // Bound by the vector instructions of the profile (multiquadric: 14 per pair
 // and row for both sides, against 2 x 13).  512 problems of 1,000 to 64,000
-// points: 118.7 -> 73.8 ms.  Shorter sums: against sums in double-double that
+// points: 118.7 -> 73.8 ms.  The other profiles, chosen outside the column
+// loops: 512 problems of 4,100 points, Gaussian in 3D 10.7 -> 6.7 ms (9.1 with the
+// switch in the loop), 1/(r + p) in 1D 6.9 -> 5.5 (7.4).  Shorter sums: against sums in double-double that
 // batch is 4.1e-15 off, one-sided 6.8e-15 (as is a plain sum by rows, which
 // therefore agrees with the one-sided form to 1.2e-15).
-template <int D, bool FP32, bool MQ>
+template <int D, bool FP32, bool MQ, int TYPE>
 __device__ __forceinline__ double sym_phi(const KernelDesc &k, const double *a, const double *b,
                                           double xj, double &row) {
   // returns the profile's value as the column side uses it and adds f xj
@@ -164,7 +199,7 @@ __device__ __forceinline__ double sym_phi(const KernelDesc &k, const double *a, 
       const float dx = float(a[d] - b[d]);
       s = fmaf(dx, dx, s);
     }
-    const float f = MQ ? __builtin_amdgcn_sqrtf(s) : abh::phi32(k, s);
+    const float f = MQ ? __builtin_amdgcn_sqrtf(s) : abh::phi32t<TYPE>(k, s);
     row += double(f * float(xj));
     return double(f);
   }
@@ -174,7 +209,7 @@ __device__ __forceinline__ double sym_phi(const KernelDesc &k, const double *a, 
     const double dx = a[d] - b[d];
     s = MQ ? fma(dx, dx, s) : s + dx * dx;
   }
-  const double f = MQ ? abh::sqrt_pos(s) : abh::phi64(k, s);  // MQ: s >= c^2 >= 1e-280
+  const double f = MQ ? abh::sqrt_pos(s) : abh::phi64t<TYPE>(k, s);  // MQ: s >= c^2 >= 1e-280
   row = fma(f, xj, row);
   return f;
 }
@@ -210,66 +245,80 @@ __global__ __launch_bounds__(kRows) void k_dense_sym(const int2 *__restrict__ ti
     acc[q] = 0.0;
   }
   const int64_t own = min(n, row0 + RPT * kRows);  // columns of the tile itself
-  for (int64_t c0 = row0; c0 < n;) {
-    const bool diag = c0 < own;
-    const int m = int(min(int64_t(kRows), (diag ? own : n) - c0));
-    __syncthreads();
-    if (int(threadIdx.x) < m) {
-      const int64_t j = base + c0 + threadIdx.x;
+  auto columns = [&](auto profile) {
+    constexpr int kType = decltype(profile)::value;
+    for (int64_t c0 = row0; c0 < n;) {
+      const bool diag = c0 < own;
+      const int m = int(min(int64_t(kRows), (diag ? own : n) - c0));
+      __syncthreads();
+      if (int(threadIdx.x) < m) {
+        const int64_t j = base + c0 + threadIdx.x;
 #pragma unroll
-      for (int d = 0; d < D; ++d) sp[d][threadIdx.x] = pos[j * D + d];
-      sx[threadIdx.x] = x[j];
-    }
-#pragma unroll
-    for (int w = 0; w < kRows / 64; ++w) csum[w][threadIdx.x] = 0.0;
-    __syncthreads();
-    if (diag) {
-      // (rows past the problem's end have sums that nobody reads)
-      for (int j = 0; j < m; ++j) {
-        double pj[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d) pj[d] = sp[d][j];
-        const double xj = sx[j];
-#pragma unroll
-        for (int q = 0; q < RPT; ++q) sym_phi<D, FP32, MQ>(k, pj, xi[q], xj, acc[q]);
+        for (int d = 0; d < D; ++d) sp[d][threadIdx.x] = pos[j * D + d];
+        sx[threadIdx.x] = x[j];
       }
-    } else {
-      // columns past a tile exist only if the tile is full: every row counts
-      for (int b = 0; b < m; b += 64) {
-        const int mm = min(64, m - b);
-        auto step = [&](int j) {
+#pragma unroll
+      for (int w = 0; w < kRows / 64; ++w) csum[w][threadIdx.x] = 0.0;
+      __syncthreads();
+      if (diag) {
+        // (rows past the problem's end have sums that nobody reads)
+        for (int j = 0; j < m; ++j) {
           double pj[D];
 #pragma unroll
           for (int d = 0; d < D; ++d) pj[d] = sp[d][j];
           const double xj = sx[j];
-          double col = 0.0;
 #pragma unroll
-          for (int q = 0; q < RPT; ++q) {
-            const double f = sym_phi<D, FP32, MQ>(k, pj, xi[q], xj, acc[q]);
-            if (FP32) col += double(float(f) * float(xr[q]));
-            else col = fma(f, xr[q], col);
-          }
-          unsafeAtomicAdd(&csum[wave][j], col);  // this lane's column alone, in step order
-        };
-        if (mm == 64) {
+          for (int q = 0; q < RPT; ++q) sym_phi<D, FP32, MQ, kType>(k, pj, xi[q], xj, acc[q]);
+        }
+      } else {
+        // columns past a tile exist only if the tile is full: every row counts
+        for (int b = 0; b < m; b += 64) {
+          const int mm = min(64, m - b);
+          auto step = [&](int j) {
+            double pj[D];
+#pragma unroll
+            for (int d = 0; d < D; ++d) pj[d] = sp[d][j];
+            const double xj = sx[j];
+            double col = 0.0;
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+              const double f = sym_phi<D, FP32, MQ, kType>(k, pj, xi[q], xj, acc[q]);
+              if (FP32) col += double(float(f) * float(xr[q]));
+              else col = fma(f, xr[q], col);
+            }
+            unsafeAtomicAdd(&csum[wave][j], col);  // this lane's column alone, in step order
+          };
+          if (mm == 64) {
 #pragma unroll 2
-          for (int s = 0; s < 64; ++s) step(b + ((lane + s) & 63));
-        } else {
-          for (int s = 0; s < 64; ++s) {
-            const int j = (lane + s) & 63;
-            if (j < mm) step(b + j);
+            for (int s = 0; s < 64; ++s) step(b + ((lane + s) & 63));
+          } else {
+            for (int s = 0; s < 64; ++s) {
+              const int j = (lane + s) & 63;
+              if (j < mm) step(b + j);
+            }
           }
         }
-      }
-      __syncthreads();
-      if (int(threadIdx.x) < m) {
-        double v = csum[0][threadIdx.x];
+        __syncthreads();
+        if (int(threadIdx.x) < m) {
+          double v = csum[0][threadIdx.x];
 #pragma unroll
-        for (int w = 1; w < kRows / 64; ++w) v += csum[w][threadIdx.x];
-        out[c0 - row0 + threadIdx.x] = v;
+          for (int w = 1; w < kRows / 64; ++w) v += csum[w][threadIdx.x];
+          out[c0 - row0 + threadIdx.x] = v;
+        }
       }
+      c0 += m;
     }
-    c0 += m;
+  };
+  if (MQ) {
+    columns(Profile<ABH_KERNEL_MULTIQUADRIC>{});
+  } else {
+    switch (k.type) {
+      case ABH_KERNEL_CONSTANT: columns(Profile<ABH_KERNEL_CONSTANT>{}); break;
+      case ABH_KERNEL_GAUSSIAN: columns(Profile<ABH_KERNEL_GAUSSIAN>{}); break;
+      case ABH_KERNEL_WENDLAND_C2: columns(Profile<ABH_KERNEL_WENDLAND_C2>{}); break;
+      case ABH_KERNEL_MULTIQUADRIC: columns(Profile<ABH_KERNEL_MULTIQUADRIC>{}); break;
+      case ABH_KERNEL_SMOOTH_INV_R: columns(Profile<ABH_KERNEL_SMOOTH_INV_R>{}); break;
+    }
   }
 #pragma unroll
   for (int q = 0; q < RPT; ++q) {
