@@ -76,7 +76,7 @@ constexpr int64_t kSmall = 16384;  // this few queries over as few particles: al
 // lanes, 1.25 with work items; 10,000 (r = 0.05, 3D) 0.27 and 0.48.
 constexpr int64_t kSmallOp = 12288;
 constexpr int64_t kFewCentres = 32768;                // lists: half a wave per SIMD as items
-constexpr double kFewTests = 2e8, kFewTestsOp = 3e7;  // tests that a plan does not pay for
+constexpr double kFewTests = 1.2e8, kFewTestsOp = 3e7;  // tests that a plan does not pay for
 
 struct WorkItem {
   int32_t home[3];
@@ -1106,6 +1106,10 @@ struct QueryPlan {
   // work lists); otherwise the two lists of k_plan_items
   bool all_light = false;
   bool op = false;     // an operator's plan
+  // an operator's list passes (count, assembly) go by the lists' rule: all its
+  // queries to k_search_group although its products have work items (16,000
+  // points in one bucket: assembly 1.50 ms, 3.61 by work items)
+  bool lists_light = false;
   bool group = false;  // k_search_group serves some of the queries
   double radius = 0, r2 = 0;
   int w[3] = {0, 0, 0};
@@ -1165,29 +1169,39 @@ static bool occupancy_within(const abh_cells *c, double most) {
   return double(c->sq_sum) <= most * double(c->n_alive);
 }
 
-// Whether k_search_group serves every query (see the constants).
-template <int D> static bool light_route(QueryPlan &p, const double *q) {
-  const abh_cells *c = p.cells;
-  const int64_t n = c->n_alive, nq = p.nq;
-  if (n > kSmall && !occupancy_within(c, p.op ? kLightOp : kLightSearch)) return false;
-  if (p.self && n > kSmall) return true;
-  if (nq <= kSmall) return !p.op || nq <= kSmallOp || occupancy_within(c, double(kSmallOp));
-  if (!p.op && nq <= kFewCentres) return true;
-  const double seen = std::min(double(n), double(p.nslots) * double(n) / double(c->nb));
-  if (double(nq) * seen <= (p.op ? kFewTestsOp : kFewTests)) return true;
+// Mean number of centres that a centre sees in its cell, by a sample.
+template <int D> static double shared_cells(QueryPlan &p, const double *q) {
   uint32_t *pairs = p.counters.as<uint32_t>() + 3, h = 0;
-  k_shared_cells<D><<<1, 1024, 0, p.ctx->stream>>>(q, nq, c->params(), pairs);
+  k_shared_cells<D><<<1, 1024, 0, p.ctx->stream>>>(q, p.nq, p.cells->params(), pairs);
   check_launch();
   ABH_HIP(hipMemcpyAsync(&h, pairs, 4, hipMemcpyDeviceToHost, p.ctx->stream));
   ABH_HIP(hipStreamSynchronize(p.ctx->stream));
-  const double shared = double(nq) * double(h) / (double(kSample) * double(kSample - 1));
-  return shared <= (p.op ? kSharedOp : kSharedSearch);
+  return double(p.nq) * double(h) / (double(kSample) * double(kSample - 1));
+}
+
+// Whether k_search_group serves every query of products (op) or of list passes
+// (see the constants).  shared: shared_cells, or negative if not asked yet.
+template <int D>
+static bool light_route(QueryPlan &p, const double *q, bool op, double &shared) {
+  const abh_cells *c = p.cells;
+  const int64_t n = c->n_alive, nq = p.nq;
+  if (n > kSmall && !occupancy_within(c, op ? kLightOp : kLightSearch)) return false;
+  if (p.self && n > kSmall) return true;
+  if (nq <= kSmall) return !op || nq <= kSmallOp || occupancy_within(c, double(kSmallOp));
+  if (!op && nq <= kFewCentres) return true;
+  const double seen = std::min(double(n), double(p.nslots) * double(n) / double(c->nb));
+  if (double(nq) * seen <= (op ? kFewTestsOp : kFewTests)) return true;
+  if (shared < 0.0) shared = shared_cells<D>(p, q);
+  return shared <= (op ? kSharedOp : kSharedSearch);
 }
 
 template <int D> static void plan_items(QueryPlan &p) {
   abh_context *ctx = p.ctx;
   const int64_t n = p.nq;
-  p.work.ensure(size_t(n + 1) * sizeof(WorkItem));
+  // every item holds kHeavyMin queries, or is the last of at least two of a
+  // run of 64 and more; without the list there may be as many items as queries
+  p.max_work = p.group ? n / kHeavyMin : n;
+  p.work.ensure(size_t(p.max_work + 1) * sizeof(WorkItem));
   p.light.ensure(size_t(n + 1) * 4);
   uint32_t *ctr = p.counters.as<uint32_t>();  // [0] = listed queries, [1] = work items
   ABH_HIP(hipMemsetAsync(ctr, 0, 8, ctx->stream));
@@ -1196,11 +1210,7 @@ template <int D> static void plan_items(QueryPlan &p) {
       p.op ? kCrowdedOp : kCrowdedSearch, p.q_sorted, p.cells->params(), p.work.as<WorkItem>(),
       p.light.as<int32_t>(), ctr);
   check_launch();
-  // every item holds kHeavyMin queries, or is the last of at least two of a
-  // run of 64 and more; without the list there may be as many items as queries,
-  // and it pays to wait for their number
-  p.max_work = n / kHeavyMin;
-  if (!p.group) {
+  if (!p.group) {  // it pays to wait for their number
     uint32_t h = 0;
     ABH_HIP(hipMemcpyAsync(&h, ctr + 1, 4, hipMemcpyDeviceToHost, ctx->stream));
     ABH_HIP(hipStreamSynchronize(ctx->stream));
@@ -1230,7 +1240,9 @@ template <int D> static void build_plan_d(QueryPlan &p, const double *q) {
   // 4 million random centres, 8 particles a cell in 3D: search 2.24 and
   // 7.76 ms sorted, 1.33 and 6.63 ms as they come).  The plan keeps a copy of
   // the centres.
-  p.all_light = p.group && light_route<D>(p, q);
+  double shared = -1.0;
+  p.all_light = p.group && light_route<D>(p, q, p.op, shared);
+  p.lists_light = p.group && p.op && !p.all_light && light_route<D>(p, q, false, shared);
   if (p.all_light) {
     ABH_HIP(hipMemsetAsync(p.counters.p, 0, 8, s));
     p.sub_levels = 0;
@@ -1332,11 +1344,11 @@ static size_t lds_bytes(int nslots) {
 }
 
 template <int D, int MODE>
-static void launch_group(const QueryPlan &p, const SearchArgs &a, const GridParams &g) {
+static void launch_group(const QueryPlan &p, const SearchArgs &a, const GridParams &g, bool all) {
   // all queries, or the ones k_plan_items listed (how many is on the device:
   // blocks past the end return at once)
-  const int32_t *list = p.all_light ? nullptr : p.light.as<int32_t>();
-  const uint32_t *nlist = p.all_light ? nullptr : p.counters.as<uint32_t>();
+  const int32_t *list = all ? nullptr : p.light.as<int32_t>();
+  const uint32_t *nlist = all ? nullptr : p.counters.as<uint32_t>();
   const unsigned grid = unsigned(ceil_div(p.nq, kGlGroups));
   constexpr bool kMV = MODE == kMatvec64 || MODE == kMatvec32;
   k_search_group<D, MODE><<<grid, kGlThreads, group_lds_bytes(a.nslots, kMV), p.ctx->stream>>>(
@@ -1359,10 +1371,12 @@ static void launch_matvec(const QueryPlan &p, const SearchArgs &a, const GridPar
 
 template <int D, int MODE> static void launch_search_d(const QueryPlan &p, const SearchArgs &a) {
   const GridParams g = p.cells->params();
-  if (p.group) launch_group<D, MODE>(p, a, g);
-  if (p.all_light || p.max_work == 0) return;
+  constexpr bool kMV = MODE == kMatvec64 || MODE == kMatvec32;
+  const bool all = p.all_light || (p.group && p.lists_light && !kMV);
+  if (p.group) launch_group<D, MODE>(p, a, g, all);
+  if (all || p.max_work == 0) return;
   const unsigned grid = unsigned(p.max_work);
-  if constexpr (MODE == kMatvec64 || MODE == kMatvec32) {
+  if constexpr (kMV) {
     launch_matvec<D, MODE == kMatvec32>(p, a, g, grid);
   } else {
     k_search<D, MODE><<<grid, kGroup, lds_bytes(a.nslots), p.ctx->stream>>>(a, g);
