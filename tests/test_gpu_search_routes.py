@@ -121,3 +121,50 @@ def test_routes(ctx, case):
     dense = torch.zeros(m, dtype=torch.float64, device="cuda")
     dense.index_add_(0, torch.tensor(row, device="cuda"), a_val * xt[0][a_col.long()])
     assert np.all(np.abs(dense.cpu().numpy() - y_o[:, 0]) <= 1e-13 * scale[:, 0])
+
+
+@pytest.mark.parametrize("kind,n", [("uniform", 3_001), ("blob", 20_003)])
+def test_stencil_widened_past_groups(ctx, kind, n):
+    """A radius a rounding above two cells: the plan is made for 125 buckets (for
+    the eight-lane form alone, or with both lists), and centres just below a
+    cell's face have a neighbour three cells on, so it is made again with 343
+    and work items only."""
+    rng = np.random.default_rng(n)
+    pos = cloud(kind, n, 3, rng)
+    face = np.arange(3, 13) / 16.0
+    pos[:10] = np.stack([face * (1.0 - 1e-13), face + 0.01, face + 0.02], 1)
+    pos[10:20] = np.stack([face + 2.0 / 16.0, face + 0.01, face + 0.02], 1)
+    low, high, per = [0.0] * 3, [1.0] * 3, [False] * 3
+    leaf = 0.999 * n / 4096.0
+    cl = ab.CellListOrdered(ctx, low, high, per, leaf)
+    cl.update_positions(torch.tensor(pos, device="cuda"))
+    oc = oracle.Cells(low, high, per, leaf)
+    oc.update(pos.copy(), np.ones(n, np.uint8))
+    assert list(oc.grid) == [16] * 3
+    r = 2.0 / 16.0 * (1.0 + 5e-10)
+    centres = cl.positions()
+    q = centres.cpu().numpy()
+    rp_o, col_o = oc.search(q, r)
+    cell = np.floor(q * 16.0)
+    apart = np.abs(np.repeat(cell, np.diff(rp_o), 0) - cell[col_o]).max(1)
+    assert apart.max() == 3
+    search = ab.Search(cl, centres, r)
+    for _ in range(2):  # the handle's plan is made anew
+        rp = search.row_ptr().cpu().numpy()
+        col = torch.zeros(search.total, dtype=torch.int32, device="cuda")
+        search.fill(col)
+        assert np.array_equal(rp, rp_o)
+        row = np.repeat(np.arange(n), np.diff(rp))
+        col = col.cpu().numpy()
+        assert np.array_equal(col[np.lexsort((col, row))], col_o[np.lexsort((col_o, row))])
+        search.run(cl, centres, r)
+    one = torch.zeros(len(col) + 5, dtype=torch.int32, device="cuda")
+    assert search.run_fused(cl, centres, r, one) == len(col)
+    assert np.array_equal(one.cpu().numpy()[:len(col)], col)
+    x = rng.standard_normal((n, 3))
+    y_o = oc.sparse_matvec(q, r, (1, 0.5 * r), x)
+    scale = oc.sparse_matvec(q, r, (1, 0.5 * r), np.abs(x))
+    op = ab.SparseOperator(ctx, cl, centres, r, ab.Kernel.gaussian(0.5 * r))
+    y = torch.zeros(3, n, dtype=torch.float64, device="cuda")
+    op.apply_colmajor(torch.tensor(x.T.copy(), device="cuda"), y)
+    assert np.all(np.abs(y.cpu().numpy().T - y_o) <= 1e-13 * scale)
