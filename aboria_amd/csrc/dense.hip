@@ -184,10 +184,11 @@ __global__ __launch_bounds__(kRows) void k_dense(const int2 *__restrict__ tiles,
 // Bound by the vector instructions of the profile (multiquadric: 14 per pair
 // and row for both sides, against 2 x 13).  512 problems of 1,000 to 64,000
 // points: 118.7 -> 73.8 ms.  The other profiles, chosen outside the column
-// loops: 512 problems of 4,100 points, Gaussian in 3D 10.7 -> 6.7 ms (9.1 with the
-// switch in the loop), 1/(r + p) in 1D 6.9 -> 5.5 (7.4).  Shorter sums: against sums in double-double that
-// batch is 4.1e-15 off, one-sided 6.8e-15 (as is a plain sum by rows, which
-// therefore agrees with the one-sided form to 1.2e-15).
+// loops: 512 problems of 4,100 points, Gaussian in 3D 10.7 -> 6.7 ms (9.1 with
+// the switch in the loop), 1/(r + p) in 1D 6.9 -> 5.5 (7.4).  Shorter sums:
+// against sums in double-double that batch is 4.1e-15 off, one-sided 6.8e-15
+// (as is a plain sum by rows, which therefore agrees with the one-sided form to
+// 1.2e-15).
 template <int D, bool FP32, bool MQ, int TYPE>
 __device__ __forceinline__ double sym_phi(const KernelDesc &k, const double *a, const double *b,
                                           double xj, double &row) {

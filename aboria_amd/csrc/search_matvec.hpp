@@ -160,11 +160,11 @@ __global__ __launch_bounds__(kGroup) __attribute__((amdgpu_waves_per_eu(3))) voi
   };
   // kernel values of the hits, added in pool order, once per visit; a pool's
   // terms are summed before they join the row's sum, since rows of a crowded
-  // cell have a thousand terms.  On the 4M-particle mixture this is 1.7e-15
-  // off a plain 64-bit evaluation, as is a row sum with full compensation
-  // (28.9 ms): what is left is that evaluation's own rounding.  One running
-  // sum per row is 1.9e-15 off (1.4e-15 when it runs in bucket order, close to
-  // the plain evaluation's order).
+  // cell have a thousand terms: against sums in extended precision 20,000 rows
+  // of 500 to 2,500 terms are 2.7e-16 off, one running sum per row 1.4e-15.  A
+  // plain 64-bit evaluation, which is such a running sum, therefore differs by
+  // its own rounding (4M-particle mixture 1.7e-15, as from a row sum with full
+  // compensation, which takes 15% longer).
   auto eval = [&](auto profile, auto plain) {
     double part[NR];
 #pragma unroll
