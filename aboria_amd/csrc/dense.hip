@@ -39,21 +39,23 @@ constexpr int kSymRpt = 4, kSymVariant = 2;
 constexpr int kSymTiles = 8;
 constexpr int64_t kSymPart = int64_t(5) << 25;
 
-template <int V> struct Profile { static constexpr int value = V; };
+// The profile of a batch is a template argument of its kernels: one of
+// abh_kernel_type, or kMq, the multiquadric sqrt(|dx|^2 + c^2) with fused
+// multiply-adds (the batched RBF systems' kernel).
+constexpr int kMq = -1;
 
-// MQ: the multiquadric sqrt(|dx|^2 + c^2) with fused multiply-adds (the
-// batched RBF systems' kernel), instead of the generic profile.
+// y += K x, one tile of RPT x 256 rows per block.
 //
 // Bound by the vector instructions of the profile, with few tiles by the
-// latency of their chains.  The profile is chosen outside the column loop (as a
-// switch inside it a branch kept the columns' chains apart, and the time hung
-// on how the switch was written: 4 to 8% either way).  One-sided, us, before and
+// latency of their chains.  (As a switch inside the column loop the profile was
+// a branch that kept the columns' chains apart, and the time hung on how the
+// switch was written: 4 to 8% either way.)  One-sided, us, before and
 // now: one problem of 60,000 points in 3D, 1/(r + p) 11,006 -> 4,325, Gaussian
 // 10,818 -> 4,853; 2,000 of 1,000 points in 2D, 1/(r + p) 1,864 -> 1,687, in
 // FP32 1,052 -> 906.  Columns in flight: four; in FP32 two (3,000 problems of
 // 700 points in 3D: 802 us with two, 891 with four), for the FP32 Gaussian one
 // (1,068, 1,079 with two, 1,191 with four).
-template <int D, bool FP32, int RPT, bool MQ>
+template <int D, bool FP32, int RPT, int PROF>
 __global__ __launch_bounds__(kRows) void k_dense(const int2 *__restrict__ tiles, int ntiles,
                                                  const int64_t *__restrict__ off,
                                                  const double *__restrict__ pos,
@@ -61,6 +63,7 @@ __global__ __launch_bounds__(kRows) void k_dense(const int2 *__restrict__ tiles,
                                                  double *__restrict__ y,
                                                  const uint8_t *__restrict__ active,
                                                  KernelDesc k, double alpha, int overwrite) {
+  constexpr bool MQ = PROF == kMq;
   __shared__ double sp[kRows][D];
   __shared__ double sx[kRows];
   const int t = blockIdx.x;
@@ -97,68 +100,54 @@ __global__ __launch_bounds__(kRows) void k_dense(const int2 *__restrict__ tiles,
     }
     __syncthreads();
     if (!any) continue;
-    auto columns = [&](auto profile) {
-      constexpr int kType = decltype(profile)::value;
-      constexpr int kUnroll = !FP32 ? 4 : (kType == ABH_KERNEL_GAUSSIAN ? 1 : 2);
-      auto column = [&](int j) {
-        double pj[D];
+    auto column = [&](int j) {
+      double pj[D];
 #pragma unroll
-        for (int d = 0; d < D; ++d) pj[d] = sp[j][d];
-        const double xj = sx[j];
+      for (int d = 0; d < D; ++d) pj[d] = sp[j][d];
+      const double xj = sx[j];
 #pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-          if (MQ && FP32) {
-            float s = float(k.param2);
+      for (int q = 0; q < RPT; ++q) {
+        if (MQ && FP32) {
+          float s = float(k.param2);
 #pragma unroll
-            for (int d = D - 1; d >= 0; --d) {
-              const float dx = float(pj[d] - xi[q][d]);
-              s = fmaf(dx, dx, s);
-            }
-            abh::kb_add(a32[q], c32[q], __builtin_amdgcn_sqrtf(s) * float(xj));
-          } else if (MQ) {
-            double s = k.param2;
-#pragma unroll
-            for (int d = D - 1; d >= 0; --d) {
-              const double dx = pj[d] - xi[q][d];
-              s = fma(dx, dx, s);
-            }
-            acc[q] = fma(abh::sqrt_pos(s), xj, acc[q]);  // s >= c^2 >= 1e-280
-          } else if (FP32) {
-            float s = 0.0f;
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-              const float dx = float(pj[d] - xi[q][d]);
-              s = s + dx * dx;
-            }
-            abh::kb_add(a32[q], c32[q], abh::phi32t<kType>(k, s) * float(xj));
-          } else {
-            double s = 0.0;
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-              const double dx = pj[d] - xi[q][d];
-              s = s + dx * dx;
-            }
-            acc[q] += abh::phi64t<kType>(k, s) * xj;
+          for (int d = D - 1; d >= 0; --d) {
+            const float dx = float(pj[d] - xi[q][d]);
+            s = fmaf(dx, dx, s);
           }
+          abh::kb_add(a32[q], c32[q], __builtin_amdgcn_sqrtf(s) * float(xj));
+        } else if (MQ) {
+          double s = k.param2;
+#pragma unroll
+          for (int d = D - 1; d >= 0; --d) {
+            const double dx = pj[d] - xi[q][d];
+            s = fma(dx, dx, s);
+          }
+          acc[q] = fma(abh::sqrt_pos(s), xj, acc[q]);  // s >= c^2 >= 1e-280
+        } else if (FP32) {
+          float s = 0.0f;
+#pragma unroll
+          for (int d = 0; d < D; ++d) {
+            const float dx = float(pj[d] - xi[q][d]);
+            s = s + dx * dx;
+          }
+          abh::kb_add(a32[q], c32[q], abh::phi32t<PROF>(k, s) * float(xj));
+        } else {
+          double s = 0.0;
+#pragma unroll
+          for (int d = 0; d < D; ++d) {
+            const double dx = pj[d] - xi[q][d];
+            s = s + dx * dx;
+          }
+          acc[q] += abh::phi64t<PROF>(k, s) * xj;
         }
-      };
-      if (MQ) {
-        for (int j = 0; j < m; ++j) column(j);
-      } else {
-#pragma unroll kUnroll
-        for (int j = 0; j < m; ++j) column(j);
       }
     };
-    if (MQ) {
-      columns(Profile<ABH_KERNEL_MULTIQUADRIC>{});
+    if constexpr (MQ) {
+      for (int j = 0; j < m; ++j) column(j);
     } else {
-      switch (k.type) {
-        case ABH_KERNEL_CONSTANT: columns(Profile<ABH_KERNEL_CONSTANT>{}); break;
-        case ABH_KERNEL_GAUSSIAN: columns(Profile<ABH_KERNEL_GAUSSIAN>{}); break;
-        case ABH_KERNEL_WENDLAND_C2: columns(Profile<ABH_KERNEL_WENDLAND_C2>{}); break;
-        case ABH_KERNEL_MULTIQUADRIC: columns(Profile<ABH_KERNEL_MULTIQUADRIC>{}); break;
-        case ABH_KERNEL_SMOOTH_INV_R: columns(Profile<ABH_KERNEL_SMOOTH_INV_R>{}); break;
-      }
+      constexpr int kUnroll = !FP32 ? 4 : (PROF == ABH_KERNEL_GAUSSIAN ? 1 : 2);
+#pragma unroll kUnroll
+      for (int j = 0; j < m; ++j) column(j);
     }
   }
 #pragma unroll
@@ -183,16 +172,17 @@ __global__ __launch_bounds__(kRows) void k_dense(const int2 *__restrict__ tiles,
 // adds its FP32 terms in FP64.
 // Bound by the vector instructions of the profile (multiquadric: 14 per pair
 // and row for both sides, against 2 x 13).  512 problems of 1,000 to 64,000
-// points: 118.7 -> 73.8 ms.  The other profiles, chosen outside the column
-// loops: 512 problems of 4,100 points, Gaussian in 3D 10.7 -> 6.7 ms (9.1 with
+// points: 118.7 -> 73.8 ms.  The other profiles:
+// 512 problems of 4,100 points, Gaussian in 3D 10.7 -> 6.7 ms (9.1 with
 // the switch in the loop), 1/(r + p) in 1D 6.9 -> 5.5 (7.4).  Shorter sums:
 // against sums in double-double that batch is 4.1e-15 off, one-sided 6.8e-15
 // (as is a plain sum by rows, which therefore agrees with the one-sided form to
 // 1.2e-15).
-template <int D, bool FP32, bool MQ, int TYPE>
+template <int D, bool FP32, int PROF>
 __device__ __forceinline__ double sym_phi(const KernelDesc &k, const double *a, const double *b,
                                           double xj, double &row) {
   // returns the profile's value as the column side uses it and adds f xj
+  constexpr bool MQ = PROF == kMq;
   if (FP32) {
     float s = MQ ? float(k.param2) : 0.0f;
 #pragma unroll
@@ -200,7 +190,7 @@ __device__ __forceinline__ double sym_phi(const KernelDesc &k, const double *a, 
       const float dx = float(a[d] - b[d]);
       s = fmaf(dx, dx, s);
     }
-    const float f = MQ ? __builtin_amdgcn_sqrtf(s) : abh::phi32t<TYPE>(k, s);
+    const float f = MQ ? __builtin_amdgcn_sqrtf(s) : abh::phi32t<PROF>(k, s);
     row += double(f * float(xj));
     return double(f);
   }
@@ -210,12 +200,12 @@ __device__ __forceinline__ double sym_phi(const KernelDesc &k, const double *a, 
     const double dx = a[d] - b[d];
     s = MQ ? fma(dx, dx, s) : s + dx * dx;
   }
-  const double f = MQ ? abh::sqrt_pos(s) : abh::phi64t<TYPE>(k, s);  // MQ: s >= c^2 >= 1e-280
+  const double f = MQ ? abh::sqrt_pos(s) : abh::phi64t<PROF>(k, s);  // MQ: s >= c^2 >= 1e-280
   row = fma(f, xj, row);
   return f;
 }
 
-template <int D, bool FP32, bool MQ>
+template <int D, bool FP32, int PROF>
 __global__ __launch_bounds__(kRows) void k_dense_sym(const int2 *__restrict__ tiles,
                                                      const int64_t *__restrict__ poff,
                                                      const int64_t *__restrict__ off,
@@ -246,80 +236,66 @@ __global__ __launch_bounds__(kRows) void k_dense_sym(const int2 *__restrict__ ti
     acc[q] = 0.0;
   }
   const int64_t own = min(n, row0 + RPT * kRows);  // columns of the tile itself
-  auto columns = [&](auto profile) {
-    constexpr int kType = decltype(profile)::value;
-    for (int64_t c0 = row0; c0 < n;) {
-      const bool diag = c0 < own;
-      const int m = int(min(int64_t(kRows), (diag ? own : n) - c0));
-      __syncthreads();
-      if (int(threadIdx.x) < m) {
-        const int64_t j = base + c0 + threadIdx.x;
+  for (int64_t c0 = row0; c0 < n;) {
+    const bool diag = c0 < own;
+    const int m = int(min(int64_t(kRows), (diag ? own : n) - c0));
+    __syncthreads();
+    if (int(threadIdx.x) < m) {
+      const int64_t j = base + c0 + threadIdx.x;
 #pragma unroll
-        for (int d = 0; d < D; ++d) sp[d][threadIdx.x] = pos[j * D + d];
-        sx[threadIdx.x] = x[j];
+      for (int d = 0; d < D; ++d) sp[d][threadIdx.x] = pos[j * D + d];
+      sx[threadIdx.x] = x[j];
+    }
+#pragma unroll
+    for (int w = 0; w < kRows / 64; ++w) csum[w][threadIdx.x] = 0.0;
+    __syncthreads();
+    if (diag) {
+      // (rows past the problem's end have sums that nobody reads)
+      for (int j = 0; j < m; ++j) {
+        double pj[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) pj[d] = sp[d][j];
+        const double xj = sx[j];
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) sym_phi<D, FP32, PROF>(k, pj, xi[q], xj, acc[q]);
       }
-#pragma unroll
-      for (int w = 0; w < kRows / 64; ++w) csum[w][threadIdx.x] = 0.0;
-      __syncthreads();
-      if (diag) {
-        // (rows past the problem's end have sums that nobody reads)
-        for (int j = 0; j < m; ++j) {
+    } else {
+      // columns past a tile exist only if the tile is full: every row counts
+      for (int b = 0; b < m; b += 64) {
+        const int mm = min(64, m - b);
+        auto step = [&](int j) {
           double pj[D];
 #pragma unroll
           for (int d = 0; d < D; ++d) pj[d] = sp[d][j];
           const double xj = sx[j];
+          double col = 0.0;
 #pragma unroll
-          for (int q = 0; q < RPT; ++q) sym_phi<D, FP32, MQ, kType>(k, pj, xi[q], xj, acc[q]);
-        }
-      } else {
-        // columns past a tile exist only if the tile is full: every row counts
-        for (int b = 0; b < m; b += 64) {
-          const int mm = min(64, m - b);
-          auto step = [&](int j) {
-            double pj[D];
-#pragma unroll
-            for (int d = 0; d < D; ++d) pj[d] = sp[d][j];
-            const double xj = sx[j];
-            double col = 0.0;
-#pragma unroll
-            for (int q = 0; q < RPT; ++q) {
-              const double f = sym_phi<D, FP32, MQ, kType>(k, pj, xi[q], xj, acc[q]);
-              if (FP32) col += double(float(f) * float(xr[q]));
-              else col = fma(f, xr[q], col);
-            }
-            unsafeAtomicAdd(&csum[wave][j], col);  // this lane's column alone, in step order
-          };
-          if (mm == 64) {
+          for (int q = 0; q < RPT; ++q) {
+            const double f = sym_phi<D, FP32, PROF>(k, pj, xi[q], xj, acc[q]);
+            if (FP32) col += double(float(f) * float(xr[q]));
+            else col = fma(f, xr[q], col);
+          }
+          unsafeAtomicAdd(&csum[wave][j], col);  // this lane's column alone, in step order
+        };
+        if (mm == 64) {
 #pragma unroll 2
-            for (int s = 0; s < 64; ++s) step(b + ((lane + s) & 63));
-          } else {
-            for (int s = 0; s < 64; ++s) {
-              const int j = (lane + s) & 63;
-              if (j < mm) step(b + j);
-            }
+          for (int s = 0; s < 64; ++s) step(b + ((lane + s) & 63));
+        } else {
+          for (int s = 0; s < 64; ++s) {
+            const int j = (lane + s) & 63;
+            if (j < mm) step(b + j);
           }
         }
-        __syncthreads();
-        if (int(threadIdx.x) < m) {
-          double v = csum[0][threadIdx.x];
-#pragma unroll
-          for (int w = 1; w < kRows / 64; ++w) v += csum[w][threadIdx.x];
-          out[c0 - row0 + threadIdx.x] = v;
-        }
       }
-      c0 += m;
+      __syncthreads();
+      if (int(threadIdx.x) < m) {
+        double v = csum[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < kRows / 64; ++w) v += csum[w][threadIdx.x];
+        out[c0 - row0 + threadIdx.x] = v;
+      }
     }
-  };
-  if (MQ) {
-    columns(Profile<ABH_KERNEL_MULTIQUADRIC>{});
-  } else {
-    switch (k.type) {
-      case ABH_KERNEL_CONSTANT: columns(Profile<ABH_KERNEL_CONSTANT>{}); break;
-      case ABH_KERNEL_GAUSSIAN: columns(Profile<ABH_KERNEL_GAUSSIAN>{}); break;
-      case ABH_KERNEL_WENDLAND_C2: columns(Profile<ABH_KERNEL_WENDLAND_C2>{}); break;
-      case ABH_KERNEL_MULTIQUADRIC: columns(Profile<ABH_KERNEL_MULTIQUADRIC>{}); break;
-      case ABH_KERNEL_SMOOTH_INV_R: columns(Profile<ABH_KERNEL_SMOOTH_INV_R>{}); break;
-    }
+    c0 += m;
   }
 #pragma unroll
   for (int q = 0; q < RPT; ++q) {
@@ -599,6 +575,27 @@ double *dense_scratch_address() {
 
 }  // namespace abh
 
+// LAUNCH(D, FP32, PROF) for the dimension, precision and profile (mq: kMq) at
+// hand
+#define ABH_DENSE_DISPATCH(LAUNCH)        \
+  if (dim == 1) ABH_DENSE_FP(LAUNCH, 1)   \
+  else if (dim == 2) ABH_DENSE_FP(LAUNCH, 2) \
+  else ABH_DENSE_FP(LAUNCH, 3)
+#define ABH_DENSE_FP(LAUNCH, DD)               \
+  {                                            \
+    if (fp32) ABH_DENSE_TYPE(LAUNCH, DD, true) \
+    else ABH_DENSE_TYPE(LAUNCH, DD, false)     \
+  }
+#define ABH_DENSE_TYPE(LAUNCH, DD, F32)                                                     \
+  switch (mq ? kMq : k.type) {                                                              \
+    case kMq: LAUNCH(DD, F32, kMq) break;                                                   \
+    case ABH_KERNEL_CONSTANT: LAUNCH(DD, F32, ABH_KERNEL_CONSTANT) break;                   \
+    case ABH_KERNEL_GAUSSIAN: LAUNCH(DD, F32, ABH_KERNEL_GAUSSIAN) break;                   \
+    case ABH_KERNEL_WENDLAND_C2: LAUNCH(DD, F32, ABH_KERNEL_WENDLAND_C2) break;             \
+    case ABH_KERNEL_MULTIQUADRIC: LAUNCH(DD, F32, ABH_KERNEL_MULTIQUADRIC) break;           \
+    case ABH_KERNEL_SMOOTH_INV_R: LAUNCH(DD, F32, ABH_KERNEL_SMOOTH_INV_R) break;           \
+  }
+
 struct abh_dense_batch {
   abh_context *ctx = nullptr;
   int dim = 2;
@@ -622,19 +619,10 @@ struct abh_dense_batch {
     const int ow = overwrite ? 1 : 0;
     const bool mq =
         k.type == ABH_KERNEL_MULTIQUADRIC && !k.row_s && !k.col_s && k.param2 >= 1e-280;
-#define ABH_DENSE_LAUNCH2(DD, MQ)                                                               \
-  if (fp32)                                                                                     \
-    k_dense<DD, true, RPT, MQ><<<nt, kRows, 0, s>>>(tl, nt, o, pos, x, y, act, k, alpha, ow);   \
-  else                                                                                          \
-    k_dense<DD, false, RPT, MQ><<<nt, kRows, 0, s>>>(tl, nt, o, pos, x, y, act, k, alpha, ow);
-#define ABH_DENSE_LAUNCH(DD)                                                                    \
-  if (mq) { ABH_DENSE_LAUNCH2(DD, true) }                                                       \
-  else { ABH_DENSE_LAUNCH2(DD, false) }
-    if (dim == 1) { ABH_DENSE_LAUNCH(1) }
-    else if (dim == 2) { ABH_DENSE_LAUNCH(2) }
-    else { ABH_DENSE_LAUNCH(3) }
-#undef ABH_DENSE_LAUNCH
-#undef ABH_DENSE_LAUNCH2
+#define ABH_DENSE_PROF(DD, F32, P) \
+  k_dense<DD, F32, RPT, P><<<nt, kRows, 0, s>>>(tl, nt, o, pos, x, y, act, k, alpha, ow);
+    ABH_DENSE_DISPATCH(ABH_DENSE_PROF)
+#undef ABH_DENSE_PROF
     abh::check_launch();
   }
 
@@ -647,17 +635,10 @@ struct abh_dense_batch {
     const int nt = ntiles[kSymVariant];
     const bool mq =
         k.type == ABH_KERNEL_MULTIQUADRIC && !k.row_s && !k.col_s && k.param2 >= 1e-280;
-#define ABH_DENSE_SYM2(DD, MQ)                                                             \
-  if (fp32) k_dense_sym<DD, true, MQ><<<nt, kRows, 0, s>>>(tl, po, o, pos, x, pt, act, k); \
-  else k_dense_sym<DD, false, MQ><<<nt, kRows, 0, s>>>(tl, po, o, pos, x, pt, act, k);
-#define ABH_DENSE_SYM(DD)             \
-  if (mq) { ABH_DENSE_SYM2(DD, true) } \
-  else { ABH_DENSE_SYM2(DD, false) }
-    if (dim == 1) { ABH_DENSE_SYM(1) }
-    else if (dim == 2) { ABH_DENSE_SYM(2) }
-    else { ABH_DENSE_SYM(3) }
-#undef ABH_DENSE_SYM
-#undef ABH_DENSE_SYM2
+#define ABH_DENSE_PROF(DD, F32, P) \
+  k_dense_sym<DD, F32, P><<<nt, kRows, 0, s>>>(tl, po, o, pos, x, pt, act, k);
+    ABH_DENSE_DISPATCH(ABH_DENSE_PROF)
+#undef ABH_DENSE_PROF
     abh::check_launch();
     k_dense_sym_sum<<<nt, kRows, 0, s>>>(tl, kSymRpt * kRows, po, o, pt, y, act, alpha,
                                          overwrite ? 1 : 0);
