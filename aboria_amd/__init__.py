@@ -932,7 +932,9 @@ class DenseBatchOperator:
 
     def tune(self, precision=FP64, force=0):
         """Runs the tile-shape autotuner (or sets rows-per-thread `force`);
-        returns (rows_per_thread, {rpt: ms})."""
+        returns (rows_per_thread, {rpt: ms}), 0 ms for shapes not timed.
+        Batches of many tiles use every kernel value for both sides, with 4
+        rows per thread alone; setting 1 or 2 takes the one-sided form."""
         rpt = ctypes.c_int(int(force))
         ms = (ctypes.c_float * 3)()
         check(C.lib().abh_dense_batch_tune(self.handle, precision, ctypes.byref(rpt), ms),

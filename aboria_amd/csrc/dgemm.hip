@@ -1,8 +1,9 @@
 // Strided-batched FP64 GEMM on the matrix cores (v_mfma_f64_16x16x4f64),
 // column-major like BLAS:  C[g] = alpha op(A[g]) op(B[g]) + beta C[g].
-// Used by the Schwarz local factorisations (panel / trailing updates and the
-// blocked triangular solves), whose operands are 64-wide panels of matrices
-// up to a few thousand rows.
+// Used by the Schwarz local factorisations (updates of block columns and of
+// what lies right of a panel, the blocked triangular solves), whose operands
+// are blocks of 64 to 512 columns of matrices up to tens of thousands of rows,
+// and by the FMM's compression.
 //
 // One workgroup (4 wavefronts) computes a 64 x 64 tile of C; each wavefront a
 // 32 x 32 quarter as 2 x 2 blocks of 16 x 16.  The k dimension is staged in
