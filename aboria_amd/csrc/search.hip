@@ -66,8 +66,13 @@ constexpr int kGroup = 64;  // queries per work item = lanes per wave
 //    300 a cell: fill 1,088 us, now 732, operator 3,038 and 1,334; the mixture's
 //    operator 21.5 and 19.7 ms).  For lists from 128 queries on: 1,000,000
 //    points at 60 a cell take 1,262 us to fill from 64 on, 1,195 from 128 on.
+//    So have the few particles of a cell beside crowded ones, whose lists are as
+//    long (a set against itself; 200,000 points with 4,000 in a blob, 2D: fill
+//    450 us, now 331, operator 2.01 and 0.87 ms).  For lists from 2,048 particles
+//    in the stencil on, since a cell of 60 has 1,650; operators from 1,024.
 constexpr int kHeavyMin = 12;
 constexpr int kCrowdedSearch = 128, kCrowdedOp = kGroup;
+constexpr uint32_t kMostListedSearch = 2048, kMostListedOp = 1024;
 constexpr double kLightSearch = 40.0;  // mean occupancy a particle sees, list passes
 constexpr double kLightOp = 13.0;      // the same for an operator's plan
 constexpr double kSharedSearch = 40.0, kSharedOp = 20.0;  // centres a centre sees in its cell
@@ -153,8 +158,10 @@ __global__ __launch_bounds__(kThreads) void k_home_keys(const double *__restrict
 // Runs of equal home cell (the key without its sub-cell bits) cut into work.
 // A run's whole groups of 64, and a remainder of at least heavy_min queries or
 // of a run of at least `crowded`, become work items of k_search; the queries of
-// another remainder go to the list that k_search_group serves.  One thread per run (its first query),
-// which finds the run's end by doubling steps and a binary search; a block of
+// another remainder go to the list that k_search_group serves.  One thread per
+// run (its first query), which finds the run's end by doubling steps and a binary search.  With bbeg
+// and bend a remainder whose stencil holds more than st.most particles is an
+// item too; a block of
 // 1,024 takes its places in both lists with one atomic each (one per
 // wavefront: 0.65 ms at 4,000,000 queries, now 0.061 ms), so the lists stay
 // close to the sorted order.  ctr[0] = listed queries, ctr[1] = work items,
@@ -162,12 +169,71 @@ __global__ __launch_bounds__(kThreads) void k_home_keys(const double *__restrict
 // query stands in the lists.
 constexpr int kPlanThreads = 1024;
 
+struct Stencil {
+  int w[3];
+  uint32_t most;
+};
+
+// Particles in the stencil around a query's home cell.  The buckets of one row
+// of the last dimension lie one after another, and so do their particles.
+template <int D>
+__device__ __forceinline__ uint32_t stencil_particles(const double *q, const GridParams &g,
+                                                      const Stencil &st,
+                                                      const uint32_t *__restrict__ bbeg,
+                                                      const uint32_t *__restrict__ bend) {
+  constexpr int kLast = D - 1;
+  int h[3] = {0, 0, 0};
+#pragma unroll
+  for (int d = 0; d < D; ++d) h[d] = home_of<D>(g, q, d);
+  const int n = g.size[kLast];
+  const int lo = h[kLast] - st.w[kLast], hi = h[kLast] + st.w[kLast];
+  auto row_sum = [&](uint32_t row) {
+    const uint32_t b = row * uint32_t(n);
+    auto range = [&](int a, int e) {
+      a = a < 0 ? 0 : a;
+      e = e < n ? e : n - 1;
+      return a <= e ? bend[b + uint32_t(e)] - bbeg[b + uint32_t(a)] : 0u;
+    };
+    uint32_t sum = range(lo, hi);
+    if (g.periodic[kLast]) {
+      if (lo < 0) sum += range(lo + n, n - 1);
+      if (hi >= n) sum += range(0, hi - n);
+    }
+    return sum;
+  };
+  // bucket of a virtual cell, -1: none
+  auto wrap = [&](int d, int v) {
+    const int m = g.size[d];
+    if (g.periodic[d]) v = v < 0 ? v + m : (v >= m ? v - m : v);
+    return v >= 0 && v < m ? v : -1;
+  };
+  if (D == 1) return row_sum(0);
+  uint32_t sum = 0;
+#pragma unroll 1
+  for (int x = h[0] - st.w[0]; x <= h[0] + st.w[0]; ++x) {
+    const int bx = wrap(0, x);
+    if (bx < 0) continue;
+    if (D == 2) {
+      sum += row_sum(uint32_t(bx));
+      continue;
+    }
+    for (int y = h[D - 2] - st.w[D - 2]; y <= h[D - 2] + st.w[D - 2]; ++y) {
+      const int by = wrap(D - 2, y);
+      if (by >= 0) sum += row_sum(uint32_t(bx) * uint32_t(g.size[D - 2]) + uint32_t(by));
+    }
+  }
+  return sum;
+}
+
 template <int D>
 __global__ __launch_bounds__(kPlanThreads) void k_plan_items(const uint32_t *__restrict__ keys,
                                                          int64_t n, int shift, int heavy_min,
                                                          int crowded,
                                                          const double *__restrict__ q_sorted,
-                                                         GridParams g, WorkItem *__restrict__ work,
+                                                         GridParams g, Stencil st,
+                                                         const uint32_t *__restrict__ bbeg,
+                                                         const uint32_t *__restrict__ bend,
+                                                         WorkItem *__restrict__ work,
                                                          int32_t *__restrict__ light,
                                                          uint32_t *__restrict__ ctr) {
   __shared__ uint32_t wsum[2][kPlanThreads / 64], wbase[2];
@@ -188,7 +254,9 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan_items(const uint32_t *__r
     ++e;
     const int64_t c = e - k;
     const int rem = int(c % kGroup);
-    const bool list = rem < heavy_min && c < crowded;
+    bool list = rem > 0 && rem < heavy_min && c < crowded;
+    if (list && bbeg)
+      list = stencil_particles<D>(q_sorted + k * D, g, st, bbeg, bend) <= st.most;
     nw = uint32_t(c / kGroup) + (rem > 0 && !list ? 1u : 0u);
     nl = list ? uint32_t(rem) : 0u;
   }
@@ -1199,18 +1267,23 @@ template <int D> static void plan_items(QueryPlan &p) {
   abh_context *ctx = p.ctx;
   const int64_t n = p.nq;
   // every item holds kHeavyMin queries, or is the last of at least two of a
-  // run of 64 and more; without the list there may be as many items as queries
-  p.max_work = p.group ? n / kHeavyMin : n;
+  // run of 64 and more, or a run's only one by its stencil; without the list
+  // there may be as many items as queries
+  const bool by_stencil = p.group && p.self && n > kSmall;
+  p.max_work = p.group ? n / kHeavyMin + (by_stencil ? std::min(n, p.cells->nb) : 0) : n;
   p.work.ensure(size_t(p.max_work + 1) * sizeof(WorkItem));
   p.light.ensure(size_t(n + 1) * 4);
   uint32_t *ctr = p.counters.as<uint32_t>();  // [0] = listed queries, [1] = work items
   ABH_HIP(hipMemsetAsync(ctr, 0, 8, ctx->stream));
   k_plan_items<D><<<unsigned(ceil_div(n, kPlanThreads)), kPlanThreads, 0, ctx->stream>>>(
       p.keys.as<uint32_t>(), n, p.sub_levels * D, p.group ? kHeavyMin : 1,
-      p.op ? kCrowdedOp : kCrowdedSearch, p.q_sorted, p.cells->params(), p.work.as<WorkItem>(),
+      p.op ? kCrowdedOp : kCrowdedSearch, p.q_sorted, p.cells->params(),
+      Stencil{{p.w[0], p.w[1], p.w[2]}, p.op ? kMostListedOp : kMostListedSearch},
+      by_stencil ? p.cells->begin.as<uint32_t>() : nullptr,
+      by_stencil ? p.cells->end.as<uint32_t>() : nullptr, p.work.as<WorkItem>(),
       p.light.as<int32_t>(), ctr);
   check_launch();
-  if (!p.group) {  // it pays to wait for their number
+  if (!p.group || p.max_work > 65536) {  // it pays to wait for their number
     uint32_t h = 0;
     ABH_HIP(hipMemcpyAsync(&h, ctr + 1, 4, hipMemcpyDeviceToHost, ctx->stream));
     ABH_HIP(hipStreamSynchronize(ctx->stream));

@@ -24,7 +24,7 @@ def cloud(kind, n, dim, rng):
     # a fifth of the particles in one small blob, the rest spread out: cells of
     # every occupancy side by side
     k = n // 5
-    blob = 0.3 + 0.02 * rng.standard_normal((k, dim))
+    blob = (0.0 if kind == "corner" else 0.3) + 0.02 * rng.standard_normal((k, dim))
     return np.concatenate([blob % 1.0, rng.random((n - k, dim))])
 
 
@@ -54,6 +54,14 @@ CASES += [
 ]
 
 
+# Cells of few particles beside crowded ones, at domain faces too.
+CASES += [
+    ("blob", 17_003, 2, True, 10.0, 0.9, 0),
+    ("blob", 30_001, 3, False, 6.0, 0.95, 0),
+    ("blob", 20_003, 1, False, 8.0, 0.7, 0),
+    ("corner", 20_003, 3, True, 5.0, 0.9, 0),
+    ("corner", 20_003, 2, False, 5.0, 1.7, 0),
+]
 # Many centres: few tests in all, centres that share cells or do not, a radius
 # well below a cell's side; most particles of a set of 12,300 in one bucket.
 CASES += [
