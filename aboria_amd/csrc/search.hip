@@ -158,15 +158,14 @@ __global__ __launch_bounds__(kThreads) void k_home_keys(const double *__restrict
 // Runs of equal home cell (the key without its sub-cell bits) cut into work.
 // A run's whole groups of 64, and a remainder of at least heavy_min queries or
 // of a run of at least `crowded`, become work items of k_search; the queries of
-// another remainder go to the list that k_search_group serves.  One thread per
-// run (its first query), which finds the run's end by doubling steps and a binary search.  With bbeg
-// and bend a remainder whose stencil holds more than st.most particles is an
-// item too; a block of
-// 1,024 takes its places in both lists with one atomic each (one per
-// wavefront: 0.65 ms at 4,000,000 queries, now 0.061 ms), so the lists stay
-// close to the sorted order.  ctr[0] = listed queries, ctr[1] = work items,
-// zero at launch.  A row's result does not depend on where its
-// query stands in the lists.
+// another remainder go to the list that k_search_group serves.  With bbeg and
+// bend a remainder whose stencil holds more than st.most particles is an item
+// too.  One thread per run (its first query), which finds the run's end by
+// doubling steps and a binary search.  A block of 1,024 takes its places in
+// both lists with one atomic each (one per wavefront: 0.65 ms at 4,000,000
+// queries, now 0.061 ms), so the lists stay close to the sorted order.
+// ctr[0] = listed queries, ctr[1] = work items, zero at launch.  A row's result
+// does not depend on where its query stands in the lists.
 constexpr int kPlanThreads = 1024;
 
 struct Stencil {
